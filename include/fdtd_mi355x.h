@@ -88,6 +88,27 @@ int fdtd_ctx_set_pml(fdtd_ctx* ctx, const float* decay_x, const float* decay_y,
 int fdtd_ctx_set_sources(fdtd_ctx* ctx, int n, const int32_t* kind, const int64_t* a,
                          const int64_t* b, const double* wave, int64_t wave_len);
 
+/* Multi-step passes (three time steps per sweep over the fields, the same
+ * arithmetic): on != 0 lets fdtd_step_n and fdtd_graph_run take them where the
+ * solve allows it (no poles, microphones or boundary planes, at most 64 probes,
+ * fewer than 2^30 cells, every source a point or plane), and promises that the
+ * field and flag buffers can be read 4 cells past their end. Off by default. No
+ * counterpart in the reference, which makes one pass per step. */
+int fdtd_ctx_set_multi_step(fdtd_ctx* ctx, int on);
+
+/* The whole source list in list order as fdtd_ctx_set_sources takes it, for the
+ * passes of a solve some of whose point or plane sources are in the per-cell
+ * tables of fdtd_ctx_set_membranes; without it such a solve steps one by one.
+ * Call it after both: each of them forgets it. */
+int fdtd_ctx_set_pass_sources(fdtd_ctx* ctx, int n, const int32_t* kind, const int64_t* a, const int64_t* b,
+                              const double* wave, int64_t wave_len);
+
+/* How a pass splits a grid: out[9] = steps per pass (0: no passes for it),
+ * threads per workgroup, 4-cell lanes per window row, lanes a k segment stores,
+ * rows per window, windows along k and j, planes per workgroup, workgroups.
+ * Host only. */
+int fdtd_pass_tiling(int nx, int ny, int nz, int32_t* out);
+
 /* Probes: host flat indices; trace: device float32 [trace_len][n]; step s
  * writes row s. Replaces _record_probes (core/solver.py:2435-2439). */
 int fdtd_ctx_set_probes(fdtd_ctx* ctx, int n, const int64_t* flat_idx, float* trace,

@@ -36,6 +36,9 @@ _SIGS = {
     "fdtd_ctx_set_pml": (_i, [_vp, _vp, _vp, _vp]),
     "fdtd_ctx_set_boundary_planes": (_i, [_vp, _i, _vp, _vp, _i64]),
     "fdtd_ctx_set_sources": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _i64]),
+    "fdtd_ctx_set_multi_step": (_i, [_vp, _i]),
+    "fdtd_ctx_set_pass_sources": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _i64]),
+    "fdtd_pass_tiling": (_i, [_i, _i, _i, _vp]),
     "fdtd_ctx_set_probes": (_i, [_vp, _i, _vp, _vp, _i64]),
     "fdtd_ctx_set_membranes": (_i, [_vp, _i, _vp, _vp, _i, _vp, _vp, _vp, _vp, _i, _vp, _i, _vp, _i64]),
     "fdtd_ctx_set_microphones": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _i64]),

@@ -18,6 +18,8 @@ namespace fdtd_amd {
 int fused_grid(FusedArgs& a, int rows, int planes, int stack);
 hipError_t launch_fused(const FusedArgs& a, int rows, int stack, bool nu, bool ade, int blocks,
                         hipStream_t st, hipEvent_t ev_before, hipEvent_t ev_after, const BoundarySet* bnd);
+bool pick_pass_tile(int nx, int ny, int nz, PassTile& best);
+hipError_t launch_pass(const FusedArgs& a, bool nu, const PassTile& m, hipStream_t st);
 hipError_t launch_advance(int64_t* step, int n, hipStream_t st);
 hipError_t launch_stream_ceiling(const FusedArgs& a, hipStream_t st);
 hipError_t launch_stream_march(const FusedArgs& a, int rows, int planes, hipStream_t st);
@@ -115,6 +117,17 @@ struct fdtd_ctx {
     std::vector<hipEvent_t> sweep_ev;  // pairs around each sweep (fdtd_time_sweeps)
     double* energy_partial = nullptr;  // owned: [energy_partials()][2]
     BoundarySet bnd;                   // boundary planes (state owned by the caller)
+    // multi-step passes: allowed by the caller, the grid's windows, and the
+    // sources they add where the one-step path has some of them in tables
+    struct Sources {
+        int n = 0;
+        int kind[FDTD_MAX_SOURCES], i[FDTD_MAX_SOURCES], j[FDTD_MAX_SOURCES], k[FDTD_MAX_SOURCES];
+        const double* wave = nullptr;
+        int64_t wave_len = 0;
+    } pass_src;
+    bool multi_step = false, have_pass_src = false;
+    bool tile_known = false, tile_ok = false;
+    PassTile tile{};
 };
 
 extern "C" {
@@ -184,6 +197,8 @@ int fdtd_ctx_set_grid(fdtd_ctx* c, int nx, int ny, int nz, int nonuniform, float
         return fail(-2, "nonuniform grid needs all six spacing tables");
     drop_graph(c);
     c->a.nx = nx; c->a.ny = ny; c->a.nz = nz;
+    c->tile_known = false;
+    c->have_pass_src = false;
     c->a.cv = cv; c->a.cp = cp;
     c->nonuniform = nonuniform != 0;
     c->a.ifc[0] = ifx; c->a.ifc[1] = ify; c->a.ifc[2] = ifz;
@@ -223,39 +238,88 @@ int fdtd_ctx_set_pml(fdtd_ctx* c, const float* dx, const float* dy, const float*
     return 0;
 }
 
-int fdtd_ctx_set_sources(fdtd_ctx* c, int n, const int32_t* kind, const int64_t* a, const int64_t* b,
-                         const double* wave, int64_t wave_len) {
-    if (!c) return fail(-1, "null context");
+// The source list of a call, checked against the grid.
+static int read_sources(const fdtd_ctx* c, int n, const int32_t* kind, const int64_t* a, const int64_t* b,
+                        const double* wave, int64_t wave_len, fdtd_ctx::Sources& out) {
     if (!c->have_grid) return fail(-3, "set the grid before the sources");
     if (n < 0 || n > FDTD_MAX_SOURCES) return fail(-2, "%d sources (max %d)", n, FDTD_MAX_SOURCES);
     if (n > 0 && (!kind || !a || !b || !wave || wave_len < 1)) return fail(-2, "bad source arrays");
     const int nx = c->a.nx, ny = c->a.ny, nz = c->a.nz;
     for (int q = 0; q < n; ++q) {
+        out.kind[q] = kind[q];
         if (kind[q] == 0) {
             const int64_t f = a[q];
             if (f < 0 || f >= static_cast<int64_t>(nx) * ny * nz)
                 return fail(-2, "point source %d: flat index %lld outside the grid", q, (long long)f);
-            c->a.src_kind[q] = 0;
-            c->a.src_k[q] = static_cast<int>(f % nz);
-            c->a.src_j[q] = static_cast<int>((f / nz) % ny);
-            c->a.src_i[q] = static_cast<int>(f / (static_cast<int64_t>(ny) * nz));
+            out.k[q] = static_cast<int>(f % nz);
+            out.j[q] = static_cast<int>((f / nz) % ny);
+            out.i[q] = static_cast<int>(f / (static_cast<int64_t>(ny) * nz));
         } else if (kind[q] == 1) {
             const int ax = static_cast<int>(a[q]);
             const int dims[3] = {nx, ny, nz};
             if (ax < 0 || ax > 2 || b[q] < 0 || b[q] >= dims[ax])
                 return fail(-2, "plane source %d: axis %d index %lld outside the grid", q, ax, (long long)b[q]);
-            c->a.src_kind[q] = 1;
-            c->a.src_i[q] = ax;
-            c->a.src_j[q] = static_cast<int>(b[q]);
-            c->a.src_k[q] = 0;
+            out.i[q] = ax;
+            out.j[q] = static_cast<int>(b[q]);
+            out.k[q] = 0;
         } else {
             return fail(-2, "source %d: unknown kind %d", q, kind[q]);
         }
     }
+    out.n = n;
+    out.wave = wave;
+    out.wave_len = n > 0 ? wave_len : 0;
+    return 0;
+}
+
+static void use_sources(FusedArgs& a, const fdtd_ctx::Sources& s) {
+    a.n_src = s.n;
+    for (int q = 0; q < s.n; ++q) {
+        a.src_kind[q] = s.kind[q];
+        a.src_i[q] = s.i[q];
+        a.src_j[q] = s.j[q];
+        a.src_k[q] = s.k[q];
+    }
+    a.wave = s.wave;
+    a.wave_len = s.wave_len;
+}
+
+int fdtd_ctx_set_sources(fdtd_ctx* c, int n, const int32_t* kind, const int64_t* a, const int64_t* b,
+                         const double* wave, int64_t wave_len) {
+    if (!c) return fail(-1, "null context");
+    fdtd_ctx::Sources s;
+    if (int rc = read_sources(c, n, kind, a, b, wave, wave_len, s)) return rc;
     drop_graph(c);
-    c->a.n_src = n;
-    c->a.wave = wave;
-    c->a.wave_len = n > 0 ? wave_len : 0;
+    use_sources(c->a, s);
+    c->have_pass_src = false;
+    return 0;
+}
+
+int fdtd_ctx_set_pass_sources(fdtd_ctx* c, int n, const int32_t* kind, const int64_t* a, const int64_t* b,
+                              const double* wave, int64_t wave_len) {
+    if (!c) return fail(-1, "null context");
+    fdtd_ctx::Sources s;
+    if (int rc = read_sources(c, n, kind, a, b, wave, wave_len, s)) return rc;
+    drop_graph(c);
+    c->pass_src = s;
+    c->have_pass_src = true;
+    return 0;
+}
+
+int fdtd_ctx_set_multi_step(fdtd_ctx* c, int on) {
+    if (!c) return fail(-1, "null context");
+    drop_graph(c);
+    c->multi_step = on != 0;
+    return 0;
+}
+
+int fdtd_pass_tiling(int nx, int ny, int nz, int32_t* out) {
+    if (!out) return fail(-1, "null output");
+    if (nx < 2 || ny < 2 || nz < 2) return fail(-2, "grid %dx%dx%d: every axis needs >= 2 cells", nx, ny, nz);
+    PassTile m{};
+    const bool ok = pick_pass_tile(nx, ny, nz, m);
+    const int32_t v[9] = {ok ? kPassSteps : 0, m.nt, m.kt, m.ko, m.rows, m.nseg, m.njt, m.units, m.nwg};
+    std::copy(v, v + 9, out);
     return 0;
 }
 
@@ -388,6 +452,7 @@ int fdtd_ctx_set_membranes(fdtd_ctx* c, int n_cells, const int64_t* cell, const 
     // steps already on the stream may still read the old tables
     if (int rc = check(hipStreamSynchronize(c->stream), "stream sync")) return rc;
     c->a.n_mcell = 0;
+    c->have_pass_src = false;
     if (n_cells == 0) return 0;
     std::vector<int32_t> cell32(cell, cell + n_cells);
     if (int rc = upload(c->m_cell, cell32.data(), sizeof(int32_t) * n_cells)) return rc;
@@ -556,10 +621,32 @@ static int ready(fdtd_ctx* c) {
     return 0;
 }
 
+// Whether the context's steps can go several to a pass (k_multi_step): what a
+// step adds around the sweep has to be in the pass as well, or absent.
+static bool pass_allowed(fdtd_ctx* c) {
+    const FusedArgs& a = c->a;
+    if (!c->multi_step || a.n_pole > 0 || a.n_mic > 0 || c->bnd.n > 0 || a.n_probe > kSweepProbes) return false;
+    if (a.n_mcell > 0 && !c->have_pass_src) return false;
+    if (!c->tile_known) {
+        c->tile_known = true;
+        c->tile_ok = pick_pass_tile(a.nx, a.ny, a.nz, c->tile);
+    }
+    return c->tile_ok;
+}
+
 static int enqueue_steps(fdtd_ctx* c, int n) {
     FusedArgs a = c->a;
     const int blocks = fused_grid(a, c->rows, c->planes, c->stack);
-    for (int s = 0; s < n; ++s) {
+    int s = 0;
+    if (n >= kPassSteps && pass_allowed(c)) {
+        FusedArgs pa = a;
+        if (a.n_mcell > 0) use_sources(pa, c->pass_src);
+        for (; n - s >= kPassSteps; s += kPassSteps) {
+            pa.koff = s;
+            if (int rc = check(launch_pass(pa, c->nonuniform, c->tile, c->stream), "multi-step pass launch")) return rc;
+        }
+    }
+    for (; s < n; ++s) {
         a.koff = s;
         if (int rc = check(launch_fused(a, c->rows, c->stack, c->nonuniform, a.n_pole > 0, blocks, c->stream,
                                         nullptr, nullptr, c->bnd.n ? &c->bnd : nullptr),

@@ -183,6 +183,21 @@ struct FusedArgs {
     int64_t n_ade_cells;            //   (null: the ADE kernels visit every box cell)
 };
 
+// Steps k_multi_step takes per pass. An odd count keeps the rule that step s
+// reads field set s & 1; three is what the LDS holds for workgroups of 1024.
+constexpr int kPassSteps = 3;
+
+// Windows and work split of such a pass.
+struct PassTile {
+    int nt;                         // threads per workgroup
+    int kt;                         // 4-cell lanes per window row
+    int ko;                         // lanes a k segment stores (the last one: the rest)
+    int rows;                       // rows per window
+    int nseg, njt;                  // windows along k and j
+    int units;                      // planes a workgroup stores
+    int nwg;                        // workgroups: windows x ceil(nx / units)
+};
+
 // The boundary planes of a context (host side of a launch).
 struct BoundarySet {
     int n = 0;

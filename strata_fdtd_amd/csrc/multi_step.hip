@@ -1,0 +1,519 @@
+// Several time steps in one pass over HBM (temporal blocking), gfx950.
+//
+// k_fused_step reads and writes every field once per step and runs at the rate
+// of a streaming pass, so a step that is not to cost 33 B per cell has to share
+// its pass with others. k_multi_step takes T steps per pass: a workgroup owns a
+// window of rows (j) and 4-cell lanes (k) and marches along i as a pipeline of
+// T stages, stage t taking step s + t on plane m - t while stage 0 is at plane
+// m. What stage t makes of a plane is what stage t + 1 reads, in registers; only
+// stage 0 loads from memory and only stage T - 1 stores.
+//
+// A thread owns 4 consecutive k cells of one row (16-byte accesses). Its row
+// above (p) and below (the updated vy) and its lane neighbours (p, vz) come from
+// LDS, posted in two phases per plane: the stages' pressures, then, once the y
+// and z faces are updated, their vy and vz. The outermost row and cell of a
+// window lack a neighbour, so each stage's valid cells shrink by one on every
+// interior side; neighbouring windows overlap by what T stages lose and store
+// only what is valid after the last one. Per cell the operations and their order
+// are k_fused_step's, so the results are the same bit for bit.
+//
+// What bounds it: at 512^3 HBM (a pass moves 4.65 GB, 1.05 times the 33 B per
+// cell of one step, since windows next to each other march the same planes at
+// the same time and share their halos in L2), with the vector units busy half
+// the time; on small grids the latency of its planes (1.2 us and 0.12 us per
+// resident wave), of which a pass over even one plane takes six. Held to 128
+// VGPRs (one workgroup of 1024 per CU) without spills in the loop: pressures and
+// updated vy stay in LDS only (with them in registers the spills made 512^3
+// 20% slower). Per step, air boxes: 512^3 850 us with k_fused_step, 335-360
+// here; 261x243x307 196, 61; 192^3 38.8, 18.5; 100^3 9.3, 7.2; 64^3 5.6, 5.4.
+
+#include <algorithm>
+#include <climits>
+
+#include "fdtd_common.hpp"
+
+namespace fdtd_amd {
+
+typedef float f4v __attribute__((ext_vector_type(4)));
+// rows of grids whose nz is no multiple of 4 start at any cell: 4-byte aligned
+// 16-byte accesses and byte-aligned flag words, which global memory takes
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32u __attribute__((aligned(1)));
+
+#if defined(__HIP_DEVICE_COMPILE__)
+#define CMEM __attribute__((address_space(4)))
+#else
+#define CMEM
+#endif
+// tables no kernel writes while it runs, read at wave-uniform indices
+template <typename T>
+__device__ __forceinline__ T uni(const T* t, int64_t i) {
+    return ((const CMEM T*)t)[i];
+}
+
+// The kernel's arguments where they lie (FusedArgs is the first), for code that
+// rarely runs: rare() hides the pointer's value, so its loads stay there and
+// hold no scalar registers across the loop.
+__device__ __forceinline__ const CMEM FusedArgs* kernargs() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return (const CMEM FusedArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+#else
+    return nullptr;
+#endif
+}
+__device__ __forceinline__ const CMEM FusedArgs* rare(const CMEM FusedArgs* p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+s"(p));
+#endif
+    return p;
+}
+
+// v, to the compiler a new value: an LDS entry read at again(v) is read where it
+// is used rather than kept in registers between uses.
+__device__ __forceinline__ int again(int v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(v));
+#endif
+    return v;
+}
+
+__device__ __forceinline__ f4v ld4(const GMEM float* base, uint32_t c) {
+    return *reinterpret_cast<const GMEM f4u*>(at32(base, c));
+}
+template <bool NTS>
+__device__ __forceinline__ void st4(GMEM float* base, uint32_t c, f4v v) {
+    if constexpr (NTS) __builtin_nontemporal_store(v, reinterpret_cast<GMEM f4u*>(at32(base, c)));
+    else *reinterpret_cast<GMEM f4u*>(at32(base, c)) = v;
+}
+
+// v where bit `bit` of byte e of f is set, else +0 (element by element)
+__device__ __forceinline__ f4v keep(f4v v, uint32_t f, int bit) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        v[e] = __int_as_float(__float_as_int(v[e]) & __builtin_amdgcn_sbfe(static_cast<int>(f), 8 * e + bit, 1));
+    return v;
+}
+
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// flags of four air cells with every face open, and their y bits alone
+constexpr uint32_t kOpen = 0x01010101u * (FDTD_FLAG_AIR | FDTD_FLAG_OPEN_X | FDTD_FLAG_OPEN_Y | FDTD_FLAG_OPEN_Z);
+constexpr uint32_t kOpenY = 0x01010101u * FDTD_FLAG_OPEN_Y;
+constexpr int kMaxLanes = 256;      // lanes of a window row at most
+constexpr int kEvery = INT_MAX, kNowhere = INT_MIN;
+
+constexpr int kWaitLoads = 0x0f70;  // s_waitcnt vmcnt(0), the other counters unlimited
+
+// One stage's state of a thread: velocities at the stage's plane (its pressure is
+// in LDS), the updated and not yet damped vx of the plane below, the plane's flags.
+struct Stage {
+    f4v vx, vy, vz, vxp;
+    uint32_t f;
+};
+
+template <bool NU, int NT, bool NTS>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_multi_step(const FusedArgs a, const PassTile mt) {
+    constexpr int T = kPassSteps;
+    __shared__ f4v sP[T][NT];
+    __shared__ f4v sY[T][NT + 1];
+    __shared__ float sX[T][NT];
+    __shared__ float sZ[T][NT + 1];
+    // nonuniform grids: damping, face and cell coefficients along k, per lane
+    __shared__ f4v sK[NU ? 3 : 1][NU ? kMaxLanes : 1];
+    const int tid = threadIdx.x;
+    const int nx = a.nx, ny = a.ny, nz = a.nz;
+    const int64_t s = uni(a.step_ptr, 0) + a.koff;
+    if (tid < T) {
+        sY[tid][NT] = f4v{0.f, 0.f, 0.f, 0.f};  // the row below the window's first
+        sZ[tid][NT] = 0.f;                      // the cell before its first lane
+    }
+    const int par = static_cast<int>(s & 1);
+    const GMEM float* __restrict__ P = gmem(par ? a.f[1][0] : a.f[0][0]);
+    const GMEM float* __restrict__ VX = gmem(par ? a.f[1][1] : a.f[0][1]);
+    const GMEM float* __restrict__ VY = gmem(par ? a.f[1][2] : a.f[0][2]);
+    const GMEM float* __restrict__ VZ = gmem(par ? a.f[1][3] : a.f[0][3]);
+    GMEM float* __restrict__ Po = gmem(par ? a.f[0][0] : a.f[1][0]);
+    GMEM float* __restrict__ VXo = gmem(par ? a.f[0][1] : a.f[1][1]);
+    GMEM float* __restrict__ VYo = gmem(par ? a.f[0][2] : a.f[1][2]);
+    GMEM float* __restrict__ VZo = gmem(par ? a.f[0][3] : a.f[1][3]);
+    const GMEM uint8_t* __restrict__ FL = gmem(a.flags);
+    const CMEM FusedArgs* ka = kernargs();
+    const uint32_t sx = static_cast<uint32_t>(ny) * static_cast<uint32_t>(nz);
+    const float cv = a.cv, cp = a.cp;
+
+    const int row = tid / mt.kt;
+    const int kl = tid - row * mt.kt;
+    const bool in_win = row < mt.rows;
+    const int iu = row + 1 < mt.rows ? tid + mt.kt : tid;  // row above
+    const int id = (row > 0 && in_win) ? tid - mt.kt : NT; // row below
+    const int ir = tid + 1 < NT ? tid + 1 : tid;           // next lane
+    const int il = kl > 0 ? tid - 1 : NT;                  // previous lane
+
+    // XCD-aware order: hardware block b runs on XCD b mod 8, which takes a
+    // contiguous range of the (window, plane) units
+    const int lb = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    const int nwin = mt.nseg * mt.njt;
+    if (lb < mt.nwg) {
+        const int chunk = lb / nwin, win = lb - chunk * nwin;
+        const int i0 = chunk * mt.units;
+        const int i1 = min(nx, i0 + mt.units);
+        const int seg = win % mt.nseg, jt = win / mt.nseg;
+        // window origin and the rows / lanes it stores
+        const int w0 = jt * (mt.rows - 2 * T);
+        const int jlo = jt == 0 ? 0 : w0 + T;
+        const int jhi = jt == mt.njt - 1 ? ny : w0 + mt.rows - T;
+        const int k0 = 4 * (seg == 0 ? 0 : seg * mt.ko - 1);
+        const int klo = 4 * seg * mt.ko;
+        const int khi = seg == mt.nseg - 1 ? nz : 4 * (seg + 1) * mt.ko;
+        const int j = w0 + row;
+        const int k = k0 + 4 * kl;
+        const bool ld = in_win && j < ny && k < nz;
+        const bool out = ld && j >= jlo && j < jhi && k >= klo && k < khi;
+        const int nv = nz - k;                               // 4 or more: a whole lane
+        const uint32_t c0 = static_cast<uint32_t>(j) * static_cast<uint32_t>(nz) + static_cast<uint32_t>(k);
+        const bool jlast = j == ny - 1;
+        const bool jlast_win = w0 + mt.rows >= ny;           // uniform
+        const bool klast_win = k0 + 4 * mt.kt >= nz;         // uniform
+        const int vlast = nz - 1 - k;                        // element of the last z face (0..3 in one lane)
+        const float dy = ld ? gmem(a.dec[1])[j] : 1.f;
+        float cvy = cv, icy = 1.f;
+        if (NU && ld) {
+            icy = gmem(a.icl[1])[j];
+            if (j + 1 < ny) cvy = cv * gmem(a.ifc[1])[j];
+        }
+        f4v dzr = {1.f, 1.f, 1.f, 1.f};
+        auto lane_tables = [&](int kk, f4v& dz, f4v& cvz, f4v& icz) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (kk + e < nz) {
+                    dz[e] = gmem(a.dec[2])[kk + e];
+                    if (NU) {
+                        icz[e] = gmem(a.icl[2])[kk + e];
+                        if (kk + e + 1 < nz) cvz[e] = cv * gmem(a.ifc[2])[kk + e];
+                    }
+                }
+        };
+        if constexpr (NU) {
+            if (tid < mt.kt) {
+                f4v dz = {1.f, 1.f, 1.f, 1.f}, cz = {cv, cv, cv, cv}, iz = {1.f, 1.f, 1.f, 1.f};
+                lane_tables(k0 + 4 * tid, dz, cz, iz);
+                sK[0][tid] = dz;
+                sK[1][tid] = cz;
+                sK[2][tid] = iz;
+            }
+        } else {
+            f4v none = {};
+            lane_tables(k, dzr, none, none);
+        }
+        // Flag bits that say nothing about walls: the last faces, which keep their
+        // velocity, cells past the row and lanes past the window or grid.
+        uint32_t ends = kOpen;
+        if (ld) {
+            ends = jlast ? kOpenY : 0u;
+            if (vlast < 4) ends |= (FDTD_FLAG_OPEN_Z << (8 * vlast)) | static_cast<uint32_t>(uint64_t(kOpen) << (8 * vlast + 8));
+        }
+        // Sources that touch the window and probes it stores: lane q holds the
+        // plane of source q (kEvery: a y or z plane source, on every plane) and
+        // of probe q, kNowhere if it is elsewhere, so a stage finds what its
+        // plane has with one compare. kNowhere is no plane: a stage's own plane
+        // runs from -(T - 1) to nx + T - 2.
+        int src_i = kNowhere, probe_i = kNowhere;
+        {
+            const int q = tid & (kWave - 1);
+            const int jw = w0 + mt.rows, kw = k0 + 4 * mt.kt;
+            if (q < a.n_src) {
+                const int at = a.src_i[q], sj = a.src_j[q], sk = a.src_k[q];
+                if (a.src_kind[q] == 0) {
+                    if (sj >= w0 && sj < jw && sk >= k0 && sk < kw) src_i = at;
+                } else if (at == 0) {
+                    src_i = sj;
+                } else if (at == 1 ? (sj >= w0 && sj < jw) : (sj >= k0 && sj < kw)) {
+                    src_i = kEvery;
+                }
+            }
+            if (q < a.n_sweep_probe) {
+                const GMEM int32_t* __restrict__ PIJK = gmem(a.probe_ijk);
+                const int pi = PIJK[3 * q], pj = PIJK[3 * q + 1], pk = PIJK[3 * q + 2];
+                if (pj >= jlo && pj < jhi && pk >= klo && pk < khi && pi >= i0 && pi < i1) probe_i = pi;
+            }
+        }
+
+        // A lane past its row's last cell reads on into the next row (or the pad
+        // past the last one): those cells feed nothing that is stored.
+        auto at = [&](int i) { return static_cast<uint32_t>(i) * sx + c0; };
+        auto flags = [&](uint32_t c) -> uint32_t { return *reinterpret_cast<const GMEM u32u*>(at32(FL, c)); };
+
+        const f4v zero = {0.f, 0.f, 0.f, 0.f};
+        Stage st[T];
+#pragma unroll
+        for (int t = 0; t < T; ++t) st[t] = Stage{zero, zero, zero, zero, 0u};
+        const int m0 = max(i0 - T, 0);
+        const int m1 = i1 + T - 1;
+        // plane m0, and p of the one after it
+        f4v p0 = zero, pn = zero;
+        if (ld) {
+            const uint32_t c = at(m0);
+            p0 = ld4(P, c);
+            st[0].vx = ld4(VX, c);
+            st[0].vy = ld4(VY, c);
+            st[0].vz = ld4(VZ, c);
+            st[0].f = flags(c);
+            if (m0 + 1 < nx) pn = ld4(P, c + sx);
+        }
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            sP[t][tid] = t ? zero : p0;
+            sX[t][tid] = t ? 0.f : p0.x;
+        }
+        __builtin_amdgcn_s_waitcnt(kWaitLoads);
+        for (int m = m0; m < m1; ++m) {
+            lds_barrier();  // the stages' pressures are posted
+            // ---- next plane's loads
+            f4v qp = zero, qx = zero, qy = zero, qz = zero;
+            uint32_t qf = 0;
+            if (ld && m + 1 < m1 && m + 1 < nx) {
+                const uint32_t c = at(m + 1);
+                if (m + 2 < nx) qp = ld4(P, c + sx);
+                qx = ld4(VX, c);
+                qy = ld4(VY, c);
+                qz = ld4(VZ, c);
+                qf = flags(c);
+            }
+            // ---- y and z faces of every stage's plane
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                Stage& S = st[t];
+                const f4v p = sP[t][tid];
+                const f4v pu = sP[t][iu];
+                const float pr = sX[t][ir];
+                f4v vy = S.vy + cvy * (pu - p);
+                const f4v pk = {p.y, p.z, p.w, pr};
+                f4v vz;
+                if constexpr (NU) vz = S.vz + sK[1][again(kl)] * (pk - p);
+                else vz = S.vz + cv * (pk - p);
+                const bool walls = __builtin_amdgcn_ballot_w64(((S.f | ends) & kOpen) != kOpen) != 0;
+                if (walls) {
+                    vy = keep(vy, S.f, 2);
+                    vz = keep(vz, S.f, 3);
+                }
+                if (jlast_win) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) vy[e] = jlast ? S.vy[e] : vy[e];
+                }
+                if (klast_win) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) vz[e] = vlast == e ? S.vz[e] : vz[e];
+                }
+                S.vz = vz;
+                sY[t][tid] = vy;
+                sZ[t][tid] = vz.w;
+            }
+            lds_barrier();
+            // ---- x faces and pressures, stage by stage: what stage t makes of
+            // its plane is p(i + 1) of stage t + 1, and its state of the next round
+            f4v cpn = pn, cx = qx, cy = qy, cz = qz;
+            uint32_t cf = qf;
+            f4v p = sP[0][tid];
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                Stage& S = st[t];
+                const int i = m - t;
+                const int ic = min(max(i, 0), nx - 1);
+                const f4v vy = sY[t][tid];
+                const f4v yb = sY[t][id];
+                const float zb = sZ[t][il];
+                const float dx = uni(a.dec[0], ic);
+                f4v vx = S.vx;
+                const bool walls = __builtin_amdgcn_ballot_w64(((S.f | ends) & kOpen) != kOpen) != 0;
+                if (i < nx - 1) {
+                    const float cvx = NU ? cv * uni(a.ifc[0], ic) : cv;
+                    vx = S.vx + cvx * (cpn - p);
+                    if (walls) vx = keep(vx, S.f, 1);
+                }
+                const f4v zl = {zb, S.vz.x, S.vz.y, S.vz.z};
+                const f4v dvx = vx - S.vxp, dvy = vy - yb, dvz = S.vz - zl;
+                f4v pnew;
+                if (NU) {
+                    const float icx = uni(a.icl[0], ic);
+                    pnew = p + cp * ((icx * dvx + icy * dvy) + sK[2][again(kl)] * dvz);
+                } else {
+                    pnew = p + cp * ((dvx + dvy) + dvz);
+                }
+                if (walls) pnew = keep(pnew, S.f, 0);
+                const f4v dz = NU ? sK[0][again(kl)] : dzr;
+                f4v ps = ((pnew * dx) * dy) * dz;
+                const f4v ox = vx * dx, oy = vy * dy, oz = S.vz * dz;
+                const uint64_t adds = __builtin_amdgcn_ballot_w64(src_i == i || src_i == kEvery);
+                if (adds) {
+                    const CMEM FusedArgs* r = rare(ka);
+                    for (uint32_t sm = static_cast<uint32_t>(adds); sm; sm &= sm - 1) {
+                        const int q = __builtin_ctz(sm);
+                        // the planes or point it acts on, -1: any (its i has matched)
+                        const bool point = r->src_kind[q] == 0;
+                        const int ax = r->src_i[q], aj = r->src_j[q], ak = r->src_k[q];
+                        const int on_j = point || ax == 1 ? aj : -1;
+                        const int on_k = point ? ak : (ax == 2 ? aj : -1);
+                        const bool known = s + t < r->wave_len;
+                        if (!known && tid == 0) atomicOr(r->health, 2u);
+                        const double w = known ? uni(r->wave, q * r->wave_len + s + t) : 0.0;
+                        const uint32_t hit = (known & ((on_j == j) | (on_j < 0))) ? S.f : 0u;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const float v = static_cast<float>(static_cast<double>(ps[e]) + w);
+                            const bool on = (((hit >> (8 * e)) & FDTD_FLAG_AIR) != 0) & ((on_k == k + e) | (on_k < 0));
+                            ps[e] = on ? v : ps[e];
+                        }
+                    }
+                }
+                const uint64_t hits = __builtin_amdgcn_ballot_w64(probe_i == i);
+                if (hits) {
+                    const CMEM FusedArgs* r = rare(ka);
+                    for (uint64_t pm = hits; pm; pm &= pm - 1) {
+                        const int q = __builtin_ctzll(pm);
+                        const int pj = uni(r->probe_ijk, 3 * q + 1), pk = uni(r->probe_ijk, 3 * q + 2);
+                        if (s + t >= r->trace_len) {
+                            if (tid == 0) atomicOr(r->health, 2u);
+                        } else if (in_win && j == pj && pk >= k && pk < k + 4) {
+                            const int e = pk - k;
+                            const float v = e == 0 ? ps.x : (e == 1 ? ps.y : (e == 2 ? ps.z : ps.w));
+                            gmem(r->trace)[(s + t) * r->n_probe + q] = v;
+                            if (!isfinite(v)) atomicOr(r->health, 1u);
+                        }
+                    }
+                }
+                if (t == T - 1) {
+                    // The next plane's loads are waited for before the stores are
+                    // issued: later, the wait would be for the stores as well.
+                    __builtin_amdgcn_s_waitcnt(kWaitLoads);
+                    if (out && i >= i0) {
+                        const uint32_t c = at(i);
+                        if (nv >= 4) {
+                            st4<NTS>(Po, c, ps);
+                            st4<NTS>(VXo, c, ox);
+                            st4<NTS>(VYo, c, oy);
+                            st4<NTS>(VZo, c, oz);
+                        } else {
+#pragma unroll
+                            for (int e = 0; e < 3; ++e)
+                                if (e < nv) {
+                                    stx(Po, c + e, ps[e]);
+                                    stx(VXo, c + e, ox[e]);
+                                    stx(VYo, c + e, oy[e]);
+                                    stx(VZo, c + e, oz[e]);
+                                }
+                        }
+                    }
+                }
+                // this stage's next plane: what came in (loads, or the stage before)
+                const uint32_t f = S.f;
+                S = Stage{cx, cy, cz, vx, cf};
+                if (t + 1 < T) p = sP[t + 1][tid];  // read before the next stage's p is posted
+                sP[t][tid] = cpn;
+                sX[t][tid] = cpn.x;
+                cpn = ps;
+                cx = ox;
+                cy = oy;
+                cz = oz;
+                cf = f;
+            }
+            pn = qp;
+        }
+    }
+}
+
+// ---- host side -------------------------------------------------------------------
+constexpr int kCUs = 256;
+
+// Windows of `nseg` k segments and workgroups of `nt` threads, marching `chunks`
+// ranges of planes; false where they do not exist.
+static bool pass_windows(int nx, int ny, int nz, int nt, int nseg, PassTile& m) {
+    const int lanes = (nz + 3) / 4;
+    m.nt = nt;
+    m.nseg = nseg;
+    if (nseg == 1) {
+        m.ko = m.kt = lanes;
+    } else {
+        m.ko = ((lanes - 1 + nseg - 1) / nseg + 3) & ~3;  // segments start on 64-byte blocks of the row
+        m.kt = m.ko + 2;
+        // every segment has lanes to store, and the last one's fit its window
+        if ((nseg - 1) * m.ko >= lanes || lanes - (nseg - 1) * m.ko > m.ko + 1) return false;
+    }
+    if (m.kt > std::min(nt, kMaxLanes)) return false;
+    m.rows = std::min(nt / m.kt, ny);
+    const int inner = m.rows - 2 * kPassSteps;
+    if (m.rows >= ny) m.njt = 1;
+    else if (inner < 1) return false;
+    else m.njt = (ny - 2 * kPassSteps + inner - 1) / inner;
+    return true;
+}
+
+// The split of a pass over the chip with the least estimated time. The estimate
+// is the marching time (plane rounds of the busiest CU: a plane takes 1.23 us of
+// latency and 0.12 us per resident wave) and, beyond the Infinity Cache, the
+// traffic at 5.2 TB/s times 1.2, the larger of the two and 0.3 of the smaller.
+// Fitted to 3337 measured (workgroup, segments, chunks) triples of 14 grids from
+// 40^3 to 400^3 (rms 16%): what it picks runs within 12% of the best triple.
+bool pick_pass_tile(int nx, int ny, int nz, PassTile& best) {
+    const int64_t cells = static_cast<int64_t>(nx) * ny * nz;
+    if (cells >= kMaxCells32) return false;
+    double low = 0.0;
+    bool found = false;
+    for (int nt : {1024, 512, 256}) {
+        const int per_cu = 1024 / nt, slots = kCUs * per_cu;
+        for (int nseg = 1; nseg <= 64; ++nseg) {
+            PassTile m{};
+            if (!pass_windows(nx, ny, nz, nt, nseg, m)) continue;
+            const int nwin = m.nseg * m.njt;
+            for (int c = 1; c <= nx; ++c) {
+                const int units = (nx + c - 1) / c;
+                if (c > 1 && units == (nx + c - 2) / (c - 1)) continue;  // the same split as c - 1
+                const int64_t n = static_cast<int64_t>(nwin) * ((nx + units - 1) / units);
+                const double planes = units + 2 * kPassSteps - 1;
+                auto plane_us = [&](int64_t wgs) {
+                    return 1.23 + 0.12 * (static_cast<double>((wgs + kCUs - 1) / kCUs) * nt / kWave);
+                };
+                const int64_t full = n / slots, rest = n % slots;
+                const double march = planes * (full * plane_us(slots) + (rest ? plane_us(rest) : 0.0));
+                double cost = march;
+                if (cells > kCacheResidentCells) {
+                    const double traffic = 1.2 * cells * (16.0 + 17.0 * (units + 2.0 * kPassSteps) / units) / 5.2e6;
+                    cost = std::max(march, traffic) + 0.3 * std::min(march, traffic);
+                }
+                if (!found || cost < low) {
+                    found = true;
+                    low = cost;
+                    m.units = units;
+                    m.nwg = static_cast<int>(n);
+                    best = m;
+                }
+            }
+        }
+    }
+    return found;
+}
+
+template <bool NU, int NT>
+static hipError_t launch_pass_t(const FusedArgs& a, const PassTile& m, hipStream_t st) {
+    const int blocks = (m.nwg + 7) & ~7;
+    if (static_cast<int64_t>(a.nx) * a.ny * a.nz <= kCacheResidentCells)
+        hipLaunchKernelGGL((k_multi_step<NU, NT, false>), dim3(blocks), dim3(NT), 0, st, a, m);
+    else
+        hipLaunchKernelGGL((k_multi_step<NU, NT, true>), dim3(blocks), dim3(NT), 0, st, a, m);
+    return hipGetLastError();
+}
+
+// Steps koff .. koff + kPassSteps - 1 of a chunk in one pass.
+hipError_t launch_pass(const FusedArgs& a, bool nu, const PassTile& m, hipStream_t st) {
+    switch (m.nt) {
+        case 1024: return nu ? launch_pass_t<true, 1024>(a, m, st) : launch_pass_t<false, 1024>(a, m, st);
+        case 512: return nu ? launch_pass_t<true, 512>(a, m, st) : launch_pass_t<false, 512>(a, m, st);
+        case 256: return nu ? launch_pass_t<true, 256>(a, m, st) : launch_pass_t<false, 256>(a, m, st);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace fdtd_amd

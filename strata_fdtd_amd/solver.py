@@ -140,8 +140,12 @@ class FDTDSolver:
         nx, ny, nz = self.shape
         dev = self._device
         f32 = torch.float32
-        self._f = [[torch.zeros(self.shape, dtype=f32, device=dev) for _ in _FIELDS] for _ in range(2)]
-        self._flags = torch.empty(self.shape, dtype=torch.uint8, device=dev)
+        # the fields and flags are readable one 4-cell access past their end
+        # (a multi-step pass reads whole 4-cell lanes)
+        n_cells = int(np.prod(self.shape))
+        padded = lambda dt: torch.zeros(n_cells + 4, dtype=dt, device=dev)[:n_cells].view(self.shape)  # noqa: E731
+        self._f = [[padded(f32) for _ in _FIELDS] for _ in range(2)]
+        self._flags = padded(torch.uint8)
         self._decay = [torch.ones(n, dtype=f32, device=dev) for n in self.shape]
         self._step_dev = torch.zeros(1, dtype=torch.int64, device=dev)
         self._health = torch.zeros(1, dtype=torch.int32, device=dev)
@@ -188,6 +192,7 @@ class FDTDSolver:
         self._cap = 0
         self._wave = None
         self._mwave = None
+        self._pwave = None
         self._trace = None
         self._probe_order: list[str] = []
         self._mic_out = None
@@ -286,11 +291,15 @@ class FDTDSolver:
         _native.call("fdtd_ctx_set_counters", ctx, _native.ptr(self._step_dev), _native.ptr(self._health))
         tiling = self._tiling or pick_tiling(self.shape, not self._grid.is_uniform, False)
         _native.call("fdtd_ctx_set_tiling", ctx, *tiling)
+        _native.call("fdtd_ctx_set_multi_step", ctx, int(self._tiling is None))
 
     def set_tiling(self, rows: int, planes: int, stack: int = 1) -> None:
         """Launch shape of the fused kernel: rows per wave, planes per wave and
-        waves per j-stack (halo rows shared through LDS)."""
+        waves per j-stack (halo rows shared through LDS). A solve whose launch
+        shape is given takes every step with that kernel; by default step_n
+        takes three steps per pass where the solve allows it."""
         self._tiling = normalize_tiling((rows, planes, stack))
+        _native.call("fdtd_ctx_set_multi_step", self._ctx, 0)
         _native.call("fdtd_ctx_set_tiling", self._ctx, *self._tiling)
 
     @property
@@ -666,6 +675,20 @@ class FDTDSolver:
             _native.call("fdtd_ctx_set_microphones", self._ctx, 0, None, None, None, None, 0)
         self._mic_out = new_mic
         self._mic_order = mics
+        kind, a, b = self._source_arrays(srcs)
+        _native.call("fdtd_ctx_set_sources", self._ctx, len(srcs), kind.ctypes.data, a.ctypes.data,
+                     b.ctypes.data, _native.ptr(self._wave), cap)
+        flat = np.array([np.ravel_multi_index(self._probes[n].position, self.shape) for n in names] or [0],
+                        dtype=np.int64)
+        _native.call("fdtd_ctx_set_probes", self._ctx, len(names), flat.ctypes.data,
+                     _native.ptr(self._trace), cap)
+        self._set_table_sources(table, names, cap)
+        self._set_pass_sources(table, cap)
+        self._cap = cap
+        self._dirty_sources = False
+
+    def _source_arrays(self, srcs: list) -> tuple[NDArray, NDArray, NDArray]:
+        """kind, a, b of point and plane sources as the C ABI takes them."""
         kind, a, b = [], [], []
         for s in srcs:
             if s.source_type == "point":
@@ -677,18 +700,22 @@ class FDTDSolver:
                 kind.append(1)
                 a.append(int(s.position["axis"]))
                 b.append(int(s.position["index"]))
-        kind = np.array(kind or [0], dtype=np.int32)
-        a = np.array(a or [0], dtype=np.int64)
-        b = np.array(b or [0], dtype=np.int64)
-        _native.call("fdtd_ctx_set_sources", self._ctx, len(srcs), kind.ctypes.data, a.ctypes.data,
-                     b.ctypes.data, _native.ptr(self._wave), cap)
-        flat = np.array([np.ravel_multi_index(self._probes[n].position, self.shape) for n in names] or [0],
-                        dtype=np.int64)
-        _native.call("fdtd_ctx_set_probes", self._ctx, len(names), flat.ctypes.data,
-                     _native.ptr(self._trace), cap)
-        self._set_table_sources(table, names, cap)
-        self._cap = cap
-        self._dirty_sources = False
+        return (np.array(kind or [0], dtype=np.int32), np.array(a or [0], dtype=np.int64),
+                np.array(b or [0], dtype=np.int64))
+
+    def _set_pass_sources(self, table: list, cap: int) -> None:
+        """The whole source list for multi-step passes when some of it is in the
+        per-cell tables (z planes): a pass adds up to SWEEP_SOURCES point and
+        plane sources of any axis itself, in list order."""
+        self._pwave = None
+        if (not table or len(self._sources) > SWEEP_SOURCES
+                or any(s.source_type == "membrane" for s in self._sources)):
+            return
+        torch = _torch()
+        self._pwave = torch.cat([w for w in (self._wave, self._mwave) if w is not None]).contiguous()
+        kind, a, b = self._source_arrays(self._sources)
+        _native.call("fdtd_ctx_set_pass_sources", self._ctx, len(self._sources), kind.ctypes.data, a.ctypes.data,
+                     b.ctypes.data, _native.ptr(self._pwave), cap)
 
     def _table_cells(self, src, air: NDArray[np.bool_]) -> tuple[NDArray, NDArray, int]:
         """(flat cells, float64 weights, field) of one table source: the air
@@ -841,7 +868,10 @@ class FDTDSolver:
         return float(ms.value)
 
     def step_n(self, n: int, graph_chunk: int = 0) -> None:
-        """Advance n steps on the device without host round trips.
+        """Advance n steps on the device without host round trips, three steps
+        per pass over the fields where the solve allows it (see
+        fdtd_ctx_set_multi_step), the rest one by one; the results are the
+        same bit for bit.
 
         graph_chunk = 0 (the default) enqueues the steps' kernels one by one;
         graph_chunk = m replays a captured hipGraph of m steps. Measured on

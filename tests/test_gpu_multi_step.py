@@ -1,0 +1,105 @@
+"""Multi-step passes (three steps per sweep over the fields) against the CPU
+oracle, bit for bit: grids at the edges of the windows, every source kind the
+passes take, step counts with each remainder, and graph replays. The step
+kernels keep the oracle's operations and their order, so the tolerance is 0."""
+
+import numpy as np
+import pytest
+
+from helpers import make_solver, oracle_problem, seeded_scenario
+from oracle import cpu
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = ("p", "vx", "vy", "vz")
+
+# nz of every remainder by 4; one and several k segments; rows that fill their
+# windows exactly and by one more; fewer planes than a pass has steps
+SHAPES = [(26, 37, 70), (13, 41, 33), (9, 25, 130), (3, 20, 31), (12, 61, 1030), (31, 19, 12), (40, 26, 64)]
+
+
+def _same(got, want, what):
+    got = np.asarray(got)
+    assert got.shape == want.shape, what
+    assert np.array_equal(got, want), f"{what}: {int((got != want).sum())} of {want.size} differ"
+
+
+def _compare(sc, s, n, st_o, tr_o):
+    tr = s.get_probe_data()
+    for q in range(len(sc.probes)):
+        _same(tr[f"probe{q}"], tr_o[:, q], f"probe{q}")
+    for k in FIELDS:
+        _same(getattr(s, k), st_o[k], k)
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("steps", [3, 31, 32])
+def test_pass_bitexact(oracle_lib, shape, steps):
+    print(f"[pass] {shape} {steps}", flush=True)
+    big = min(shape) >= 12
+    sc = seeded_scenario(5, shape=shape, pml=3 if big else 0, geometry=big)
+    st_o, tr_o = cpu.run(oracle_problem(sc, steps), steps)
+    s = make_solver(sc)
+    s.step_n(steps)
+    _compare(sc, s, steps, st_o, tr_o)
+
+
+@pytest.mark.parametrize("nonuniform", [False, True])
+@pytest.mark.parametrize("axes", [(0,), (1,), (2,), (2, 0, 1)])
+def test_pass_plane_sources(oracle_lib, axes, nonuniform):
+    """Plane sources of each axis, z planes (which single steps add from tables) among them."""
+    print(f"[pass] planes {axes} nonuniform={nonuniform}", flush=True)
+    sc = seeded_scenario(6, shape=(22, 38, 52), pml=4, nonuniform=nonuniform)
+    for ax in axes:
+        sc.sources.append(("plane", ax, 7 + ax, 7000.0 + 500 * ax))
+    sc.sources.append(("point", sc.sources[0][1], 5000.0))
+    sc.probes.append((11, 8, 9))
+    n = 26
+    st_o, tr_o = cpu.run(oracle_problem(sc, n), n)
+    s = make_solver(sc)
+    s.step_n(5)
+    s.step()
+    s.step_n(n - 6)
+    _compare(sc, s, n, st_o, tr_o)
+
+
+def test_pass_many_probes_of_one_window(oracle_lib):
+    """64 probes, the most a pass records, close together and on every wall of the grid."""
+    sc = seeded_scenario(7, shape=(24, 30, 44), pml=4)
+    rng = np.random.default_rng(1)
+    sc.probes = [tuple(int(v) for v in rng.integers((8, 8, 8), (14, 14, 14))) for _ in range(56)]
+    sc.probes += [(i, j, k) for i in (0, 23) for j in (0, 29) for k in (0, 43)]
+    n = 21
+    st_o, tr_o = cpu.run(oracle_problem(sc, n), n)
+    s = make_solver(sc)
+    s.step_n(n)
+    _compare(sc, s, n, st_o, tr_o)
+
+
+def test_pass_graph_replays(oracle_lib):
+    """Captured chunks (two passes and a single step each), replayed between eager steps."""
+    sc = seeded_scenario(8, shape=(25, 33, 47), pml=4)
+    n = 7 * 4 + 5 + 7 * 3
+    st_o, tr_o = cpu.run(oracle_problem(sc, n), n)
+    s = make_solver(sc)
+    s.step_n(28, graph_chunk=7)
+    s.step_n(5)
+    s.synchronize()
+    s.step_n(21, graph_chunk=7)
+    _compare(sc, s, n, st_o, tr_o)
+
+
+def test_pass_keeps_initial_values(oracle_lib):
+    """Fields written by the caller, last faces (which keep their velocity) and
+    solid cells among them, evolve as single steps take them."""
+    rng = np.random.default_rng(4)
+    sc = seeded_scenario(9, shape=(19, 23, 41), pml=3)
+    one, three = make_solver(sc, tiling=(2, 2)), make_solver(sc)
+    for k in FIELDS:
+        v = rng.standard_normal(sc.shape).astype(np.float32)
+        setattr(one, k, v)
+        setattr(three, k, v)
+    one.step_n(18)
+    three.step_n(18)
+    for k in FIELDS:
+        _same(getattr(three, k), getattr(one, k), k)
