@@ -20,6 +20,8 @@ hipError_t launch_fused(const FusedArgs& a, int rows, int stack, bool nu, bool a
                         hipStream_t st, hipEvent_t ev_before, hipEvent_t ev_after, const BoundarySet* bnd);
 bool pick_pass_tile(int nx, int ny, int nz, PassTile& best);
 hipError_t launch_pass(const FusedArgs& a, bool nu, const PassTile& m, hipStream_t st);
+int64_t patch_floats(const FusedArgs& a, int64_t off[3]);
+hipError_t launch_patch(const FusedArgs& a, bool nu, const PatchArgs& pt, hipStream_t st);
 hipError_t launch_advance(int64_t* step, int n, hipStream_t st);
 hipError_t launch_stream_ceiling(const FusedArgs& a, hipStream_t st);
 hipError_t launch_stream_march(const FusedArgs& a, int rows, int planes, hipStream_t st);
@@ -128,6 +130,9 @@ struct fdtd_ctx {
     bool multi_step = false, have_pass_src = false;
     bool tile_known = false, tile_ok = false;
     PassTile tile{};
+    bool have_patch = false;           // scratch for the poles' cells of a pass
+    PatchArgs patch{};
+    DevBuf patch_buf;
 };
 
 extern "C" {
@@ -169,7 +174,7 @@ int fdtd_ctx_destroy(fdtd_ctx* c) {
     if (c->mic_w_dev) (void)hipFree(c->mic_w_dev);
     if (c->mic_f64_dev) (void)hipFree(c->mic_f64_dev);
     for (fdtd_ctx::DevBuf* b : {&c->ade_cells, &c->m_cell, &c->m_estart, &c->m_esrc, &c->m_efield, &c->m_eweight, &c->m_pstart,
-                                &c->m_pidx, &c->ade_poles, &c->probes})
+                                &c->m_pidx, &c->ade_poles, &c->probes, &c->patch_buf})
         if (b->p) (void)hipFree(b->p);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
@@ -402,16 +407,20 @@ int fdtd_ctx_set_microphones(fdtd_ctx* c, int n, const int32_t* idx, const doubl
     return 0;
 }
 
-// Copy a host table into an owned device buffer (set-up only: grows with
-// hipMalloc when needed; the copy is synchronous).
+// Owned device buffers of the set-up calls: reserve grows one with hipMalloc when
+// needed, upload copies a host table into it (synchronously).
+static int reserve(fdtd_ctx::DevBuf& b, size_t bytes) {
+    if (bytes <= b.bytes) return 0;
+    if (b.p) (void)hipFree(b.p);
+    b.p = nullptr;
+    b.bytes = 0;
+    if (int rc = check(hipMalloc(&b.p, bytes), "hipMalloc")) return rc;
+    b.bytes = bytes;
+    return 0;
+}
+
 static int upload(fdtd_ctx::DevBuf& b, const void* host, size_t bytes) {
-    if (bytes > b.bytes) {
-        if (b.p) (void)hipFree(b.p);
-        b.p = nullptr;
-        b.bytes = 0;
-        if (int rc = check(hipMalloc(&b.p, bytes), "hipMalloc")) return rc;
-        b.bytes = bytes;
-    }
+    if (int rc = reserve(b, bytes)) return rc;
     if (bytes) return check(hipMemcpy(b.p, host, bytes, hipMemcpyHostToDevice), "hipMemcpy");
     return 0;
 }
@@ -527,6 +536,7 @@ int fdtd_ctx_set_ade(fdtd_ctx* c, int n_pole, const int32_t* mat_id, const int32
     // when the call succeeds, and a failed call leaves it without poles (never
     // with a pole count over stale tables).
     c->a.n_pole = 0;
+    c->have_patch = false;
     if (n_pole == 0) return 0;
     if (!mat_id || !target || !lorentz || !pa || !pb || !pd || !corr || !material || !lo || !hi || !J)
         return fail(-2, "bad ADE arrays");
@@ -589,6 +599,17 @@ int fdtd_ctx_set_ade(fdtd_ctx* c, int n_pole, const int32_t* mat_id, const int32
     if (int rc = upload(c->ade_poles, poles.data(), sizeof(AdePole) * poles.size())) return rc;
     a.poles = static_cast<const AdePole*>(c->ade_poles.p);
     a.n_pole = n_pole;
+    if (c->multi_step) {
+        int64_t off[3];
+        const int64_t floats = patch_floats(a, off);
+        // without room for the scratch the solve steps one by one
+        if (floats > 0 && reserve(c->patch_buf, sizeof(float) * static_cast<size_t>(floats)) != 0) (void)hipGetLastError();
+        else if (floats > 0) {
+            float* base = static_cast<float*>(c->patch_buf.p);
+            c->patch = PatchArgs{{base + off[0], base + off[1]}, base + off[2]};
+            c->have_patch = true;
+        }
+    }
     c->a = a;
     return 0;
 }
@@ -625,8 +646,9 @@ static int ready(fdtd_ctx* c) {
 // step adds around the sweep has to be in the pass as well, or absent.
 static bool pass_allowed(fdtd_ctx* c) {
     const FusedArgs& a = c->a;
-    if (!c->multi_step || a.n_pole > 0 || a.n_mic > 0 || c->bnd.n > 0 || a.n_probe > kSweepProbes) return false;
+    if (!c->multi_step || a.n_mic > 0 || c->bnd.n > 0 || a.n_probe > kSweepProbes) return false;
     if (a.n_mcell > 0 && !c->have_pass_src) return false;
+    if (a.n_pole > 0 && !c->have_patch) return false;
     if (!c->tile_known) {
         c->tile_known = true;
         c->tile_ok = pick_pass_tile(a.nx, a.ny, a.nz, c->tile);
@@ -644,6 +666,8 @@ static int enqueue_steps(fdtd_ctx* c, int n) {
         for (; n - s >= kPassSteps; s += kPassSteps) {
             pa.koff = s;
             if (int rc = check(launch_pass(pa, c->nonuniform, c->tile, c->stream), "multi-step pass launch")) return rc;
+            if (pa.n_pole > 0)
+                if (int rc = check(launch_patch(pa, c->nonuniform, c->patch, c->stream), "patch launch")) return rc;
         }
     }
     for (; s < n; ++s) {

@@ -198,6 +198,12 @@ struct PassTile {
     int nwg;                        // workgroups: windows x ceil(nx / units)
 };
 
+// Scratch of the cells such a pass leaves to single steps (k_patch_step).
+struct PatchArgs {
+    float* box[kPassSteps - 1];     // [4][cells] of the material box grown after steps 1 and 2
+    float* J;                       // [n_pole][box cells]: the density poles' J of step 2
+};
+
 // The boundary planes of a context (host side of a launch).
 struct BoundarySet {
     int n = 0;

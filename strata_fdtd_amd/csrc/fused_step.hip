@@ -33,6 +33,7 @@
 
 #include <algorithm>
 
+#include "ade_device.hpp"
 #include "fdtd_common.hpp"
 
 namespace fdtd_amd {
@@ -468,16 +469,6 @@ __global__ void k_batch_advance(const FusedArgs* __restrict__ table, const int* 
 }
 
 // ---- ADE --------------------------------------------------------------------
-__device__ __forceinline__ int64_t box_index(const FusedArgs& a, int i, int j, int k) {
-    const int by = a.box_hi[1] - a.box_lo[1], bz = a.box_hi[2] - a.box_lo[2];
-    return ((static_cast<int64_t>(i - a.box_lo[0]) * by) + (j - a.box_lo[1])) * bz + (k - a.box_lo[2]);
-}
-
-__device__ __forceinline__ int64_t box_cells(const FusedArgs& a) {
-    return static_cast<int64_t>(a.box_hi[0] - a.box_lo[0]) * (a.box_hi[1] - a.box_lo[1]) *
-           (a.box_hi[2] - a.box_lo[2]);
-}
-
 // Density-pole auxiliary update over the ADE box, run before the sweep of the
 // same time step (J <- a J + b p, Lorentz with history), ade.cpp:25-166.
 __device__ __forceinline__ void ade_density_part(const FusedArgs& a, int64_t first, int64_t stride) {
@@ -499,16 +490,8 @@ __device__ __forceinline__ void ade_density_part(const FusedArgs& a, int64_t fir
         for (int q = 0; q < a.n_pole; ++q) {
             const AdePole pl = pole_at(a.poles, q);
             if (pl.target != 0 || pl.mat != m) continue;
-            float* Jq = a.J + q * box_n;
-            if (!pl.lorentz) {
-                Jq[b] = pl.a * Jq[b] + pl.b * pv;
-            } else {
-                float* Jp = a.Jprev + q * box_n;
-                const float j0v = Jq[b], j1v = Jp[b];
-                const float jn = pl.a * j0v + pl.b * j1v + pl.d * pv;
-                Jp[b] = j0v;
-                Jq[b] = jn;
-            }
+            float* Jq = a.J + q * box_n + b;
+            *Jq = ade_recur(pl, *Jq, pl.lorentz ? a.Jprev + q * box_n + b : nullptr, pv);
         }
     }
 }
@@ -518,127 +501,42 @@ __global__ void k_ade_density(const FusedArgs a) {
                      static_cast<int64_t>(gridDim.x) * blockDim.x);
 }
 
-// v' of the face between cells lo (flat c) and hi (c + step along `axis`), with
-// the density-pole correction (Debye poles first, then Lorentz, ade.cpp:240-401).
-template <bool NU>
-__device__ __forceinline__ float ade_face(const FusedArgs& a, const float* __restrict__ P,
-                                          const float* __restrict__ V, int axis, int i, int j, int k,
-                                          int64_t c, int64_t step) {
-    const int n_ax = axis == 0 ? a.nx : (axis == 1 ? a.ny : a.nz);
-    const int idx = axis == 0 ? i : (axis == 1 ? j : k);
-    const float vo = V[c];
-    if (idx + 1 >= n_ax) return vo;  // last face: not updated, not masked
-    const float cf = NU ? a.cv * a.ifc[axis][idx] : a.cv;
-    float v = vo + cf * (P[c + step] - P[c]);
-    const int m_lo = a.material[c], m_hi = a.material[c + step];
-    if (m_lo && m_lo == m_hi) {
-        const int64_t box_n = box_cells(a);
-        const int ih = i + (axis == 0), jh = j + (axis == 1), kh = k + (axis == 2);
-        for (int pass = 0; pass < 2; ++pass)
-            for (int q = 0; q < a.n_pole; ++q) {
-                const AdePole pl = pole_at(a.poles, q);
-                if (pl.target != 0 || pl.lorentz != pass || pl.mat != m_lo) continue;
-                const float* Jq = a.J + q * box_n;
-                v += pl.corr * (Jq[box_index(a, ih, jh, kh)] - Jq[box_index(a, i, j, k)]);
-            }
-    }
-    const uint32_t open = axis == 0 ? FDTD_FLAG_OPEN_X : (axis == 1 ? FDTD_FLAG_OPEN_Y : FDTD_FLAG_OPEN_Z);
-    return (a.flags[c] & open) ? v : 0.f;
-}
-
 // Full ADE update of every pole-material cell in the box, from the input set,
 // overwriting what the plain sweep wrote for those cells (see file comment).
 template <bool NU>
 __global__ void k_ade_fixup(const FusedArgs a) {
-    const int ny = a.ny, nz = a.nz;
     const int by = a.box_hi[1] - a.box_lo[1], bz = a.box_hi[2] - a.box_lo[2];
-    const int64_t box_n = box_cells(a);
     const int64_t s = *a.step_ptr + a.koff;
     if (s >= a.step_limit) return;
     const int par = static_cast<int>(s & 1);
-    const float* __restrict__ P = par ? a.f[1][0] : a.f[0][0];
-    const float* __restrict__ VX = par ? a.f[1][1] : a.f[0][1];
-    const float* __restrict__ VY = par ? a.f[1][2] : a.f[0][2];
-    const float* __restrict__ VZ = par ? a.f[1][3] : a.f[0][3];
-    float* __restrict__ Po = par ? a.f[0][0] : a.f[1][0];
-    float* __restrict__ VXo = par ? a.f[0][1] : a.f[1][1];
-    float* __restrict__ VYo = par ? a.f[0][2] : a.f[1][2];
-    float* __restrict__ VZo = par ? a.f[0][3] : a.f[1][3];
-    const int64_t sy = nz, sx = static_cast<int64_t>(ny) * nz;
-    const int64_t n_visit = a.ade_cells ? a.n_ade_cells : box_n;
+    FieldView S{{}, 0, 0, 0, a.ny, a.nz};
+    for (int g = 0; g < 4; ++g) S.f[g] = a.f[par][g];
+    float* __restrict__ Po = a.f[par ^ 1][0];
+    float* __restrict__ VXo = a.f[par ^ 1][1];
+    float* __restrict__ VYo = a.f[par ^ 1][2];
+    float* __restrict__ VZo = a.f[par ^ 1][3];
+    const int64_t n_visit = a.ade_cells ? a.n_ade_cells : box_cells(a);
     for (int64_t e = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; e < n_visit;
          e += static_cast<int64_t>(gridDim.x) * blockDim.x) {
         const int64_t b = a.ade_cells ? static_cast<int64_t>(a.ade_cells[e]) : e;
         const int k = static_cast<int>(b % bz) + a.box_lo[2];
         const int j = static_cast<int>((b / bz) % by) + a.box_lo[1];
         const int i = static_cast<int>(b / (static_cast<int64_t>(by) * bz)) + a.box_lo[0];
-        const int64_t c = lin(i, j, k, ny, nz);
+        const int64_t c = lin(i, j, k, a.ny, a.nz);
         const int m = a.material[c];
-        bool has_pole = false;
-        for (int q = 0; q < a.n_pole; ++q) has_pole |= pole_at(a.poles, q).mat == m;
-        if (!m || !has_pole) continue;
-        const uint32_t f = a.flags[c];
-        const float vxn = ade_face<NU>(a, P, VX, 0, i, j, k, c, sx);
-        const float vyn = ade_face<NU>(a, P, VY, 1, i, j, k, c, sy);
-        const float vzn = ade_face<NU>(a, P, VZ, 2, i, j, k, c, 1);
-        const float vxm = i > 0 ? ade_face<NU>(a, P, VX, 0, i - 1, j, k, c - sx, sx) : 0.f;
-        const float vym = j > 0 ? ade_face<NU>(a, P, VY, 1, i, j - 1, k, c - sy, sy) : 0.f;
-        const float vzm = k > 0 ? ade_face<NU>(a, P, VZ, 2, i, j, k - 1, c - 1, 1) : 0.f;
-        const float dvx = vxn - vxm, dvy = vyn - vym, dvz = vzn - vzm;
-        const float icx = NU ? a.icl[0][i] : 1.f, icy = NU ? a.icl[1][j] : 1.f, icz = NU ? a.icl[2][k] : 1.f;
-        // modulus poles: source is the native divergence of v'
-        const float ix = NU ? icx : a.ade_inv_dx, iy = NU ? icy : a.ade_inv_dx, iz = NU ? icz : a.ade_inv_dx;
-        float dA = dvx * ix;
-        dA += dvy * iy;
-        dA += dvz * iz;
-        for (int pass = 0; pass < 2; ++pass)
-            for (int q = 0; q < a.n_pole; ++q) {
-                const AdePole pl = pole_at(a.poles, q);
-                if (pl.target != 1 || pl.lorentz != pass || pl.mat != m) continue;
-                float* Jq = a.J + q * box_n;
-                if (!pass) {
-                    Jq[b] = pl.a * Jq[b] + pl.b * dA;
-                } else {
-                    float* Jp = a.Jprev + q * box_n;
-                    const float j0v = Jq[b], j1v = Jp[b];
-                    const float jn = pl.a * j0v + pl.b * j1v + pl.d * dA;
-                    Jp[b] = j0v;
-                    Jq[b] = jn;
-                }
-            }
-        float pnew;
-        if (NU) pnew = P[c] + a.cp * (((icx * dvx) + (icy * dvy)) + (icz * dvz));
-        else pnew = P[c] + a.cp * ((dvx + dvy) + dvz);
-        for (int pass = 0; pass < 2; ++pass)
-            for (int q = 0; q < a.n_pole; ++q) {
-                const AdePole pl = pole_at(a.poles, q);
-                if (pl.target != 1 || pl.lorentz != pass || pl.mat != m) continue;
-                pnew += pl.corr * a.J[q * box_n + b];
-            }
-        if (!(f & FDTD_FLAG_AIR)) pnew = 0.f;
-        const float dx = a.dec[0][i], dy = a.dec[1][j], dz = a.dec[2][k];
-        float ps = ((pnew * dx) * dy) * dz;
-        if (s < a.wave_len && (f & FDTD_FLAG_AIR)) {
-            for (int q = 0; q < a.n_src; ++q) {
-                bool on;
-                if (a.src_kind[q] == 0) {
-                    on = a.src_i[q] == i && a.src_j[q] == j && a.src_k[q] == k;
-                } else {
-                    const int ax = a.src_i[q], id = a.src_j[q];
-                    on = ax == 0 ? id == i : (ax == 1 ? id == j : id == k);
-                }
-                if (on) ps = static_cast<float>(static_cast<double>(ps) + a.wave[q * a.wave_len + s]);
-            }
-        }
-        Po[c] = ps;
-        VXo[c] = vxn * dx;
-        VYo[c] = vyn * dy;
-        VZo[c] = vzn * dz;
+        if (!has_pole(a, m)) continue;
+        float o[4];
+        ade_cell<NU>(a, S, a.J, i, j, k, m, o);
+        if (s < a.wave_len && (a.flags[c] & FDTD_FLAG_AIR)) o[0] = ade_sources(a, i, j, k, s, o[0]);
+        Po[c] = o[0];
+        VXo[c] = o[1];
+        VYo[c] = o[2];
+        VZo[c] = o[3];
         if (s < a.trace_len)
             for (int q = 0; q < a.n_sweep_probe; ++q)
                 if (a.probe_ijk[3 * q] == i && a.probe_ijk[3 * q + 1] == j && a.probe_ijk[3 * q + 2] == k) {
-                    a.trace[s * a.n_probe + q] = ps;
-                    if (!isfinite(ps)) atomicOr(a.health, 1u);
+                    a.trace[s * a.n_probe + q] = o[0];
+                    if (!isfinite(o[0])) atomicOr(a.health, 1u);
                 }
     }
 }
@@ -839,6 +737,19 @@ int fused_grid(FusedArgs& a, int rows, int planes, int stack) {
     return blocks;
 }
 
+// blocks of the ADE kernels over the listed (or all) box cells
+static int ade_blocks(const FusedArgs& a) {
+    const int64_t bn = a.ade_cells ? a.n_ade_cells
+                                   : static_cast<int64_t>(a.box_hi[0] - a.box_lo[0]) *
+                                         (a.box_hi[1] - a.box_lo[1]) * (a.box_hi[2] - a.box_lo[2]);
+    return static_cast<int>(std::min<int64_t>(std::max<int64_t>((bn + 255) / 256, 1), 1 << 16));
+}
+
+hipError_t launch_density(const FusedArgs& a, hipStream_t st) {
+    hipLaunchKernelGGL(k_ade_density, dim3(ade_blocks(a)), dim3(256), 0, st, a);
+    return hipGetLastError();
+}
+
 // One full step: [ADE density] -> fused sweep -> [ADE fix-up] -> [boundary
 // planes] -> [table sources] -> [probes past the sweep's] -> [microphones].
 // ev_before / ev_after (optional) are recorded around the sweep alone, for
@@ -848,17 +759,12 @@ hipError_t launch_fused(const FusedArgs& a_in, int rows, int stack, bool nu, boo
     FusedArgs a = a_in;
     a.sweep_blocks = blocks;
     a.dens_blocks = 0;
-    int box_blocks = 1;
+    const int box_blocks = ade ? ade_blocks(a) : 1;
     if (ade) {
-        const int64_t bn = a.ade_cells ? a.n_ade_cells
-                                       : static_cast<int64_t>(a.box_hi[0] - a.box_lo[0]) *
-                                             (a.box_hi[1] - a.box_lo[1]) * (a.box_hi[2] - a.box_lo[2]);
-        box_blocks = static_cast<int>(std::min<int64_t>(std::max<int64_t>((bn + 255) / 256, 1), 1 << 16));
         if (stack == 1) {
             a.dens_blocks = box_blocks;  // run inside the sweep launch (k_fused_step)
         } else {
-            hipLaunchKernelGGL(k_ade_density, dim3(box_blocks), dim3(256), 0, st, a);
-            hipError_t e = hipGetLastError();
+            hipError_t e = launch_density(a, st);
             if (e != hipSuccess) return e;
         }
     }

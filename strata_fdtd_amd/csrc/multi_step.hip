@@ -30,6 +30,7 @@
 #include <algorithm>
 #include <climits>
 
+#include "ade_device.hpp"
 #include "fdtd_common.hpp"
 
 namespace fdtd_amd {
@@ -425,6 +426,94 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     }
 }
 
+// ---- ADE patch ------------------------------------------------------------------
+// A pass takes every cell as plain air. Poles change the cells of their material
+// after one step and those up to t - 1 cells around them after t, so the pass is
+// wrong on the material's box grown by two cells, and only there. Those cells are
+// stepped one step at a time from the same input state: step 1 on the box grown by
+// four cells into dense scratch, step 2 on it grown by three, step 3 on it grown by
+// two into the output, over what the pass wrote. The scratch stays in the caches
+// (the 512^3 enclosure's 81^3 box: 23 MB per step).
+template <bool NU>
+__global__ __launch_bounds__(256) void k_patch_step(const FusedArgs a, const PatchArgs pt, int t) {
+    const int64_t s = uni(a.step_ptr, 0) + a.koff + t;
+    const int par = static_cast<int>((s - t) & 1);
+    const int grow = 2 * kPassSteps - 2 - t;
+    int lo[3], n[3];
+    const int dim[3] = {a.nx, a.ny, a.nz};
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+        lo[x] = max(a.box_lo[x] - grow, 0);
+        n[x] = min(a.box_hi[x] + grow, dim[x]) - lo[x];
+    }
+    // the step's input: the state or the box of the step before, one cell larger
+    FieldView S{{}, 0, 0, 0, a.ny, a.nz};
+    if (t == 0) {
+        for (int g = 0; g < 4; ++g) S.f[g] = a.f[par][g];
+    } else {
+        const int from = grow + 1;
+        S.oi = max(a.box_lo[0] - from, 0);
+        S.oj = max(a.box_lo[1] - from, 0);
+        S.ok = max(a.box_lo[2] - from, 0);
+        S.ny = min(a.box_hi[1] + from, a.ny) - S.oj;
+        S.nz = min(a.box_hi[2] + from, a.nz) - S.ok;
+        const int64_t cells = static_cast<int64_t>(min(a.box_hi[0] + from, a.nx) - S.oi) * S.ny * S.nz;
+        for (int g = 0; g < 4; ++g) S.f[g] = pt.box[t - 1] + g * cells;
+    }
+    // probes in the region (the pass recorded what it made of them)
+    const GMEM int32_t* __restrict__ PIJK = gmem(a.probe_ijk);
+    const int lane = threadIdx.x & (kWave - 1);
+    bool in = lane < a.n_sweep_probe;
+    if (in)
+#pragma unroll
+        for (int x = 0; x < 3; ++x) {
+            const int v = PIJK[3 * lane + x];
+            in = in && v >= lo[x] && v < lo[x] + n[x];
+        }
+    const uint64_t probes = __builtin_amdgcn_ballot_w64(in);
+    const int64_t cells = static_cast<int64_t>(n[0]) * n[1] * n[2];
+    const uint32_t e = blockIdx.x * 256u + threadIdx.x;
+    if (e >= cells) return;
+    const uint32_t row = e / static_cast<uint32_t>(n[2]);
+    const int k = lo[2] + static_cast<int>(e - row * static_cast<uint32_t>(n[2]));
+    const int i = lo[0] + static_cast<int>(row / static_cast<uint32_t>(n[1]));
+    const int j = lo[1] + static_cast<int>(row % static_cast<uint32_t>(n[1]));
+    const int64_t c = lin(i, j, k, a.ny, a.nz);
+    int m = a.material[c];
+    if (!has_pole(a, m)) m = 0;
+    float o[4];
+    ade_cell<NU>(a, S, t == 1 ? pt.J : a.J, i, j, k, m, o);
+    if (s < a.wave_len && (a.flags[c] & FDTD_FLAG_AIR)) o[0] = ade_sources(a, i, j, k, s, o[0]);
+    if (t == kPassSteps - 1) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) a.f[par ^ 1][g][c] = o[g];
+    } else {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) pt.box[t][g * cells + e] = o[g];
+        // density poles' J of the next step, from this step's pressure: from a.J
+        // into pt.J and back, since neighbours still read this step's
+        if (m) {
+            const int64_t box_n = box_cells(a), b = box_index(a, i, j, k);
+            const float* from = t == 1 ? pt.J : a.J;
+            float* to = t == 1 ? a.J : pt.J;
+            for (int q = 0; q < a.n_pole; ++q) {
+                const AdePole po = pole_at(a.poles, q);
+                if (po.target != 0 || po.mat != m) continue;
+                to[q * box_n + b] = ade_recur(po, from[q * box_n + b],
+                                              po.lorentz ? a.Jprev + q * box_n + b : nullptr, o[0]);
+            }
+        }
+    }
+    for (uint64_t pm = probes; pm; pm &= pm - 1) {
+        const int q = __builtin_ctzll(pm);
+        if (uni(a.probe_ijk, 3 * q) == i && uni(a.probe_ijk, 3 * q + 1) == j && uni(a.probe_ijk, 3 * q + 2) == k &&
+            s < a.trace_len) {
+            a.trace[s * a.n_probe + q] = o[0];
+            if (!isfinite(o[0])) atomicOr(a.health, 1u);
+        }
+    }
+}
+
 // ---- host side -------------------------------------------------------------------
 constexpr int kCUs = 256;
 
@@ -504,6 +593,41 @@ static hipError_t launch_pass_t(const FusedArgs& a, const PassTile& m, hipStream
     else
         hipLaunchKernelGGL((k_multi_step<NU, NT, true>), dim3(blocks), dim3(NT), 0, st, a, m);
     return hipGetLastError();
+}
+
+static int64_t grown_cells(const FusedArgs& a, int grow) {
+    const int dim[3] = {a.nx, a.ny, a.nz};
+    int64_t n = 1;
+    for (int x = 0; x < 3; ++x) n *= std::min(a.box_hi[x] + grow, dim[x]) - std::max(a.box_lo[x] - grow, 0);
+    return n;
+}
+
+// Scratch floats of the patch: the boxes of steps 1 and 2, then the density
+// poles' second J; 0 where a pass is not worth its patch. A patch takes the
+// box's cells about as long as single steps of them take; beyond a third of the
+// grid that is most of what the pass saves.
+int64_t patch_floats(const FusedArgs& a, int64_t off[3]) {
+    const int64_t first = grown_cells(a, 2 * kPassSteps - 2), second = grown_cells(a, 2 * kPassSteps - 3);
+    if (3 * first > static_cast<int64_t>(a.nx) * a.ny * a.nz) return 0;
+    off[0] = 0;
+    off[1] = 4 * first;
+    off[2] = off[1] + 4 * second;
+    return off[2] + a.n_pole * grown_cells(a, 0);
+}
+
+hipError_t launch_density(const FusedArgs& a, hipStream_t st);
+
+// The cells a pass took wrongly (after it, on the same steps).
+hipError_t launch_patch(const FusedArgs& a, bool nu, const PatchArgs& pt, hipStream_t st) {
+    hipError_t e = launch_density(a, st);
+    for (int t = 0; t < kPassSteps && e == hipSuccess; ++t) {
+        const int64_t cells = grown_cells(a, 2 * kPassSteps - 2 - t);
+        const dim3 grid(static_cast<unsigned>((cells + 255) / 256));
+        if (nu) hipLaunchKernelGGL(k_patch_step<true>, grid, dim3(256), 0, st, a, pt, t);
+        else hipLaunchKernelGGL(k_patch_step<false>, grid, dim3(256), 0, st, a, pt, t);
+        e = hipGetLastError();
+    }
+    return e;
 }
 
 // Steps koff .. koff + kPassSteps - 1 of a chunk in one pass.

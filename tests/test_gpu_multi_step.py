@@ -103,3 +103,41 @@ def test_pass_keeps_initial_values(oracle_lib):
     three.step_n(18)
     for k in FIELDS:
         _same(getattr(three, k), getattr(one, k), k)
+
+
+POLES = {
+    "debye": [dict(kind="debye", target="density", tau=2e-5, dchi=0.5),
+              dict(kind="debye", target="modulus", tau=1e-5, dchi=0.3)],
+    "lorentz": [dict(kind="lorentz", target="modulus", w0=2 * np.pi * 3000, gamma=500.0, dchi=0.4),
+                dict(kind="lorentz", target="density", w0=2 * np.pi * 2000, gamma=300.0, dchi=0.2)],
+}
+
+
+@pytest.mark.parametrize("nonuniform", [False, True])
+@pytest.mark.parametrize("where", ["inside", "corner"])
+def test_pass_ade_patch(oracle_lib, where, nonuniform):
+    """Materials with poles in a pass: a sphere of two materials away from the
+    walls, or in a corner (its grown boxes are cut by the grid), with the source
+    and probes in, next to and away from it, over passes and single steps."""
+    print(f"[pass] ade {where} nonuniform={nonuniform}", flush=True)
+    shape = (36, 44, 60)
+    sc = seeded_scenario(10, shape=shape, pml=4, nonuniform=nonuniform)
+    c = np.array((15, 20, 30) if where == "inside" else (0, 43, 57))
+    g = np.indices(shape)
+    d2 = sum((g[x] - c[x]) ** 2 for x in range(3))
+    sc.material = np.where(d2 <= 20, np.where(g[2] > c[2], 2, 1), 0).astype(np.uint8)
+    sc.material[~sc.air] = 0
+    sc.materials = {1: POLES["debye"], 2: POLES["lorentz"] + POLES["debye"][:1]}
+    near = [tuple(int(v) for v in np.clip(c + d, 0, np.array(shape) - 1))
+            for d in ((0, 0, 0), (0, 0, 1), (6, 0, 0), (0, -7, 0), (3, -3, -2), (1, -1, 8))]
+    sc.probes += near + [(20, 5, 9)]
+    sc.sources.append(("point", near[3], 7000.0))
+    sc.sources.append(("point", near[1], 9000.0))
+    n = 29
+    st_o, tr_o = cpu.run(oracle_problem(sc, n), n)
+    s = make_solver(sc)
+    s.step_n(7)
+    s.step()
+    s.step_n(12, graph_chunk=6)
+    s.step_n(n - 20)
+    _compare(sc, s, n, st_o, tr_o)
