@@ -18,7 +18,7 @@ namespace fdtd_amd {
 int fused_grid(FusedArgs& a, int rows, int planes, int stack);
 hipError_t launch_fused(const FusedArgs& a, int rows, int stack, bool nu, bool ade, int blocks,
                         hipStream_t st, hipEvent_t ev_before, hipEvent_t ev_after, const BoundarySet* bnd);
-bool pick_pass_tile(int nx, int ny, int nz, PassTile& best);
+bool pick_pass_tile(int nx, int ny, int nz, int only_nt, double share, PassTile& best);
 hipError_t launch_pass(const FusedArgs& a, bool nu, const PassTile& m, hipStream_t st);
 int64_t patch_floats(const FusedArgs& a, int64_t off[3]);
 hipError_t launch_patch(const FusedArgs& a, bool nu, const PatchArgs& pt, hipStream_t st);
@@ -29,7 +29,9 @@ int energy_partials();
 hipError_t launch_energy(const FusedArgs& a, double* partial, double* out, hipStream_t st);
 hipError_t launch_centre_velocity(const FusedArgs& a, float* ox, float* oy, float* oz, hipStream_t st);
 hipError_t launch_batch(const FusedArgs* table, const int* offsets, const int* n_ptr, int cap_waves, int rows,
-                        bool nts, int koff, hipStream_t st);
+                        bool nts, int koff, int chunk, bool after_passes, hipStream_t st);
+hipError_t launch_batch_pass(const FusedArgs* table, const PassTile* tiles, const int* offsets, const int* n_ptr,
+                             int cap_wgs, bool nts, int koff, int chunk, hipStream_t st);
 hipError_t launch_batch_advance(const FusedArgs* table, const int* n_ptr, int cap_solves, int n, hipStream_t st);
 hipError_t phase_velocity(const float*, float*, float*, float*, int, int, int, float, const float*,
                           const float*, const float*, hipStream_t);
@@ -127,9 +129,12 @@ struct fdtd_ctx {
         const double* wave = nullptr;
         int64_t wave_len = 0;
     } pass_src;
-    bool multi_step = false, have_pass_src = false;
+    bool multi_step = false, padded = false, have_pass_src = false;
     bool tile_known = false, tile_ok = false;
     PassTile tile{};
+    // in a batch: the windows for a share of the chip of 1, 1/2, 1/4 .. 1/64
+    bool batch_tile_known[7] = {}, batch_tile_ok[7] = {};
+    PassTile batch_tile[7] = {};
     bool have_patch = false;           // scratch for the poles' cells of a pass
     PatchArgs patch{};
     DevBuf patch_buf;
@@ -203,6 +208,7 @@ int fdtd_ctx_set_grid(fdtd_ctx* c, int nx, int ny, int nz, int nonuniform, float
     drop_graph(c);
     c->a.nx = nx; c->a.ny = ny; c->a.nz = nz;
     c->tile_known = false;
+    std::fill(std::begin(c->batch_tile_known), std::end(c->batch_tile_known), false);
     c->have_pass_src = false;
     c->a.cv = cv; c->a.cp = cp;
     c->nonuniform = nonuniform != 0;
@@ -311,10 +317,12 @@ int fdtd_ctx_set_pass_sources(fdtd_ctx* c, int n, const int32_t* kind, const int
     return 0;
 }
 
-int fdtd_ctx_set_multi_step(fdtd_ctx* c, int on) {
+int fdtd_ctx_set_multi_step(fdtd_ctx* c, int mode) {
     if (!c) return fail(-1, "null context");
+    if (mode < 0 || mode > 2) return fail(-2, "multi-step mode must be 0, 1 or 2");
     drop_graph(c);
-    c->multi_step = on != 0;
+    c->multi_step = mode == 1;
+    c->padded = mode != 0;
     return 0;
 }
 
@@ -322,7 +330,7 @@ int fdtd_pass_tiling(int nx, int ny, int nz, int32_t* out) {
     if (!out) return fail(-1, "null output");
     if (nx < 2 || ny < 2 || nz < 2) return fail(-2, "grid %dx%dx%d: every axis needs >= 2 cells", nx, ny, nz);
     PassTile m{};
-    const bool ok = pick_pass_tile(nx, ny, nz, m);
+    const bool ok = pick_pass_tile(nx, ny, nz, 0, 1.0, m);
     const int32_t v[9] = {ok ? kPassSteps : 0, m.nt, m.kt, m.ko, m.rows, m.nseg, m.njt, m.units, m.nwg};
     std::copy(v, v + 9, out);
     return 0;
@@ -651,7 +659,7 @@ static bool pass_allowed(fdtd_ctx* c) {
     if (a.n_pole > 0 && !c->have_patch) return false;
     if (!c->tile_known) {
         c->tile_known = true;
-        c->tile_ok = pick_pass_tile(a.nx, a.ny, a.nz, c->tile);
+        c->tile_ok = pick_pass_tile(a.nx, a.ny, a.nz, 0, 1.0, c->tile);
     }
     return c->tile_ok;
 }
@@ -1025,18 +1033,23 @@ struct fdtd_batch {
     int rows = 4;
     int cap = 0;                        // solves the buffers hold
     FusedArgs* table_dev = nullptr;     // [cap]
-    int* meta_dev = nullptr;            // [cap + 2]: n, then offsets[0..n]
+    int* meta_dev = nullptr;            // [2 cap + 3]: n, offsets[0..n] of the waves, from cap + 2 those of
+                                        // the passes' workgroups
+    PassTile* tile_dev = nullptr;       // [cap]: windows of the passes
     FusedArgs* table_host[2] = {};      // pinned staging, used alternately
     int* meta_host[2] = {};
+    PassTile* tile_host[2] = {};
     hipEvent_t copied[2] = {};          // the staging buffer's last upload has run
     bool pending[2] = {};
     int stage = 0;
     int n = 0;
     int total_waves = 0;
+    int total_wgs = 0;                  // workgroups of a pass; 0: single steps only
     bool nts = true;                    // non-temporal stores (the solves exceed the cache)
     hipGraphExec_t graph = nullptr;
     int graph_steps = 0;
     int graph_waves = 0;                // wave capacity of the captured grid
+    int graph_wgs = 0;                  // workgroup capacity of its passes (0: none)
     bool graph_nts = true;
 };
 
@@ -1046,16 +1059,21 @@ static void batch_drop_graph(fdtd_batch* b) {
         b->graph = nullptr;
         b->graph_steps = 0;
         b->graph_waves = 0;
+        b->graph_wgs = 0;
     }
 }
 
 static void batch_free(fdtd_batch* b) {
     if (b->table_dev) (void)hipFree(b->table_dev);
     if (b->meta_dev) (void)hipFree(b->meta_dev);
+    if (b->tile_dev) (void)hipFree(b->tile_dev);
+    b->tile_dev = nullptr;
     for (int i = 0; i < 2; ++i) {
         if (b->table_host[i]) (void)hipHostFree(b->table_host[i]);
         if (b->meta_host[i]) (void)hipHostFree(b->meta_host[i]);
         b->table_host[i] = nullptr;
+        if (b->tile_host[i]) (void)hipHostFree(b->tile_host[i]);
+        b->tile_host[i] = nullptr;
         b->meta_host[i] = nullptr;
         b->pending[i] = false;
     }
@@ -1118,11 +1136,14 @@ int fdtd_batch_set(fdtd_batch* b, fdtd_ctx* const* ctxs, const int64_t* step_lim
         const int cap = std::max({n, 2 * b->cap, 16});
         batch_free(b);
         if (int rc = check(hipMalloc(&b->table_dev, sizeof(FusedArgs) * cap), "hipMalloc")) return rc;
-        if (int rc = check(hipMalloc(&b->meta_dev, sizeof(int) * (cap + 2)), "hipMalloc")) return rc;
+        if (int rc = check(hipMalloc(&b->meta_dev, sizeof(int) * (2 * cap + 3)), "hipMalloc")) return rc;
+        if (int rc = check(hipMalloc(&b->tile_dev, sizeof(PassTile) * cap), "hipMalloc")) return rc;
         for (int i = 0; i < 2; ++i) {
             if (int rc = check(hipHostMalloc(&b->table_host[i], sizeof(FusedArgs) * cap, 0), "hipHostMalloc"))
                 return rc;
-            if (int rc = check(hipHostMalloc(&b->meta_host[i], sizeof(int) * (cap + 2), 0), "hipHostMalloc"))
+            if (int rc = check(hipHostMalloc(&b->meta_host[i], sizeof(int) * (2 * cap + 3), 0), "hipHostMalloc"))
+                return rc;
+            if (int rc = check(hipHostMalloc(&b->tile_host[i], sizeof(PassTile) * cap, 0), "hipHostMalloc"))
                 return rc;
         }
         b->cap = cap;
@@ -1147,11 +1168,39 @@ int fdtd_batch_set(fdtd_batch* b, fdtd_ctx* const* ctxs, const int64_t* step_lim
         total += a.nwaves;
         meta[q + 2] = total;
     }
+    // the passes' windows, each solve's for its share of the chip
+    int* wgs = meta + b->cap + 2;
+    int total_wgs = 0;
+    bool passes = n > 0;
+    wgs[0] = 0;
+    for (int q = 0; q < n && passes; ++q) {
+        fdtd_ctx* c = ctxs[q];
+        const double part = static_cast<double>(c->a.nx) * c->a.ny * c->a.nz / static_cast<double>(cells);
+        int h = 0;
+        while (h < 6 && part < 0.7 / (1 << h)) ++h;
+        if (!c->batch_tile_known[h]) {
+            c->batch_tile_known[h] = true;
+            c->batch_tile_ok[h] = pick_pass_tile(c->a.nx, c->a.ny, c->a.nz, kBatchPassThreads, 1.0 / (1 << h),
+                                                 c->batch_tile[h]);
+        }
+        passes = c->padded && c->batch_tile_ok[h];
+        b->tile_host[i][q] = c->batch_tile[h];
+        total_wgs += c->batch_tile[h].nwg;
+        wgs[q + 1] = total_wgs;
+    }
+    if (!passes) total_wgs = 0;
+    if (n > 0) {
+        if (int rc = check(hipMemcpyAsync(b->tile_dev, b->tile_host[i], sizeof(PassTile) * n, hipMemcpyHostToDevice,
+                                          b->stream),
+                           "tile upload"))
+            return rc;
+    }
     if (n > 0)
         if (int rc = check(hipMemcpyAsync(b->table_dev, tab, sizeof(FusedArgs) * n, hipMemcpyHostToDevice, b->stream),
                            "table upload"))
             return rc;
-    if (int rc = check(hipMemcpyAsync(b->meta_dev, meta, sizeof(int) * (n + 2), hipMemcpyHostToDevice, b->stream),
+    if (int rc = check(hipMemcpyAsync(b->meta_dev, meta, sizeof(int) * (2 * b->cap + 3), hipMemcpyHostToDevice,
+                                      b->stream),
                        "offsets upload"))
         return rc;
     if (int rc = check(hipEventRecord(b->copied[i], b->stream), "event record")) return rc;
@@ -1159,15 +1208,29 @@ int fdtd_batch_set(fdtd_batch* b, fdtd_ctx* const* ctxs, const int64_t* step_lim
     b->stage ^= 1;
     b->n = n;
     b->total_waves = total;
+    b->total_wgs = total_wgs;
     b->nts = cells > kCacheResidentCells;
     return 0;
 }
 
-// n_steps launches (step koff = 0 .. n_steps - 1 of the chunk, each counted
-// from the solves' counters), then one launch that moves the counters.
-static int batch_enqueue(fdtd_batch* b, hipStream_t st, int n_steps, int cap_waves) {
-    for (int s = 0; s < n_steps; ++s)
-        if (int rc = check(launch_batch(b->table_dev, b->meta_dev + 1, b->meta_dev, cap_waves, b->rows, b->nts, s, st),
+// A chunk of n_steps steps of every solve: passes of kPassSteps steps where every
+// solve takes them (cap_wgs > 0), then the one or two steps they leave (to the
+// chunk's end or a solve's limit), or n_steps single steps; then one launch that
+// moves the counters. Steps are counted from the solves' counters.
+static int batch_enqueue(fdtd_batch* b, hipStream_t st, int n_steps, int cap_waves, int cap_wgs) {
+    int singles = n_steps;
+    const bool passes = cap_wgs > 0 && n_steps >= kPassSteps;
+    if (passes) {
+        for (int s = 0; s + kPassSteps <= n_steps; s += kPassSteps)
+            if (int rc = check(launch_batch_pass(b->table_dev, b->tile_dev, b->meta_dev + b->cap + 2, b->meta_dev, cap_wgs,
+                                                 b->nts, s, n_steps, st),
+                               "batch pass launch"))
+                return rc;
+        singles = kPassSteps - 1;
+    }
+    for (int s = 0; s < singles; ++s)
+        if (int rc = check(launch_batch(b->table_dev, b->meta_dev + 1, b->meta_dev, cap_waves, b->rows, b->nts, s, n_steps,
+                                        passes, st),
                            "batch step launch"))
             return rc;
     return check(launch_batch_advance(b->table_dev, b->meta_dev, b->cap, n_steps, st), "batch advance launch");
@@ -1178,12 +1241,15 @@ int fdtd_batch_step_n(fdtd_batch* b, int n_steps, int use_graph) {
     if (n_steps < 0) return fail(-2, "negative step count");
     if (b->n == 0 || n_steps == 0) return 0;
     DeviceGuard g(b->device);
-    if (!use_graph) return batch_enqueue(b, b->stream, n_steps, b->total_waves);
-    if (!b->graph || b->graph_steps != n_steps || b->graph_waves < b->total_waves || b->graph_nts != b->nts) {
+    if (!use_graph) return batch_enqueue(b, b->stream, n_steps, b->total_waves, b->total_wgs);
+    if (!b->graph || b->graph_steps != n_steps || b->graph_waves < b->total_waves || b->graph_nts != b->nts ||
+        b->graph_wgs < b->total_wgs || (b->graph_wgs > 0) != (b->total_wgs > 0)) {
         // capture with head room so that later tables of up to this many waves
         // replay it; a recapture for another reason keeps the capacity
         int cap_waves = b->graph_waves;
         if (cap_waves < b->total_waves) cap_waves = std::max(b->total_waves + b->total_waves / 2, b->graph_waves * 2);
+        int cap_wgs = b->total_wgs > 0 ? b->graph_wgs : 0;
+        if (cap_wgs < b->total_wgs) cap_wgs = std::max(b->total_wgs + b->total_wgs / 2, cap_wgs * 2);
         batch_drop_graph(b);
         hipStream_t cap = nullptr;
         if (int rc = check(hipStreamCreateWithFlags(&cap, hipStreamNonBlocking), "hipStreamCreate")) return rc;
@@ -1192,7 +1258,7 @@ int fdtd_batch_step_n(fdtd_batch* b, int n_steps, int use_graph) {
             (void)hipStreamDestroy(cap);
             return rc;
         }
-        int rc = batch_enqueue(b, cap, n_steps, cap_waves);
+        int rc = batch_enqueue(b, cap, n_steps, cap_waves, cap_wgs);
         hipError_t e = hipStreamEndCapture(cap, &gr);
         (void)hipStreamDestroy(cap);
         if (rc) { if (gr) (void)hipGraphDestroy(gr); return rc; }
@@ -1202,6 +1268,7 @@ int fdtd_batch_step_n(fdtd_batch* b, int n_steps, int use_graph) {
         if (int r3 = check(e, "graph instantiate")) return r3;
         b->graph_steps = n_steps;
         b->graph_waves = cap_waves;
+        b->graph_wgs = cap_wgs;
         b->graph_nts = b->nts;
     }
     return check(hipGraphLaunch(b->graph, b->stream), "graph launch");

@@ -187,6 +187,9 @@ struct FusedArgs {
 // reads field set s & 1; three is what the LDS holds for workgroups of 1024.
 constexpr int kPassSteps = 3;
 
+// Threads per workgroup of a batch's passes (one launch, one size).
+constexpr int kBatchPassThreads = 512;
+
 // Windows and work split of such a pass.
 struct PassTile {
     int nt;                         // threads per workgroup

@@ -421,8 +421,9 @@ __global__ __launch_bounds__(W * kWave) void k_fused_stack(const FusedArgs a) {
 }
 
 // Batched step: one launch advances every solve in `table` by one step, step
-// `koff` of a chunk whose first step is each solve's counter (the counters
-// move once per chunk, by k_batch_advance). Waves are dealt out by solve
+// `koff` of a chunk of `chunk` steps whose first step is each solve's counter
+// (the counters move once per chunk, by k_batch_advance). after_passes: the
+// chunk's multi-step passes went before, and koff counts from the steps they left. Waves are dealt out by solve
 // through the prefix sums `offsets` (n + 1 entries); a solve whose step
 // reached its limit is left untouched. Solves below 2^30 cells.
 // The number of solves is read from device memory (n_ptr), so a captured
@@ -432,7 +433,8 @@ __global__ __launch_bounds__(W * kWave) void k_fused_stack(const FusedArgs a) {
 // compiler picks unguided; measured about 8% faster on the 64-request sweep.
 template <int R, bool NTS>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_batch_step(
-    const FusedArgs* __restrict__ table, const int* __restrict__ offsets, const int* __restrict__ n_ptr, int koff) {
+    const FusedArgs* __restrict__ table, const int* __restrict__ offsets, const int* __restrict__ n_ptr, int koff,
+    int chunk, bool after_passes) {
     const int lane = threadIdx.x & (kWave - 1);
     // XCD-aware remap over the blocks the live table needs (the grid may be
     // larger): XCD x takes logical blocks [x * bpx, (x + 1) * bpx)
@@ -451,8 +453,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 8))) 
     }
     const FusedArgs& a = table[lo];
     const int w = gw - offsets[lo];
-    const int64_t s = *a.step_ptr + koff;
-    if (s >= a.step_limit) return;
+    const int64_t s0 = *a.step_ptr;
+    int64_t s = s0 + koff;
+    const int64_t end = min(a.step_limit, s0 + chunk);
+    if (after_passes && end > s0) s += (end - s0) / kPassSteps * kPassSteps;
+    if (s >= end) return;
     const int seg = w % a.nseg;
     const int t = w / a.nseg;
     fused_strip<R, false, 1, NTS, uint32_t, false>(a, s, seg, t % a.nstrip_j, t / a.nstrip_j, lane, nullptr, 0);
@@ -814,24 +819,33 @@ hipError_t launch_fused(const FusedArgs& a_in, int rows, int stack, bool nu, boo
 // `cap_waves` waves (the grid covers the capacity; n is read on the device).
 template <bool NTS>
 static hipError_t launch_batch_t(const FusedArgs* table, const int* offsets, const int* n_ptr, int blocks, int rows,
-                                 int koff, hipStream_t st) {
+                                 int koff, int chunk, bool after_passes, hipStream_t st) {
     switch (rows) {
-        case 2: hipLaunchKernelGGL((k_batch_step<2, NTS>), dim3(blocks), dim3(kBlock), 0, st, table, offsets, n_ptr, koff); break;
-        case 4: hipLaunchKernelGGL((k_batch_step<4, NTS>), dim3(blocks), dim3(kBlock), 0, st, table, offsets, n_ptr, koff); break;
-        case 8: hipLaunchKernelGGL((k_batch_step<8, NTS>), dim3(blocks), dim3(kBlock), 0, st, table, offsets, n_ptr, koff); break;
+        case 2:
+            hipLaunchKernelGGL((k_batch_step<2, NTS>), dim3(blocks), dim3(kBlock), 0, st, table, offsets, n_ptr, koff,
+                               chunk, after_passes);
+            break;
+        case 4:
+            hipLaunchKernelGGL((k_batch_step<4, NTS>), dim3(blocks), dim3(kBlock), 0, st, table, offsets, n_ptr, koff,
+                               chunk, after_passes);
+            break;
+        case 8:
+            hipLaunchKernelGGL((k_batch_step<8, NTS>), dim3(blocks), dim3(kBlock), 0, st, table, offsets, n_ptr, koff,
+                               chunk, after_passes);
+            break;
         default: return hipErrorInvalidValue;
     }
     return hipSuccess;
 }
 
-// Step koff of a chunk. nts: non-temporal stores (a batch whose solves
+// Step koff of a chunk of `chunk` steps (after_passes: of what its passes left). nts: non-temporal stores (a batch whose solves
 // together exceed the Infinity Cache), else ordinary stores.
 hipError_t launch_batch(const FusedArgs* table, const int* offsets, const int* n_ptr, int cap_waves, int rows,
-                        bool nts, int koff, hipStream_t st) {
+                        bool nts, int koff, int chunk, bool after_passes, hipStream_t st) {
     int blocks = (cap_waves + kBlockWaves - 1) / kBlockWaves;
     blocks = std::max(8, (blocks + 7) & ~7);
-    const hipError_t le = nts ? launch_batch_t<true>(table, offsets, n_ptr, blocks, rows, koff, st)
-                              : launch_batch_t<false>(table, offsets, n_ptr, blocks, rows, koff, st);
+    const hipError_t le = nts ? launch_batch_t<true>(table, offsets, n_ptr, blocks, rows, koff, chunk, after_passes, st)
+                              : launch_batch_t<false>(table, offsets, n_ptr, blocks, rows, koff, chunk, after_passes, st);
     if (le != hipSuccess) return le;
     return hipGetLastError();
 }

@@ -116,8 +116,11 @@ struct Stage {
     uint32_t f;
 };
 
+// The pass of steps s .. s + kPassSteps - 1 over one workgroup's windows: number
+// lb of the windows-by-chunks of `mt`, of the solve described at `ka`.
 template <bool NU, int NT, bool NTS>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_multi_step(const FusedArgs a, const PassTile mt) {
+__device__ __forceinline__ void pass_workgroup(const CMEM FusedArgs* ka, const PassTile& mt, int64_t s, int lb) {
+    const CMEM FusedArgs& a = *ka;
     constexpr int T = kPassSteps;
     __shared__ f4v sP[T][NT];
     __shared__ f4v sY[T][NT + 1];
@@ -127,7 +130,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     __shared__ f4v sK[NU ? 3 : 1][NU ? kMaxLanes : 1];
     const int tid = threadIdx.x;
     const int nx = a.nx, ny = a.ny, nz = a.nz;
-    const int64_t s = uni(a.step_ptr, 0) + a.koff;
     if (tid < T) {
         sY[tid][NT] = f4v{0.f, 0.f, 0.f, 0.f};  // the row below the window's first
         sZ[tid][NT] = 0.f;                      // the cell before its first lane
@@ -142,7 +144,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     GMEM float* __restrict__ VYo = gmem(par ? a.f[0][2] : a.f[1][2]);
     GMEM float* __restrict__ VZo = gmem(par ? a.f[0][3] : a.f[1][3]);
     const GMEM uint8_t* __restrict__ FL = gmem(a.flags);
-    const CMEM FusedArgs* ka = kernargs();
     const uint32_t sx = static_cast<uint32_t>(ny) * static_cast<uint32_t>(nz);
     const float cv = a.cv, cp = a.cp;
 
@@ -154,276 +155,311 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     const int ir = tid + 1 < NT ? tid + 1 : tid;           // next lane
     const int il = kl > 0 ? tid - 1 : NT;                  // previous lane
 
-    // XCD-aware order: hardware block b runs on XCD b mod 8, which takes a
-    // contiguous range of the (window, plane) units
-    const int lb = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
     const int nwin = mt.nseg * mt.njt;
-    if (lb < mt.nwg) {
-        const int chunk = lb / nwin, win = lb - chunk * nwin;
-        const int i0 = chunk * mt.units;
-        const int i1 = min(nx, i0 + mt.units);
-        const int seg = win % mt.nseg, jt = win / mt.nseg;
-        // window origin and the rows / lanes it stores
-        const int w0 = jt * (mt.rows - 2 * T);
-        const int jlo = jt == 0 ? 0 : w0 + T;
-        const int jhi = jt == mt.njt - 1 ? ny : w0 + mt.rows - T;
-        const int k0 = 4 * (seg == 0 ? 0 : seg * mt.ko - 1);
-        const int klo = 4 * seg * mt.ko;
-        const int khi = seg == mt.nseg - 1 ? nz : 4 * (seg + 1) * mt.ko;
-        const int j = w0 + row;
-        const int k = k0 + 4 * kl;
-        const bool ld = in_win && j < ny && k < nz;
-        const bool out = ld && j >= jlo && j < jhi && k >= klo && k < khi;
-        const int nv = nz - k;                               // 4 or more: a whole lane
-        const uint32_t c0 = static_cast<uint32_t>(j) * static_cast<uint32_t>(nz) + static_cast<uint32_t>(k);
-        const bool jlast = j == ny - 1;
-        const bool jlast_win = w0 + mt.rows >= ny;           // uniform
-        const bool klast_win = k0 + 4 * mt.kt >= nz;         // uniform
-        const int vlast = nz - 1 - k;                        // element of the last z face (0..3 in one lane)
-        const float dy = ld ? gmem(a.dec[1])[j] : 1.f;
-        float cvy = cv, icy = 1.f;
-        if (NU && ld) {
-            icy = gmem(a.icl[1])[j];
-            if (j + 1 < ny) cvy = cv * gmem(a.ifc[1])[j];
-        }
-        f4v dzr = {1.f, 1.f, 1.f, 1.f};
-        auto lane_tables = [&](int kk, f4v& dz, f4v& cvz, f4v& icz) {
+    const int chunk = lb / nwin, win = lb - chunk * nwin;
+    const int i0 = chunk * mt.units;
+    const int i1 = min(nx, i0 + mt.units);
+    const int seg = win % mt.nseg, jt = win / mt.nseg;
+    // window origin and the rows / lanes it stores
+    const int w0 = jt * (mt.rows - 2 * T);
+    const int jlo = jt == 0 ? 0 : w0 + T;
+    const int jhi = jt == mt.njt - 1 ? ny : w0 + mt.rows - T;
+    const int k0 = 4 * (seg == 0 ? 0 : seg * mt.ko - 1);
+    const int klo = 4 * seg * mt.ko;
+    const int khi = seg == mt.nseg - 1 ? nz : 4 * (seg + 1) * mt.ko;
+    const int j = w0 + row;
+    const int k = k0 + 4 * kl;
+    const bool ld = in_win && j < ny && k < nz;
+    const bool out = ld && j >= jlo && j < jhi && k >= klo && k < khi;
+    const int nv = nz - k;                               // 4 or more: a whole lane
+    const uint32_t c0 = static_cast<uint32_t>(j) * static_cast<uint32_t>(nz) + static_cast<uint32_t>(k);
+    const bool jlast = j == ny - 1;
+    const bool jlast_win = w0 + mt.rows >= ny;           // uniform
+    const bool klast_win = k0 + 4 * mt.kt >= nz;         // uniform
+    const int vlast = nz - 1 - k;                        // element of the last z face (0..3 in one lane)
+    const float dy = ld ? gmem(a.dec[1])[j] : 1.f;
+    float cvy = cv, icy = 1.f;
+    if (NU && ld) {
+        icy = gmem(a.icl[1])[j];
+        if (j + 1 < ny) cvy = cv * gmem(a.ifc[1])[j];
+    }
+    f4v dzr = {1.f, 1.f, 1.f, 1.f};
+    auto lane_tables = [&](int kk, f4v& dz, f4v& cvz, f4v& icz) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (kk + e < nz) {
-                    dz[e] = gmem(a.dec[2])[kk + e];
-                    if (NU) {
-                        icz[e] = gmem(a.icl[2])[kk + e];
-                        if (kk + e + 1 < nz) cvz[e] = cv * gmem(a.ifc[2])[kk + e];
-                    }
-                }
-        };
-        if constexpr (NU) {
-            if (tid < mt.kt) {
-                f4v dz = {1.f, 1.f, 1.f, 1.f}, cz = {cv, cv, cv, cv}, iz = {1.f, 1.f, 1.f, 1.f};
-                lane_tables(k0 + 4 * tid, dz, cz, iz);
-                sK[0][tid] = dz;
-                sK[1][tid] = cz;
-                sK[2][tid] = iz;
-            }
-        } else {
-            f4v none = {};
-            lane_tables(k, dzr, none, none);
-        }
-        // Flag bits that say nothing about walls: the last faces, which keep their
-        // velocity, cells past the row and lanes past the window or grid.
-        uint32_t ends = kOpen;
-        if (ld) {
-            ends = jlast ? kOpenY : 0u;
-            if (vlast < 4) ends |= (FDTD_FLAG_OPEN_Z << (8 * vlast)) | static_cast<uint32_t>(uint64_t(kOpen) << (8 * vlast + 8));
-        }
-        // Sources that touch the window and probes it stores: lane q holds the
-        // plane of source q (kEvery: a y or z plane source, on every plane) and
-        // of probe q, kNowhere if it is elsewhere, so a stage finds what its
-        // plane has with one compare. kNowhere is no plane: a stage's own plane
-        // runs from -(T - 1) to nx + T - 2.
-        int src_i = kNowhere, probe_i = kNowhere;
-        {
-            const int q = tid & (kWave - 1);
-            const int jw = w0 + mt.rows, kw = k0 + 4 * mt.kt;
-            if (q < a.n_src) {
-                const int at = a.src_i[q], sj = a.src_j[q], sk = a.src_k[q];
-                if (a.src_kind[q] == 0) {
-                    if (sj >= w0 && sj < jw && sk >= k0 && sk < kw) src_i = at;
-                } else if (at == 0) {
-                    src_i = sj;
-                } else if (at == 1 ? (sj >= w0 && sj < jw) : (sj >= k0 && sj < kw)) {
-                    src_i = kEvery;
-                }
-            }
-            if (q < a.n_sweep_probe) {
-                const GMEM int32_t* __restrict__ PIJK = gmem(a.probe_ijk);
-                const int pi = PIJK[3 * q], pj = PIJK[3 * q + 1], pk = PIJK[3 * q + 2];
-                if (pj >= jlo && pj < jhi && pk >= klo && pk < khi && pi >= i0 && pi < i1) probe_i = pi;
-            }
-        }
-
-        // A lane past its row's last cell reads on into the next row (or the pad
-        // past the last one): those cells feed nothing that is stored.
-        auto at = [&](int i) { return static_cast<uint32_t>(i) * sx + c0; };
-        auto flags = [&](uint32_t c) -> uint32_t { return *reinterpret_cast<const GMEM u32u*>(at32(FL, c)); };
-
-        const f4v zero = {0.f, 0.f, 0.f, 0.f};
-        Stage st[T];
-#pragma unroll
-        for (int t = 0; t < T; ++t) st[t] = Stage{zero, zero, zero, zero, 0u};
-        const int m0 = max(i0 - T, 0);
-        const int m1 = i1 + T - 1;
-        // plane m0, and p of the one after it
-        f4v p0 = zero, pn = zero;
-        if (ld) {
-            const uint32_t c = at(m0);
-            p0 = ld4(P, c);
-            st[0].vx = ld4(VX, c);
-            st[0].vy = ld4(VY, c);
-            st[0].vz = ld4(VZ, c);
-            st[0].f = flags(c);
-            if (m0 + 1 < nx) pn = ld4(P, c + sx);
-        }
-#pragma unroll
-        for (int t = 0; t < T; ++t) {
-            sP[t][tid] = t ? zero : p0;
-            sX[t][tid] = t ? 0.f : p0.x;
-        }
-        __builtin_amdgcn_s_waitcnt(kWaitLoads);
-        for (int m = m0; m < m1; ++m) {
-            lds_barrier();  // the stages' pressures are posted
-            // ---- next plane's loads
-            f4v qp = zero, qx = zero, qy = zero, qz = zero;
-            uint32_t qf = 0;
-            if (ld && m + 1 < m1 && m + 1 < nx) {
-                const uint32_t c = at(m + 1);
-                if (m + 2 < nx) qp = ld4(P, c + sx);
-                qx = ld4(VX, c);
-                qy = ld4(VY, c);
-                qz = ld4(VZ, c);
-                qf = flags(c);
-            }
-            // ---- y and z faces of every stage's plane
-#pragma unroll
-            for (int t = 0; t < T; ++t) {
-                Stage& S = st[t];
-                const f4v p = sP[t][tid];
-                const f4v pu = sP[t][iu];
-                const float pr = sX[t][ir];
-                f4v vy = S.vy + cvy * (pu - p);
-                const f4v pk = {p.y, p.z, p.w, pr};
-                f4v vz;
-                if constexpr (NU) vz = S.vz + sK[1][again(kl)] * (pk - p);
-                else vz = S.vz + cv * (pk - p);
-                const bool walls = __builtin_amdgcn_ballot_w64(((S.f | ends) & kOpen) != kOpen) != 0;
-                if (walls) {
-                    vy = keep(vy, S.f, 2);
-                    vz = keep(vz, S.f, 3);
-                }
-                if (jlast_win) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) vy[e] = jlast ? S.vy[e] : vy[e];
-                }
-                if (klast_win) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) vz[e] = vlast == e ? S.vz[e] : vz[e];
-                }
-                S.vz = vz;
-                sY[t][tid] = vy;
-                sZ[t][tid] = vz.w;
-            }
-            lds_barrier();
-            // ---- x faces and pressures, stage by stage: what stage t makes of
-            // its plane is p(i + 1) of stage t + 1, and its state of the next round
-            f4v cpn = pn, cx = qx, cy = qy, cz = qz;
-            uint32_t cf = qf;
-            f4v p = sP[0][tid];
-#pragma unroll
-            for (int t = 0; t < T; ++t) {
-                Stage& S = st[t];
-                const int i = m - t;
-                const int ic = min(max(i, 0), nx - 1);
-                const f4v vy = sY[t][tid];
-                const f4v yb = sY[t][id];
-                const float zb = sZ[t][il];
-                const float dx = uni(a.dec[0], ic);
-                f4v vx = S.vx;
-                const bool walls = __builtin_amdgcn_ballot_w64(((S.f | ends) & kOpen) != kOpen) != 0;
-                if (i < nx - 1) {
-                    const float cvx = NU ? cv * uni(a.ifc[0], ic) : cv;
-                    vx = S.vx + cvx * (cpn - p);
-                    if (walls) vx = keep(vx, S.f, 1);
-                }
-                const f4v zl = {zb, S.vz.x, S.vz.y, S.vz.z};
-                const f4v dvx = vx - S.vxp, dvy = vy - yb, dvz = S.vz - zl;
-                f4v pnew;
+        for (int e = 0; e < 4; ++e)
+            if (kk + e < nz) {
+                dz[e] = gmem(a.dec[2])[kk + e];
                 if (NU) {
-                    const float icx = uni(a.icl[0], ic);
-                    pnew = p + cp * ((icx * dvx + icy * dvy) + sK[2][again(kl)] * dvz);
-                } else {
-                    pnew = p + cp * ((dvx + dvy) + dvz);
+                    icz[e] = gmem(a.icl[2])[kk + e];
+                    if (kk + e + 1 < nz) cvz[e] = cv * gmem(a.ifc[2])[kk + e];
                 }
-                if (walls) pnew = keep(pnew, S.f, 0);
-                const f4v dz = NU ? sK[0][again(kl)] : dzr;
-                f4v ps = ((pnew * dx) * dy) * dz;
-                const f4v ox = vx * dx, oy = vy * dy, oz = S.vz * dz;
-                const uint64_t adds = __builtin_amdgcn_ballot_w64(src_i == i || src_i == kEvery);
-                if (adds) {
-                    const CMEM FusedArgs* r = rare(ka);
-                    for (uint32_t sm = static_cast<uint32_t>(adds); sm; sm &= sm - 1) {
-                        const int q = __builtin_ctz(sm);
-                        // the planes or point it acts on, -1: any (its i has matched)
-                        const bool point = r->src_kind[q] == 0;
-                        const int ax = r->src_i[q], aj = r->src_j[q], ak = r->src_k[q];
-                        const int on_j = point || ax == 1 ? aj : -1;
-                        const int on_k = point ? ak : (ax == 2 ? aj : -1);
-                        const bool known = s + t < r->wave_len;
-                        if (!known && tid == 0) atomicOr(r->health, 2u);
-                        const double w = known ? uni(r->wave, q * r->wave_len + s + t) : 0.0;
-                        const uint32_t hit = (known & ((on_j == j) | (on_j < 0))) ? S.f : 0u;
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            const float v = static_cast<float>(static_cast<double>(ps[e]) + w);
-                            const bool on = (((hit >> (8 * e)) & FDTD_FLAG_AIR) != 0) & ((on_k == k + e) | (on_k < 0));
-                            ps[e] = on ? v : ps[e];
-                        }
-                    }
-                }
-                const uint64_t hits = __builtin_amdgcn_ballot_w64(probe_i == i);
-                if (hits) {
-                    const CMEM FusedArgs* r = rare(ka);
-                    for (uint64_t pm = hits; pm; pm &= pm - 1) {
-                        const int q = __builtin_ctzll(pm);
-                        const int pj = uni(r->probe_ijk, 3 * q + 1), pk = uni(r->probe_ijk, 3 * q + 2);
-                        if (s + t >= r->trace_len) {
-                            if (tid == 0) atomicOr(r->health, 2u);
-                        } else if (in_win && j == pj && pk >= k && pk < k + 4) {
-                            const int e = pk - k;
-                            const float v = e == 0 ? ps.x : (e == 1 ? ps.y : (e == 2 ? ps.z : ps.w));
-                            gmem(r->trace)[(s + t) * r->n_probe + q] = v;
-                            if (!isfinite(v)) atomicOr(r->health, 1u);
-                        }
-                    }
-                }
-                if (t == T - 1) {
-                    // The next plane's loads are waited for before the stores are
-                    // issued: later, the wait would be for the stores as well.
-                    __builtin_amdgcn_s_waitcnt(kWaitLoads);
-                    if (out && i >= i0) {
-                        const uint32_t c = at(i);
-                        if (nv >= 4) {
-                            st4<NTS>(Po, c, ps);
-                            st4<NTS>(VXo, c, ox);
-                            st4<NTS>(VYo, c, oy);
-                            st4<NTS>(VZo, c, oz);
-                        } else {
-#pragma unroll
-                            for (int e = 0; e < 3; ++e)
-                                if (e < nv) {
-                                    stx(Po, c + e, ps[e]);
-                                    stx(VXo, c + e, ox[e]);
-                                    stx(VYo, c + e, oy[e]);
-                                    stx(VZo, c + e, oz[e]);
-                                }
-                        }
-                    }
-                }
-                // this stage's next plane: what came in (loads, or the stage before)
-                const uint32_t f = S.f;
-                S = Stage{cx, cy, cz, vx, cf};
-                if (t + 1 < T) p = sP[t + 1][tid];  // read before the next stage's p is posted
-                sP[t][tid] = cpn;
-                sX[t][tid] = cpn.x;
-                cpn = ps;
-                cx = ox;
-                cy = oy;
-                cz = oz;
-                cf = f;
             }
-            pn = qp;
+    };
+    if constexpr (NU) {
+        if (tid < mt.kt) {
+            f4v dz = {1.f, 1.f, 1.f, 1.f}, cz = {cv, cv, cv, cv}, iz = {1.f, 1.f, 1.f, 1.f};
+            lane_tables(k0 + 4 * tid, dz, cz, iz);
+            sK[0][tid] = dz;
+            sK[1][tid] = cz;
+            sK[2][tid] = iz;
+        }
+    } else {
+        f4v none = {};
+        lane_tables(k, dzr, none, none);
+    }
+    // Flag bits that say nothing about walls: the last faces, which keep their
+    // velocity, cells past the row and lanes past the window or grid.
+    uint32_t ends = kOpen;
+    if (ld) {
+        ends = jlast ? kOpenY : 0u;
+        if (vlast < 4) ends |= (FDTD_FLAG_OPEN_Z << (8 * vlast)) | static_cast<uint32_t>(uint64_t(kOpen) << (8 * vlast + 8));
+    }
+    // Sources that touch the window and probes it stores: lane q holds the
+    // plane of source q (kEvery: a y or z plane source, on every plane) and
+    // of probe q, kNowhere if it is elsewhere, so a stage finds what its
+    // plane has with one compare. kNowhere is no plane: a stage's own plane
+    // runs from -(T - 1) to nx + T - 2.
+    int src_i = kNowhere, probe_i = kNowhere;
+    {
+        const int q = tid & (kWave - 1);
+        const int jw = w0 + mt.rows, kw = k0 + 4 * mt.kt;
+        if (q < a.n_src) {
+            const int at = a.src_i[q], sj = a.src_j[q], sk = a.src_k[q];
+            if (a.src_kind[q] == 0) {
+                if (sj >= w0 && sj < jw && sk >= k0 && sk < kw) src_i = at;
+            } else if (at == 0) {
+                src_i = sj;
+            } else if (at == 1 ? (sj >= w0 && sj < jw) : (sj >= k0 && sj < kw)) {
+                src_i = kEvery;
+            }
+        }
+        if (q < a.n_sweep_probe) {
+            const GMEM int32_t* __restrict__ PIJK = gmem(a.probe_ijk);
+            const int pi = PIJK[3 * q], pj = PIJK[3 * q + 1], pk = PIJK[3 * q + 2];
+            if (pj >= jlo && pj < jhi && pk >= klo && pk < khi && pi >= i0 && pi < i1) probe_i = pi;
         }
     }
+
+    // A lane past its row's last cell reads on into the next row (or the pad
+    // past the last one): those cells feed nothing that is stored.
+    auto at = [&](int i) { return static_cast<uint32_t>(i) * sx + c0; };
+    auto flags = [&](uint32_t c) -> uint32_t { return *reinterpret_cast<const GMEM u32u*>(at32(FL, c)); };
+
+    const f4v zero = {0.f, 0.f, 0.f, 0.f};
+    Stage st[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) st[t] = Stage{zero, zero, zero, zero, 0u};
+    const int m0 = max(i0 - T, 0);
+    const int m1 = i1 + T - 1;
+    // plane m0, and p of the one after it
+    f4v p0 = zero, pn = zero;
+    if (ld) {
+        const uint32_t c = at(m0);
+        p0 = ld4(P, c);
+        st[0].vx = ld4(VX, c);
+        st[0].vy = ld4(VY, c);
+        st[0].vz = ld4(VZ, c);
+        st[0].f = flags(c);
+        if (m0 + 1 < nx) pn = ld4(P, c + sx);
+    }
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        sP[t][tid] = t ? zero : p0;
+        sX[t][tid] = t ? 0.f : p0.x;
+    }
+    __builtin_amdgcn_s_waitcnt(kWaitLoads);
+    for (int m = m0; m < m1; ++m) {
+        lds_barrier();  // the stages' pressures are posted
+        // ---- next plane's loads
+        f4v qp = zero, qx = zero, qy = zero, qz = zero;
+        uint32_t qf = 0;
+        if (ld && m + 1 < m1 && m + 1 < nx) {
+            const uint32_t c = at(m + 1);
+            if (m + 2 < nx) qp = ld4(P, c + sx);
+            qx = ld4(VX, c);
+            qy = ld4(VY, c);
+            qz = ld4(VZ, c);
+            qf = flags(c);
+        }
+        // ---- y and z faces of every stage's plane
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            Stage& S = st[t];
+            const f4v p = sP[t][tid];
+            const f4v pu = sP[t][iu];
+            const float pr = sX[t][ir];
+            f4v vy = S.vy + cvy * (pu - p);
+            const f4v pk = {p.y, p.z, p.w, pr};
+            f4v vz;
+            if constexpr (NU) vz = S.vz + sK[1][again(kl)] * (pk - p);
+            else vz = S.vz + cv * (pk - p);
+            const bool walls = __builtin_amdgcn_ballot_w64(((S.f | ends) & kOpen) != kOpen) != 0;
+            if (walls) {
+                vy = keep(vy, S.f, 2);
+                vz = keep(vz, S.f, 3);
+            }
+            if (jlast_win) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) vy[e] = jlast ? S.vy[e] : vy[e];
+            }
+            if (klast_win) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) vz[e] = vlast == e ? S.vz[e] : vz[e];
+            }
+            S.vz = vz;
+            sY[t][tid] = vy;
+            sZ[t][tid] = vz.w;
+        }
+        lds_barrier();
+        // ---- x faces and pressures, stage by stage: what stage t makes of
+        // its plane is p(i + 1) of stage t + 1, and its state of the next round
+        f4v cpn = pn, cx = qx, cy = qy, cz = qz;
+        uint32_t cf = qf;
+        f4v p = sP[0][tid];
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            Stage& S = st[t];
+            const int i = m - t;
+            const int ic = min(max(i, 0), nx - 1);
+            const f4v vy = sY[t][tid];
+            const f4v yb = sY[t][id];
+            const float zb = sZ[t][il];
+            const float dx = uni(a.dec[0], ic);
+            f4v vx = S.vx;
+            const bool walls = __builtin_amdgcn_ballot_w64(((S.f | ends) & kOpen) != kOpen) != 0;
+            if (i < nx - 1) {
+                const float cvx = NU ? cv * uni(a.ifc[0], ic) : cv;
+                vx = S.vx + cvx * (cpn - p);
+                if (walls) vx = keep(vx, S.f, 1);
+            }
+            const f4v zl = {zb, S.vz.x, S.vz.y, S.vz.z};
+            const f4v dvx = vx - S.vxp, dvy = vy - yb, dvz = S.vz - zl;
+            f4v pnew;
+            if (NU) {
+                const float icx = uni(a.icl[0], ic);
+                pnew = p + cp * ((icx * dvx + icy * dvy) + sK[2][again(kl)] * dvz);
+            } else {
+                pnew = p + cp * ((dvx + dvy) + dvz);
+            }
+            if (walls) pnew = keep(pnew, S.f, 0);
+            const f4v dz = NU ? sK[0][again(kl)] : dzr;
+            f4v ps = ((pnew * dx) * dy) * dz;
+            const f4v ox = vx * dx, oy = vy * dy, oz = S.vz * dz;
+            const uint64_t adds = __builtin_amdgcn_ballot_w64(src_i == i || src_i == kEvery);
+            if (adds) {
+                const CMEM FusedArgs* r = rare(ka);
+                for (uint32_t sm = static_cast<uint32_t>(adds); sm; sm &= sm - 1) {
+                    const int q = __builtin_ctz(sm);
+                    // the planes or point it acts on, -1: any (its i has matched)
+                    const bool point = r->src_kind[q] == 0;
+                    const int ax = r->src_i[q], aj = r->src_j[q], ak = r->src_k[q];
+                    const int on_j = point || ax == 1 ? aj : -1;
+                    const int on_k = point ? ak : (ax == 2 ? aj : -1);
+                    const bool known = s + t < r->wave_len;
+                    if (!known && tid == 0) atomicOr(r->health, 2u);
+                    const double w = known ? uni(r->wave, q * r->wave_len + s + t) : 0.0;
+                    const uint32_t hit = (known & ((on_j == j) | (on_j < 0))) ? S.f : 0u;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float v = static_cast<float>(static_cast<double>(ps[e]) + w);
+                        const bool on = (((hit >> (8 * e)) & FDTD_FLAG_AIR) != 0) & ((on_k == k + e) | (on_k < 0));
+                        ps[e] = on ? v : ps[e];
+                    }
+                }
+            }
+            const uint64_t hits = __builtin_amdgcn_ballot_w64(probe_i == i);
+            if (hits) {
+                const CMEM FusedArgs* r = rare(ka);
+                for (uint64_t pm = hits; pm; pm &= pm - 1) {
+                    const int q = __builtin_ctzll(pm);
+                    const int pj = uni(r->probe_ijk, 3 * q + 1), pk = uni(r->probe_ijk, 3 * q + 2);
+                    if (s + t >= r->trace_len) {
+                        if (tid == 0) atomicOr(r->health, 2u);
+                    } else if (in_win && j == pj && pk >= k && pk < k + 4) {
+                        const int e = pk - k;
+                        const float v = e == 0 ? ps.x : (e == 1 ? ps.y : (e == 2 ? ps.z : ps.w));
+                        gmem(r->trace)[(s + t) * r->n_probe + q] = v;
+                        if (!isfinite(v)) atomicOr(r->health, 1u);
+                    }
+                }
+            }
+            if (t == T - 1) {
+                // The next plane's loads are waited for before the stores are
+                // issued: later, the wait would be for the stores as well.
+                __builtin_amdgcn_s_waitcnt(kWaitLoads);
+                if (out && i >= i0) {
+                    const uint32_t c = at(i);
+                    if (nv >= 4) {
+                        st4<NTS>(Po, c, ps);
+                        st4<NTS>(VXo, c, ox);
+                        st4<NTS>(VYo, c, oy);
+                        st4<NTS>(VZo, c, oz);
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 3; ++e)
+                            if (e < nv) {
+                                stx(Po, c + e, ps[e]);
+                                stx(VXo, c + e, ox[e]);
+                                stx(VYo, c + e, oy[e]);
+                                stx(VZo, c + e, oz[e]);
+                            }
+                    }
+                }
+            }
+            // this stage's next plane: what came in (loads, or the stage before)
+            const uint32_t f = S.f;
+            S = Stage{cx, cy, cz, vx, cf};
+            if (t + 1 < T) p = sP[t + 1][tid];  // read before the next stage's p is posted
+            sP[t][tid] = cpn;
+            sX[t][tid] = cpn.x;
+            cpn = ps;
+            cx = ox;
+            cy = oy;
+            cz = oz;
+            cf = f;
+        }
+        pn = qp;
+    }
+}
+
+template <bool NU, int NT, bool NTS>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_multi_step(const FusedArgs a,
+                                                                                             const PassTile mt) {
+    // XCD-aware order: hardware block b runs on XCD b mod 8, which takes a
+    // contiguous range of the windows
+    const int lb = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    if (lb < mt.nwg) pass_workgroup<NU, NT, NTS>(kernargs(), mt, uni(a.step_ptr, 0) + a.koff, lb);
+}
+
+// A pass of every solve in a batch table: steps koff .. koff + kPassSteps - 1 of a
+// chunk of `chunk` steps that starts at each solve's counter. A solve with fewer
+// steps left, to its limit or the chunk's end, skips the pass (k_batch_step takes
+// the rest). Workgroups are dealt out through the prefix sums `offsets`; the
+// number of solves and the sums are read from device memory, as k_batch_step
+// reads its own. Each solve's windows are picked for its share of the chip. 24
+// enclosures of 64-192 cells a side, 1000-3000 steps, served in 709 ms with single
+// steps and in 404 with passes (430 with workgroups of 256, 405 with 1024).
+template <bool NTS>
+__global__ __launch_bounds__(kBatchPassThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_batch_pass(
+    const FusedArgs* __restrict__ table, const PassTile* __restrict__ tiles, const int* __restrict__ offsets,
+    const int* __restrict__ n_ptr, int koff, int chunk) {
+    const int n = uni(n_ptr, 0);
+    const int total = uni(offsets, n);
+    const int bpx = (total + 7) / 8;
+    const int xb = blockIdx.x >> 3;
+    if (xb >= bpx) return;
+    const int g = (blockIdx.x & 7) * bpx + xb;
+    if (g >= total) return;
+    int lo = 0, hi = n;  // offsets[lo] <= g < offsets[hi]
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (uni(offsets, mid) <= g) lo = mid; else hi = mid;
+    }
+    const CMEM FusedArgs* ka = (const CMEM FusedArgs*)table + lo;
+    const int64_t s0 = uni(ka->step_ptr, 0);
+    if (s0 + koff + kPassSteps > min(ka->step_limit, s0 + chunk)) return;
+    const PassTile mt = ((const CMEM PassTile*)tiles)[lo];
+    pass_workgroup<false, kBatchPassThreads, NTS>(ka, mt, s0 + koff, g - uni(offsets, lo));
 }
 
 // ---- ADE patch ------------------------------------------------------------------
@@ -546,13 +582,17 @@ static bool pass_windows(int nx, int ny, int nz, int nt, int nseg, PassTile& m) 
 // traffic at 5.2 TB/s times 1.2, the larger of the two and 0.3 of the smaller.
 // Fitted to 3337 measured (workgroup, segments, chunks) triples of 14 grids from
 // 40^3 to 400^3 (rms 16%): what it picks runs within 12% of the best triple.
-bool pick_pass_tile(int nx, int ny, int nz, PassTile& best) {
+// only_nt: that workgroup size alone (0: any). share: the part of the chip the
+// pass has (a solve in a batch).
+bool pick_pass_tile(int nx, int ny, int nz, int only_nt, double share, PassTile& best) {
     const int64_t cells = static_cast<int64_t>(nx) * ny * nz;
     if (cells >= kMaxCells32) return false;
     double low = 0.0;
     bool found = false;
     for (int nt : {1024, 512, 256}) {
-        const int per_cu = 1024 / nt, slots = kCUs * per_cu;
+        if (only_nt && nt != only_nt) continue;
+        const int cus = std::max(1, static_cast<int>(kCUs * share));
+        const int per_cu = 1024 / nt, slots = cus * per_cu;
         for (int nseg = 1; nseg <= 64; ++nseg) {
             PassTile m{};
             if (!pass_windows(nx, ny, nz, nt, nseg, m)) continue;
@@ -563,7 +603,7 @@ bool pick_pass_tile(int nx, int ny, int nz, PassTile& best) {
                 const int64_t n = static_cast<int64_t>(nwin) * ((nx + units - 1) / units);
                 const double planes = units + 2 * kPassSteps - 1;
                 auto plane_us = [&](int64_t wgs) {
-                    return 1.23 + 0.12 * (static_cast<double>((wgs + kCUs - 1) / kCUs) * nt / kWave);
+                    return 1.23 + 0.12 * (static_cast<double>((wgs + cus - 1) / cus) * nt / kWave);
                 };
                 const int64_t full = n / slots, rest = n % slots;
                 const double march = planes * (full * plane_us(slots) + (rest ? plane_us(rest) : 0.0));
@@ -638,6 +678,19 @@ hipError_t launch_pass(const FusedArgs& a, bool nu, const PassTile& m, hipStream
         case 256: return nu ? launch_pass_t<true, 256>(a, m, st) : launch_pass_t<false, 256>(a, m, st);
         default: return hipErrorInvalidValue;
     }
+}
+
+// Passes of a batch (workgroups up to cap_wgs, the grid covers the capacity).
+hipError_t launch_batch_pass(const FusedArgs* table, const PassTile* tiles, const int* offsets, const int* n_ptr,
+                             int cap_wgs, bool nts, int koff, int chunk, hipStream_t st) {
+    const int blocks = std::max(8, (cap_wgs + 7) & ~7);
+    if (nts)
+        hipLaunchKernelGGL(k_batch_pass<true>, dim3(blocks), dim3(kBatchPassThreads), 0, st, table, tiles, offsets,
+                           n_ptr, koff, chunk);
+    else
+        hipLaunchKernelGGL(k_batch_pass<false>, dim3(blocks), dim3(kBatchPassThreads), 0, st, table, tiles, offsets,
+                           n_ptr, koff, chunk);
+    return hipGetLastError();
 }
 
 }  // namespace fdtd_amd

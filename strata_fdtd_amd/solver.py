@@ -291,7 +291,7 @@ class FDTDSolver:
         _native.call("fdtd_ctx_set_counters", ctx, _native.ptr(self._step_dev), _native.ptr(self._health))
         tiling = self._tiling or pick_tiling(self.shape, not self._grid.is_uniform, False)
         _native.call("fdtd_ctx_set_tiling", ctx, *tiling)
-        _native.call("fdtd_ctx_set_multi_step", ctx, int(self._tiling is None))
+        _native.call("fdtd_ctx_set_multi_step", ctx, 1 if self._tiling is None else 2)
 
     def set_tiling(self, rows: int, planes: int, stack: int = 1) -> None:
         """Launch shape of the fused kernel: rows per wave, planes per wave and
@@ -299,7 +299,7 @@ class FDTDSolver:
         shape is given takes every step with that kernel; by default step_n
         takes three steps per pass where the solve allows it."""
         self._tiling = normalize_tiling((rows, planes, stack))
-        _native.call("fdtd_ctx_set_multi_step", self._ctx, 0)
+        _native.call("fdtd_ctx_set_multi_step", self._ctx, 2)
         _native.call("fdtd_ctx_set_tiling", self._ctx, *self._tiling)
 
     @property
