@@ -361,6 +361,25 @@ int fdtd_design_adjoint(float* const* lam, const uint8_t* flags, const float* co
                         int64_t n_hi, const float* hist_p, const float* hist_div, int64_t hist0, int64_t hist_steps,
                         float* acc, float* face_e, float* pb_box, int planes, void* stream);
 
+/* The same two calls with `scratch`: device float32, 16-byte aligned, of
+ * fdtd_design_pass_floats entries (adjoint 0 for the forward alone), in which
+ * three steps are taken per pass over the fields where the grid has such passes
+ * (the rest, and everything if scratch is NULL, one by one). The results are the
+ * same bit for bit. The fields and flags must be readable 4 cells past their end. */
+int64_t fdtd_design_pass_floats(const int32_t* box_lo, const int32_t* box_hi, int adjoint);
+int fdtd_design_forward_passes(float* const* fields, const uint8_t* flags, const float* const* dec, int nx, int ny,
+                               int nz, float cv0, float cp0, const int32_t* box_lo, const int32_t* box_hi,
+                               const float* rk, const int32_t* src_ijk, const double* wave, int n_probe,
+                               const int32_t* probe_ijk, float* trace, int64_t steps_len, int64_t step0, int n_steps,
+                               float* hist_p, float* hist_div, int64_t hist0, int64_t hist_steps, int planes,
+                               float* scratch, void* stream);
+int fdtd_design_adjoint_passes(float* const* lam, const uint8_t* flags, const float* const* dec, int nx, int ny,
+                               int nz, float cv0, float cp0, const int32_t* box_lo, const int32_t* box_hi,
+                               const float* rk, int n_probe, const int32_t* probe_ijk, const float* g,
+                               int64_t steps_len, int64_t n_lo, int64_t n_hi, const float* hist_p,
+                               const float* hist_div, int64_t hist0, int64_t hist_steps, float* acc, float* face_e,
+                               float* pb_box, int planes, float* scratch, void* stream);
+
 /* ---- per-phase entry points (one kernel per reference function) --------- */
 /* All in place, on `stream`, float32, uniform unless noted. */
 /* Replaces fdtd::update_velocity (fdtd_step.cpp:15-82). */

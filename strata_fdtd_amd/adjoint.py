@@ -82,7 +82,10 @@ class _Device:
             self.cv0, self.cp0 = float(np.float32(self.cv0)), float(np.float32(self.cp0))
         air = np.ones(pb.shape, np.uint8) if pb.geometry is None else pb.geometry.astype(np.uint8)
         air_d = torch.from_numpy(air).to(device)
-        self.flags = torch.empty(pb.shape, dtype=torch.uint8, device=device)
+        # flags and fields are readable one 4-cell access past their end
+        # (multi-step passes read whole 4-cell lanes)
+        n = int(np.prod(pb.shape))
+        self.flags = torch.zeros(n + 4, dtype=torch.uint8, device=device)[:n].view(pb.shape)
         _native.call("fdtd_build_flags", _ptr(air_d), None, _ptr(self.flags), nx, ny, nz,
                      torch.cuda.current_stream(device).cuda_stream)
         self.air = air_d
@@ -125,7 +128,7 @@ class _Device:
         90-92 ms every time."""
         import torch
         n = int(np.prod(self.pb.shape))
-        slab = torch.zeros(8 * pairs * n, dtype=self.dtype, device=self.dev)
+        slab = torch.zeros(8 * pairs * n + 4, dtype=self.dtype, device=self.dev)
         views = [slab[q * n:(q + 1) * n].view(self.pb.shape) for q in range(8 * pairs)]
         out = [[views[8 * m:8 * m + 4], views[8 * m + 4:8 * m + 8]] for m in range(pairs)]
         return out[0] if pairs == 1 else out
@@ -200,6 +203,20 @@ class _Fast:
         lo, hi = np.array(pb.box_lo), np.array(pb.box_hi)
         self.ecells = int(np.prod(hi - lo + 2))
         self.bcells = int(np.prod(hi - lo))
+        self._scratch = None
+
+    def _pass_scratch(self, adjoint: bool):
+        """Device scratch of the multi-step passes (face coefficients; for the
+        adjoint also the steps' velocities and pb on the box), kept for this
+        solve; None (single steps) where there is no room for it."""
+        import torch
+        n = _native.load().fdtd_design_pass_floats(self.dv.lo.ctypes.data, self.dv.hi.ctypes.data, int(adjoint))
+        if n > 0 and (self._scratch is None or self._scratch.numel() < n):
+            try:
+                self._scratch = torch.empty(n, dtype=torch.float32, device=self.dv.dev)
+            except torch.cuda.OutOfMemoryError:
+                return None
+        return self._scratch if n > 0 else None
 
     @staticmethod
     def _sets(sets):
@@ -229,10 +246,10 @@ class _Fast:
         hp, hd = hist if hist is not None else (None, None)
         hist_steps = (hp.numel() // self.ecells) if hp is not None else 0
         rows = trace.shape[0] if self.dv.n_probe > 0 else self.wave_dev.numel()
-        _native.call("fdtd_design_forward", self._sets(sets), *self._common(rk), self.src,
+        _native.call("fdtd_design_forward_passes", self._sets(sets), *self._common(rk), self.src,
                      _ptr(self.wave_dev), self.dv.n_probe, _ptr(self.probe_ijk), _ptr(trace),
                      min(rows, self.wave_dev.numel()), step0, n_steps, _ptr(hp), _ptr(hd), hist0, hist_steps,
-                     self.PLANES, self.dv.stream)
+                     self.PLANES, _ptr(self._pass_scratch(False)), self.dv.stream)
 
     def adjoint(self, lam, rk, g, n_lo, n_hi, hist, hist0, acc):
         """acc: float32 [box][4], Kahan (sum, compensation) of dL/dr, then dL/dkappa."""
@@ -242,10 +259,10 @@ class _Fast:
             n = _native.load().fdtd_design_face_count(self.dv.lo.ctypes.data, self.dv.hi.ctypes.data)
             self._faces = torch.empty(n, dtype=torch.float32, device=self.dv.dev)
             self._pb_box = torch.empty(2 * self.bcells, dtype=torch.float32, device=self.dv.dev)
-        _native.call("fdtd_design_adjoint", self._sets(lam), *self._common(rk), self.dv.n_probe,
+        _native.call("fdtd_design_adjoint_passes", self._sets(lam), *self._common(rk), self.dv.n_probe,
                      _ptr(self.probe_ijk), _ptr(g), g.shape[0], n_lo, n_hi, _ptr(hp), _ptr(hd), hist0,
                      hp.numel() // self.ecells, _ptr(acc), _ptr(self._faces), _ptr(self._pb_box), self.ADJ_PLANES,
-                     self.dv.stream)
+                     _ptr(self._pass_scratch(True)), self.dv.stream)
 
 
 def history_bytes(pb: DesignProblem, steps: int | None = None) -> int:

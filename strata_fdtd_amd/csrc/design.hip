@@ -20,16 +20,10 @@
 
 #include <algorithm>
 
-#include "fdtd_common.hpp"
+#include "design_common.hpp"
 
 namespace fdtd_amd {
 
-constexpr int kDesignMaxProbes = 8;
-
-// (r, kappa) of a voxel and the four Kahan words of its gradients, loaded
-// and stored whole
-typedef float f2v __attribute__((ext_vector_type(2)));
-typedef float f4v __attribute__((ext_vector_type(4)));
 // strips: rows per strip of the forward launch (plain and box strips), rows
 // per strip of the adjoint's plain strips and of its box strips (the box
 // sweep's register budget), planes per strip of the box launches at most.
@@ -40,59 +34,6 @@ constexpr int kDesignRows = 2;
 constexpr int kDesignAdjRows = 4;
 constexpr int kDesignAdjBoxRows = 2;
 constexpr int kDesignBoxPlanes = 4;
-
-struct DesignArgs {
-    // fields: ping-pong sets {p, vx, vy, vz}; step s reads set s & 1
-    float* f[2][4];
-    const uint8_t* flags;
-    const float* dec[3];
-    int nx, ny, nz;
-    float cv0, cp0;
-    // design box [lo, hi) with r = rho/rho0 and kappa = K/K0 (float32)
-    int lo[3], hi[3];
-    const f2v* rk;                   // device [box][2]: (r, kappa) per voxel, or NULL (air)
-    // source (one point source; -1 none) and probes
-    int src_i, src_j, src_k;
-    const double* wave;              // device [steps]
-    int n_probe;
-    const int32_t* probe;            // device [n_probe][3] (i, j, k)
-    float* trace;                    // device [steps][n_probe] (forward)
-    const float* g;                  // device [steps][n_probe] (adjoint: dL/dy)
-    // history: p on [lo-1, hi+1), div on [lo, hi); slot of step s = s - hist0
-    float* hist_p;
-    float* hist_div;
-    int64_t hist0;
-    int64_t hist_steps;
-    // gradient accumulators on the box: Kahan (sum, compensation) of dL/dr,
-    // then of dL/dkappa, per voxel
-    f4v* acc;
-    // pb of every box voxel (the adjoint sweep of step n writes pbb[n & 1]),
-    // read by the gradient pass of step n after the next step's sweep
-    float* pbb[2];
-    // gradient factor -cv / (r_lo + r_hi) of every face of the box, formed once
-    // per adjoint call: x faces of cells [lo0, hi0] x [lo1, hi1) x [lo2, hi2)
-    // (the face below each cell), likewise y and z; see face_offsets()
-    float* face_e;
-    // tiling; the strips that meet the design box form the sub-grid
-    // [b_seg0, b_seg1) x [b_sj0, b_sj1) x [b_si0, b_si1)
-    int planes, nseg, nstrip_j, nwaves, blocks_per_xcd;
-    int b_seg0, b_seg1, b_sj0, b_sj1, b_si0, b_si1, b_blocks_per_xcd;
-    int rows;  // rows per plain strip; the box strips split them
-    // the box launch: planes [b_i0, b_i1) in nb_i strips of box_planes planes
-    int box_planes, b_i0, b_i1, nb_i;
-};
-
-__device__ __forceinline__ int64_t ebox_cells(const DesignArgs& a) {
-    return static_cast<int64_t>(a.hi[0] - a.lo[0] + 2) * (a.hi[1] - a.lo[1] + 2) * (a.hi[2] - a.lo[2] + 2);
-}
-
-__device__ __forceinline__ int64_t dbox_cells(const DesignArgs& a) {
-    return static_cast<int64_t>(a.hi[0] - a.lo[0]) * (a.hi[1] - a.lo[1]) * (a.hi[2] - a.lo[2]);
-}
-
-__device__ __forceinline__ float cvf(const DesignArgs& a, float r_lo, float r_hi) {
-    return a.cv0 / ((r_lo + r_hi) * 0.5f);
-}
 
 // Probes in [i0-1, i1] x [j0-1, j1] x [k0-1, k1] (halo = 1), or in the strip
 // itself [i0, i1) x [j0, j1) x [k0, k1) (halo = 0), as a bit mask.
@@ -108,19 +49,9 @@ __device__ __forceinline__ uint32_t strip_probes(const DesignArgs& a, int i0, in
     return m;
 }
 
-template <typename T>
-__device__ __forceinline__ GMEM T* gm(T* p) { return gmem(p); }
-template <typename T>
-__device__ __forceinline__ const GMEM T* gm(const T* p) { return gmem(p); }
-
 __device__ __forceinline__ float sdown(float v) { return __shfl_down(v, 1, kWave); }
 __device__ __forceinline__ float sup(float v) { return __shfl_up(v, 1, kWave); }
 
-__device__ __forceinline__ uint32_t cix(int i, int j, int k, int ny, int nz) { return lidx<uint32_t>(i, j, k, ny, nz); }
-template <typename T>
-__device__ __forceinline__ T ldo(const GMEM T* base, uint32_t idx) { return ldx(base, idx); }
-template <typename T>
-__device__ __forceinline__ void sto(GMEM T* base, uint32_t idx, T v) { stx(base, idx, v); }
 // A step's field outputs: non-temporal stores for grids beyond the Infinity
 // Cache (kCacheResidentCells), ordinary stores below it so that the next step
 // finds them on chip.
@@ -149,25 +80,6 @@ __device__ __forceinline__ Ax dax(int x, int lo, int n) {
 __device__ __forceinline__ Ax eax(int x, int lo, int n) {
     const int b = x - lo + 1;
     return {min(max(b, 0), n + 1), static_cast<unsigned>(b) < static_cast<unsigned>(n + 2)};
-}
-
-// An absent (r, kappa) array means (1, 1) everywhere: its loads read this.
-__device__ __align__(8) float kDesignOne[2] = {1.0f, 1.0f};
-
-struct BoxTab {
-    const GMEM f2v* p;
-    uint32_t mask;  // offsets are masked to 0 when the array is absent
-    bool has;
-};
-__device__ __forceinline__ BoxTab box_tab(const f2v* p) {
-    if (p) return {gm(p), 0xffffffffu, true};
-    return {gm(reinterpret_cast<const f2v*>(kDesignOne)), 0u, false};
-}
-// (r, kappa) of a voxel, (1, 1) outside the box
-__device__ __forceinline__ f2v box_val(const BoxTab& t, int off, bool in) {
-    const f2v v = ldo(t.p, static_cast<uint32_t>(off) & t.mask);
-    const f2v one = {1.0f, 1.0f};
-    return (in && t.has) ? v : one;
 }
 
 // ---------------------------------------------------------------- forward
@@ -995,10 +907,6 @@ __device__ __forceinline__ void design_adjoint_box_strip(const DesignArgs& a, in
 // Layout of face_e: x faces (bx+1) by bz, then y faces bx (by+1) bz, then z
 // faces bx by (bz+1); the face of axis d below box cell (bi, bj, bk) (between
 // it and its -d neighbour) has that cell's index in the axis' array.
-__host__ __device__ inline int64_t face_count(int bx, int by, int bz, int d) {
-    return static_cast<int64_t>(bx + (d == 0)) * (by + (d == 1)) * (bz + (d == 2));
-}
-
 // The gradient factor of every face of the box: the same expression of the
 // same two r values as in the per-cell adjoint kernel.
 __global__ __launch_bounds__(256) void k_design_faces(const DesignArgs a) {
@@ -1144,6 +1052,40 @@ static int design_grid(DesignArgs& a, int planes, int rows, int box_rows) {
     return 8 * (a.blocks_per_xcd + a.b_blocks_per_xcd);
 }
 
+// Multi-step passes (design_pass.hip).
+bool design_pass_tile(const DesignArgs& a, PassTile& m);
+hipError_t launch_design_coefs(const DesignArgs& a, float* coef, hipStream_t st);
+hipError_t launch_design_forward_pass(const DesignArgs& a, const PassTile& m, int64_t s, bool nts, hipStream_t st);
+hipError_t launch_design_adjoint_pass(const DesignArgs& a, const PassTile& m, int64_t n, bool nts, hipStream_t st);
+
+// Offsets of the passes' scratch (coefficients, velocities, pb), and its size, in
+// floats; each part starts on 16 bytes.
+static int64_t pass_layout(const DesignArgs& a, int64_t off[3]) {
+    auto round4 = [](int64_t n) { return (n + 3) & ~int64_t(3); };
+    const int64_t box = static_cast<int64_t>(a.hi[0] - a.lo[0]) * (a.hi[1] - a.lo[1]) * (a.hi[2] - a.lo[2]);
+    off[0] = 0;
+    off[1] = round4(4 * coef_cells(a));
+    off[2] = off[1] + round4(3 * (kPassSteps - 1) * wall_cells(a));
+    return off[2] + round4(kPassSteps * box);
+}
+
+// The split of the grid and the coefficients for a call's passes; false where the
+// grid has no passes (the call then steps one by one). 32-bit offsets: four
+// coefficients and three velocities per cell of boxes below 2^26 cells.
+static bool pass_ready(DesignArgs& a, float* scratch, PassTile& tile, hipStream_t st) {
+    if (coef_cells(a) >= (1ll << 26) || wall_cells(a) >= (1ll << 26) || !design_pass_tile(a, tile)) return false;
+    int64_t off[3];
+    pass_layout(a, off);
+    a.pass_w = scratch + off[1];
+    a.pass_pb = scratch + off[2];
+    a.coef = nullptr;
+    if (a.rk) {
+        if (launch_design_coefs(a, scratch, st) != hipSuccess) return false;
+        a.coef = scratch;
+    }
+    return true;
+}
+
 }  // namespace fdtd_amd
 
 using namespace fdtd_amd;
@@ -1213,11 +1155,35 @@ int64_t fdtd_design_history_bytes(const int32_t* box_lo, const int32_t* box_hi, 
     return 4 * (e + b) * steps;
 }
 
+int64_t fdtd_design_pass_floats(const int32_t* box_lo, const int32_t* box_hi, int adjoint) {
+    if (!box_lo || !box_hi) return -2;
+    DesignArgs a{};
+    for (int d = 0; d < 3; ++d) {
+        a.lo[d] = box_lo[d];
+        a.hi[d] = box_hi[d];
+        if (a.lo[d] < 1 || a.hi[d] <= a.lo[d]) return -3;
+    }
+    int64_t off[3];
+    const int64_t all = pass_layout(a, off);
+    return adjoint ? all : off[1];
+}
+
 int fdtd_design_forward(float* const* fields, const uint8_t* flags, const float* const* dec, int nx, int ny, int nz,
                         float cv0, float cp0, const int32_t* box_lo, const int32_t* box_hi, const float* rk,
                         const int32_t* src_ijk, const double* wave, int n_probe, const int32_t* probe_ijk,
                         float* trace, int64_t steps_len, int64_t step0, int n_steps, float* hist_p, float* hist_div,
                         int64_t hist0, int64_t hist_steps, int planes, void* stream) {
+    return fdtd_design_forward_passes(fields, flags, dec, nx, ny, nz, cv0, cp0, box_lo, box_hi, rk, src_ijk, wave,
+                                      n_probe, probe_ijk, trace, steps_len, step0, n_steps, hist_p, hist_div, hist0,
+                                      hist_steps, planes, nullptr, stream);
+}
+
+int fdtd_design_forward_passes(float* const* fields, const uint8_t* flags, const float* const* dec, int nx, int ny,
+                               int nz, float cv0, float cp0, const int32_t* box_lo, const int32_t* box_hi,
+                               const float* rk, const int32_t* src_ijk, const double* wave, int n_probe,
+                               const int32_t* probe_ijk, float* trace, int64_t steps_len, int64_t step0, int n_steps,
+                               float* hist_p, float* hist_div, int64_t hist0, int64_t hist_steps, int planes,
+                               float* scratch, void* stream) {
     DesignArgs a;
     if (int rc = fill_design(a, fields, flags, dec, nx, ny, nz, cv0, cp0, box_lo, box_hi, rk, src_ijk, wave,
                              n_probe, probe_ijk))
@@ -1234,7 +1200,13 @@ int fdtd_design_forward(float* const* fields, const uint8_t* flags, const float*
     const int blocks = design_grid(a, planes, kDesignRows, kDesignRows);
     hipStream_t st = static_cast<hipStream_t>(stream);
     const bool nts = static_cast<int64_t>(nx) * ny * nz > kCacheResidentCells;
-    for (int m = 0; m < n_steps; ++m) {
+    int m = 0;
+    PassTile tile{};
+    if (scratch && n_steps >= kPassSteps && pass_ready(a, scratch, tile, st)) {
+        for (; n_steps - m >= kPassSteps; m += kPassSteps)
+            if (launch_design_forward_pass(a, tile, step0 + m, nts, st) != hipSuccess) return -5;
+    }
+    for (; m < n_steps; ++m) {
         if (nts)
             hipLaunchKernelGGL((k_design_forward<kDesignRows, true>), dim3(blocks), dim3(kBlock), 0, st, a, step0 + m);
         else
@@ -1250,6 +1222,17 @@ int fdtd_design_adjoint(float* const* lam, const uint8_t* flags, const float* co
                         int n_probe, const int32_t* probe_ijk, const float* g, int64_t steps_len, int64_t n_lo,
                         int64_t n_hi, const float* hist_p, const float* hist_div, int64_t hist0, int64_t hist_steps,
                         float* acc, float* face_e, float* pb_box, int planes, void* stream) {
+    return fdtd_design_adjoint_passes(lam, flags, dec, nx, ny, nz, cv0, cp0, box_lo, box_hi, rk, n_probe, probe_ijk, g,
+                                      steps_len, n_lo, n_hi, hist_p, hist_div, hist0, hist_steps, acc, face_e, pb_box,
+                                      planes, nullptr, stream);
+}
+
+int fdtd_design_adjoint_passes(float* const* lam, const uint8_t* flags, const float* const* dec, int nx, int ny,
+                               int nz, float cv0, float cp0, const int32_t* box_lo, const int32_t* box_hi,
+                               const float* rk, int n_probe, const int32_t* probe_ijk, const float* g,
+                               int64_t steps_len, int64_t n_lo, int64_t n_hi, const float* hist_p,
+                               const float* hist_div, int64_t hist0, int64_t hist_steps, float* acc, float* face_e,
+                               float* pb_box, int planes, float* scratch, void* stream) {
     DesignArgs a;
     if (int rc = fill_design(a, lam, flags, dec, nx, ny, nz, cv0, cp0, box_lo, box_hi, rk, nullptr, nullptr, n_probe,
                              probe_ijk))
@@ -1277,6 +1260,11 @@ int fdtd_design_adjoint(float* const* lam, const uint8_t* flags, const float* co
         const int64_t faces = face_count(fbx, fby, fbz, 0) + face_count(fbx, fby, fbz, 1) + face_count(fbx, fby, fbz, 2);
         hipLaunchKernelGGL(k_design_faces, dim3(static_cast<unsigned>((faces + 255) / 256)), dim3(256), 0, st, a);
         if (hipGetLastError() != hipSuccess) return -5;
+    }
+    PassTile tile{};
+    if (scratch && n_hi - n_lo >= kPassSteps && pass_ready(a, scratch, tile, st)) {
+        for (; n_hi - n_lo >= kPassSteps; n_hi -= kPassSteps)
+            if (launch_design_adjoint_pass(a, tile, n_hi - 1, nts, st) != hipSuccess) return -5;
     }
     for (int64_t n = n_hi - 1; n >= n_lo; --n) {
         if (nts)

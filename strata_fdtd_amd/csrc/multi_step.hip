@@ -28,29 +28,12 @@
 // here; 261x243x307 196, 61; 192^3 38.8, 18.5; 100^3 9.3, 7.2; 64^3 5.6, 5.4.
 
 #include <algorithm>
-#include <climits>
 
 #include "ade_device.hpp"
 #include "fdtd_common.hpp"
+#include "pass_device.hpp"
 
 namespace fdtd_amd {
-
-typedef float f4v __attribute__((ext_vector_type(4)));
-// rows of grids whose nz is no multiple of 4 start at any cell: 4-byte aligned
-// 16-byte accesses and byte-aligned flag words, which global memory takes
-typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-typedef uint32_t u32u __attribute__((aligned(1)));
-
-#if defined(__HIP_DEVICE_COMPILE__)
-#define CMEM __attribute__((address_space(4)))
-#else
-#define CMEM
-#endif
-// tables no kernel writes while it runs, read at wave-uniform indices
-template <typename T>
-__device__ __forceinline__ T uni(const T* t, int64_t i) {
-    return ((const CMEM T*)t)[i];
-}
 
 // The kernel's arguments where they lie (FusedArgs is the first), for code that
 // rarely runs: rare() hides the pointer's value, so its loads stay there and
@@ -68,46 +51,6 @@ __device__ __forceinline__ const CMEM FusedArgs* rare(const CMEM FusedArgs* p) {
 #endif
     return p;
 }
-
-// v, to the compiler a new value: an LDS entry read at again(v) is read where it
-// is used rather than kept in registers between uses.
-__device__ __forceinline__ int again(int v) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("" : "+v"(v));
-#endif
-    return v;
-}
-
-__device__ __forceinline__ f4v ld4(const GMEM float* base, uint32_t c) {
-    return *reinterpret_cast<const GMEM f4u*>(at32(base, c));
-}
-template <bool NTS>
-__device__ __forceinline__ void st4(GMEM float* base, uint32_t c, f4v v) {
-    if constexpr (NTS) __builtin_nontemporal_store(v, reinterpret_cast<GMEM f4u*>(at32(base, c)));
-    else *reinterpret_cast<GMEM f4u*>(at32(base, c)) = v;
-}
-
-// v where bit `bit` of byte e of f is set, else +0 (element by element)
-__device__ __forceinline__ f4v keep(f4v v, uint32_t f, int bit) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-        v[e] = __int_as_float(__float_as_int(v[e]) & __builtin_amdgcn_sbfe(static_cast<int>(f), 8 * e + bit, 1));
-    return v;
-}
-
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// flags of four air cells with every face open, and their y bits alone
-constexpr uint32_t kOpen = 0x01010101u * (FDTD_FLAG_AIR | FDTD_FLAG_OPEN_X | FDTD_FLAG_OPEN_Y | FDTD_FLAG_OPEN_Z);
-constexpr uint32_t kOpenY = 0x01010101u * FDTD_FLAG_OPEN_Y;
-constexpr int kMaxLanes = 256;      // lanes of a window row at most
-constexpr int kEvery = INT_MAX, kNowhere = INT_MIN;
-
-constexpr int kWaitLoads = 0x0f70;  // s_waitcnt vmcnt(0), the other counters unlimited
 
 // One stage's state of a thread: velocities at the stage's plane (its pressure is
 // in LDS), the updated and not yet damped vx of the plane below, the plane's flags.
