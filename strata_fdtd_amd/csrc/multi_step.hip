@@ -67,15 +67,23 @@ __device__ __forceinline__ void pass_workgroup(const CMEM FusedArgs* ka, const P
     constexpr int T = kPassSteps;
     __shared__ f4v sP[T][NT];
     __shared__ f4v sY[T][NT + 1];
-    __shared__ float sX[T][NT];
-    __shared__ float sZ[T][NT + 1];
+    // vz: nonuniform grids keep it in LDS as well (with their coefficients it would
+    // not fit the registers), uniform ones the last element and p's first alone
+    __shared__ f4v sV[NU ? T : 1][NU ? NT + 1 : 1];
+    __shared__ float sX[NU ? 1 : T][NU ? 1 : NT];
+    __shared__ float sZ[NU ? 1 : T][NU ? 1 : NT + 1];
     // nonuniform grids: damping, face and cell coefficients along k, per lane
     __shared__ f4v sK[NU ? 3 : 1][NU ? kMaxLanes : 1];
+    // the window's sources: their samples of the pass's steps, and the row and cell
+    // they act on (-1: any)
+    __shared__ double sW[NU ? FDTD_MAX_SOURCES : 1][T];
+    __shared__ int sOn[NU ? FDTD_MAX_SOURCES : 1][2];
     const int tid = threadIdx.x;
     const int nx = a.nx, ny = a.ny, nz = a.nz;
     if (tid < T) {
         sY[tid][NT] = f4v{0.f, 0.f, 0.f, 0.f};  // the row below the window's first
-        sZ[tid][NT] = 0.f;                      // the cell before its first lane
+        if constexpr (NU) sV[tid][NT] = f4v{0.f, 0.f, 0.f, 0.f};  // the cell before its first lane
+        else sZ[tid][NT] = 0.f;
     }
     const int par = static_cast<int>(s & 1);
     const GMEM float* __restrict__ P = gmem(par ? a.f[1][0] : a.f[0][0]);
@@ -175,6 +183,16 @@ __device__ __forceinline__ void pass_workgroup(const CMEM FusedArgs* ka, const P
             } else if (at == 1 ? (sj >= w0 && sj < jw) : (sj >= k0 && sj < kw)) {
                 src_i = kEvery;
             }
+            if (NU && tid < kWave && src_i != kNowhere) {
+                const bool point = a.src_kind[q] == 0;
+                sOn[q][0] = point || at == 1 ? sj : -1;
+                sOn[q][1] = point ? sk : (at == 2 ? sj : -1);
+                for (int t = 0; t < T; ++t) {
+                    const bool known = s + t < a.wave_len;
+                    if (!known) atomicOr(a.health, 2u);
+                    sW[q][t] = known ? gmem(a.wave)[q * a.wave_len + s + t] : 0.0;
+                }
+            }
         }
         if (q < a.n_sweep_probe) {
             const GMEM int32_t* __restrict__ PIJK = gmem(a.probe_ijk);
@@ -208,8 +226,23 @@ __device__ __forceinline__ void pass_workgroup(const CMEM FusedArgs* ka, const P
 #pragma unroll
     for (int t = 0; t < T; ++t) {
         sP[t][tid] = t ? zero : p0;
-        sX[t][tid] = t ? 0.f : p0.x;
+        if constexpr (!NU) sX[t][tid] = t ? 0.f : p0.x;
     }
+    // the stages' damping (and coefficients) along x: read one plane ahead and
+    // handed on from stage to stage, so that no stage waits for a scalar load
+    float dxs[T], ifs[T], ics[T];
+    auto x_tables = [&](int i, float& dx, float& ifx, float& icx) {
+        const int ic = min(i, nx - 1);
+        dx = uni(a.dec[0], ic);
+        ifx = icx = 1.f;
+        if (NU) {
+            ifx = uni(a.ifc[0], min(i, nx - 2));
+            icx = uni(a.icl[0], ic);
+        }
+    };
+#pragma unroll
+    for (int t = 1; t < T; ++t) dxs[t] = ifs[t] = ics[t] = 1.f;
+    x_tables(m0, dxs[0], ifs[0], ics[0]);
     __builtin_amdgcn_s_waitcnt(kWaitLoads);
     for (int m = m0; m < m1; ++m) {
         lds_barrier();  // the stages' pressures are posted
@@ -224,13 +257,17 @@ __device__ __forceinline__ void pass_workgroup(const CMEM FusedArgs* ka, const P
             qz = ld4(VZ, c);
             qf = flags(c);
         }
+        float dxn, ifn, icn;
+        x_tables(m + 1, dxn, ifn, icn);
         // ---- y and z faces of every stage's plane
 #pragma unroll
         for (int t = 0; t < T; ++t) {
             Stage& S = st[t];
             const f4v p = sP[t][tid];
             const f4v pu = sP[t][iu];
-            const float pr = sX[t][ir];
+            float pr;
+            if constexpr (NU) pr = sP[t][ir].x;
+            else pr = sX[t][ir];
             f4v vy = S.vy + cvy * (pu - p);
             const f4v pk = {p.y, p.z, p.w, pr};
             f4v vz;
@@ -249,9 +286,13 @@ __device__ __forceinline__ void pass_workgroup(const CMEM FusedArgs* ka, const P
 #pragma unroll
                 for (int e = 0; e < 4; ++e) vz[e] = vlast == e ? S.vz[e] : vz[e];
             }
-            S.vz = vz;
             sY[t][tid] = vy;
-            sZ[t][tid] = vz.w;
+            if constexpr (NU) {
+                sV[t][tid] = vz;
+            } else {
+                S.vz = vz;
+                sZ[t][tid] = vz.w;
+            }
         }
         lds_barrier();
         // ---- x faces and pressures, stage by stage: what stage t makes of
@@ -263,23 +304,30 @@ __device__ __forceinline__ void pass_workgroup(const CMEM FusedArgs* ka, const P
         for (int t = 0; t < T; ++t) {
             Stage& S = st[t];
             const int i = m - t;
-            const int ic = min(max(i, 0), nx - 1);
             const f4v vy = sY[t][tid];
             const f4v yb = sY[t][id];
-            const float zb = sZ[t][il];
-            const float dx = uni(a.dec[0], ic);
+            f4v vz;
+            float zb;
+            if constexpr (NU) {
+                vz = sV[t][tid];
+                zb = sV[t][il].w;
+            } else {
+                vz = S.vz;
+                zb = sZ[t][il];
+            }
+            const float dx = dxs[t];
             f4v vx = S.vx;
             const bool walls = __builtin_amdgcn_ballot_w64(((S.f | ends) & kOpen) != kOpen) != 0;
             if (i < nx - 1) {
-                const float cvx = NU ? cv * uni(a.ifc[0], ic) : cv;
+                const float cvx = NU ? cv * ifs[t] : cv;
                 vx = S.vx + cvx * (cpn - p);
                 if (walls) vx = keep(vx, S.f, 1);
             }
-            const f4v zl = {zb, S.vz.x, S.vz.y, S.vz.z};
-            const f4v dvx = vx - S.vxp, dvy = vy - yb, dvz = S.vz - zl;
+            const f4v zl = {zb, vz.x, vz.y, vz.z};
+            const f4v dvx = vx - S.vxp, dvy = vy - yb, dvz = vz - zl;
             f4v pnew;
             if (NU) {
-                const float icx = uni(a.icl[0], ic);
+                const float icx = ics[t];
                 pnew = p + cp * ((icx * dvx + icy * dvy) + sK[2][again(kl)] * dvz);
             } else {
                 pnew = p + cp * ((dvx + dvy) + dvz);
@@ -287,26 +335,45 @@ __device__ __forceinline__ void pass_workgroup(const CMEM FusedArgs* ka, const P
             if (walls) pnew = keep(pnew, S.f, 0);
             const f4v dz = NU ? sK[0][again(kl)] : dzr;
             f4v ps = ((pnew * dx) * dy) * dz;
-            const f4v ox = vx * dx, oy = vy * dy, oz = S.vz * dz;
+            const f4v ox = vx * dx, oy = vy * dy, oz = vz * dz;
             const uint64_t adds = __builtin_amdgcn_ballot_w64(src_i == i || src_i == kEvery);
             if (adds) {
-                const CMEM FusedArgs* r = rare(ka);
-                for (uint32_t sm = static_cast<uint32_t>(adds); sm; sm &= sm - 1) {
-                    const int q = __builtin_ctz(sm);
-                    // the planes or point it acts on, -1: any (its i has matched)
-                    const bool point = r->src_kind[q] == 0;
-                    const int ax = r->src_i[q], aj = r->src_j[q], ak = r->src_k[q];
-                    const int on_j = point || ax == 1 ? aj : -1;
-                    const int on_k = point ? ak : (ax == 2 ? aj : -1);
-                    const bool known = s + t < r->wave_len;
-                    if (!known && tid == 0) atomicOr(r->health, 2u);
-                    const double w = known ? uni(r->wave, q * r->wave_len + s + t) : 0.0;
-                    const uint32_t hit = (known & ((on_j == j) | (on_j < 0))) ? S.f : 0u;
+                // A z plane source acts on every plane of its windows: through the
+                // scalar loads below it costs the 320x320x480 plate 9% of its step,
+                // from LDS 3%. Uniform grids keep the loads: there the LDS form,
+                // with or without sources, made every plane 2% slower.
+                if constexpr (NU) {
+                    for (uint32_t sm = static_cast<uint32_t>(adds); sm; sm &= sm - 1) {
+                        const int q = __builtin_ctz(sm);
+                        const double w = sW[q][t];
+                        const int on_j = sOn[q][0], on_k = sOn[q][1];
+                        const uint32_t hit = ((on_j == j) | (on_j < 0)) ? S.f : 0u;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float v = static_cast<float>(static_cast<double>(ps[e]) + w);
-                        const bool on = (((hit >> (8 * e)) & FDTD_FLAG_AIR) != 0) & ((on_k == k + e) | (on_k < 0));
-                        ps[e] = on ? v : ps[e];
+                        for (int e = 0; e < 4; ++e) {
+                            const float v = static_cast<float>(static_cast<double>(ps[e]) + w);
+                            const bool on = (((hit >> (8 * e)) & FDTD_FLAG_AIR) != 0) & ((on_k == k + e) | (on_k < 0));
+                            ps[e] = on ? v : ps[e];
+                        }
+                    }
+                } else {
+                    const CMEM FusedArgs* r = rare(ka);
+                    for (uint32_t sm = static_cast<uint32_t>(adds); sm; sm &= sm - 1) {
+                        const int q = __builtin_ctz(sm);
+                        // the planes or point it acts on, -1: any (its i has matched)
+                        const bool point = r->src_kind[q] == 0;
+                        const int ax = r->src_i[q], aj = r->src_j[q], ak = r->src_k[q];
+                        const int on_j = point || ax == 1 ? aj : -1;
+                        const int on_k = point ? ak : (ax == 2 ? aj : -1);
+                        const bool known = s + t < r->wave_len;
+                        if (!known && tid == 0) atomicOr(r->health, 2u);
+                        const double w = known ? uni(r->wave, q * r->wave_len + s + t) : 0.0;
+                        const uint32_t hit = (known & ((on_j == j) | (on_j < 0))) ? S.f : 0u;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const float v = static_cast<float>(static_cast<double>(ps[e]) + w);
+                            const bool on = (((hit >> (8 * e)) & FDTD_FLAG_AIR) != 0) & ((on_k == k + e) | (on_k < 0));
+                            ps[e] = on ? v : ps[e];
+                        }
                     }
                 }
             }
@@ -354,7 +421,7 @@ __device__ __forceinline__ void pass_workgroup(const CMEM FusedArgs* ka, const P
             S = Stage{cx, cy, cz, vx, cf};
             if (t + 1 < T) p = sP[t + 1][tid];  // read before the next stage's p is posted
             sP[t][tid] = cpn;
-            sX[t][tid] = cpn.x;
+            if constexpr (!NU) sX[t][tid] = cpn.x;
             cpn = ps;
             cx = ox;
             cy = oy;
@@ -362,6 +429,15 @@ __device__ __forceinline__ void pass_workgroup(const CMEM FusedArgs* ka, const P
             cf = f;
         }
         pn = qp;
+#pragma unroll
+        for (int t = T - 1; t > 0; --t) {
+            dxs[t] = dxs[t - 1];
+            ifs[t] = ifs[t - 1];
+            ics[t] = ics[t - 1];
+        }
+        dxs[0] = dxn;
+        ifs[0] = ifn;
+        ics[0] = icn;
     }
 }
 
