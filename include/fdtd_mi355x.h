@@ -365,7 +365,10 @@ int fdtd_design_adjoint(float* const* lam, const uint8_t* flags, const float* co
  * fdtd_design_pass_floats entries (adjoint 0 for the forward alone), in which
  * three steps are taken per pass over the fields where the grid has such passes
  * (the rest, and everything if scratch is NULL, one by one). The results are the
- * same bit for bit. The fields and flags must be readable 4 cells past their end. */
+ * same bit for bit. The fields and flags must be readable 4 cells past their end.
+ * With scratch the history's rows along k are whole 4-cell lanes (from multiples of
+ * 4 on): fdtd_design_pass_history gives the floats per step of its p and div. */
+int fdtd_design_pass_history(const int32_t* box_lo, const int32_t* box_hi, int64_t* p_floats, int64_t* div_floats);
 int64_t fdtd_design_pass_floats(const int32_t* box_lo, const int32_t* box_hi, int adjoint);
 int fdtd_design_forward_passes(float* const* fields, const uint8_t* flags, const float* const* dec, int nx, int ny,
                                int nz, float cv0, float cp0, const int32_t* box_lo, const int32_t* box_hi,

@@ -190,7 +190,8 @@ class _Fast:
     PLANES = 2
     ADJ_PLANES = 4
 
-    def __init__(self, dv: _Device):
+    def __init__(self, dv: _Device, adjoint: bool = False):
+        """adjoint: the solve records the history its adjoint will read."""
         import torch
         self.dv = dv
         pb = dv.pb
@@ -200,23 +201,22 @@ class _Fast:
         self.probe_ijk = torch.tensor(np.array(pb.probes or [(0, 0, 0)], dtype=np.int32).reshape(-1, 3),
                                       device=dv.dev)
         self.dec = (_vp * 3)(*[_ptr(d) for d in dv.dec])
-        lo, hi = np.array(pb.box_lo), np.array(pb.box_hi)
-        self.ecells = int(np.prod(hi - lo + 2))
-        self.bcells = int(np.prod(hi - lo))
-        self._scratch = None
-
-    def _pass_scratch(self, adjoint: bool):
-        """Device scratch of the multi-step passes (face coefficients; for the
-        adjoint also the steps' velocities and pb on the box), kept for this
-        solve; None (single steps) where there is no room for it."""
-        import torch
-        n = _native.load().fdtd_design_pass_floats(self.dv.lo.ctypes.data, self.dv.hi.ctypes.data, int(adjoint))
-        if n > 0 and (self._scratch is None or self._scratch.numel() < n):
-            try:
-                self._scratch = torch.empty(n, dtype=torch.float32, device=self.dv.dev)
-            except torch.cuda.OutOfMemoryError:
-                return None
-        return self._scratch if n > 0 else None
+        # Scratch of the multi-step passes (face coefficients; for the adjoint also
+        # its steps' velocities and pb on the box), kept with the solve. Without
+        # room for it every step is taken singly, and the history's rows are the
+        # box's own rather than whole 4-cell lanes.
+        n = _lib().fdtd_design_pass_floats(dv.lo.ctypes.data, dv.hi.ctypes.data, int(adjoint))
+        try:
+            self._scratch = torch.empty(n, dtype=torch.float32, device=dv.dev) if n > 0 else None
+        except torch.cuda.OutOfMemoryError:
+            self._scratch = None
+        if self._scratch is not None:
+            e, d = C.c_int64(), C.c_int64()
+            _native.call("fdtd_design_pass_history", dv.lo.ctypes.data, dv.hi.ctypes.data, C.byref(e), C.byref(d))
+            self.ecells, self.bcells = e.value, d.value
+        else:
+            lo, hi = np.array(pb.box_lo), np.array(pb.box_hi)
+            self.ecells, self.bcells = int(np.prod(hi - lo + 2)), int(np.prod(hi - lo))
 
     @staticmethod
     def _sets(sets):
@@ -249,7 +249,7 @@ class _Fast:
         _native.call("fdtd_design_forward_passes", self._sets(sets), *self._common(rk), self.src,
                      _ptr(self.wave_dev), self.dv.n_probe, _ptr(self.probe_ijk), _ptr(trace),
                      min(rows, self.wave_dev.numel()), step0, n_steps, _ptr(hp), _ptr(hd), hist0, hist_steps,
-                     self.PLANES, _ptr(self._pass_scratch(False)), self.dv.stream)
+                     self.PLANES, _ptr(self._scratch), self.dv.stream)
 
     def adjoint(self, lam, rk, g, n_lo, n_hi, hist, hist0, acc):
         """acc: float32 [box][4], Kahan (sum, compensation) of dL/dr, then dL/dkappa."""
@@ -258,11 +258,11 @@ class _Fast:
         if getattr(self, "_faces", None) is None:
             n = _native.load().fdtd_design_face_count(self.dv.lo.ctypes.data, self.dv.hi.ctypes.data)
             self._faces = torch.empty(n, dtype=torch.float32, device=self.dv.dev)
-            self._pb_box = torch.empty(2 * self.bcells, dtype=torch.float32, device=self.dv.dev)
+            self._pb_box = torch.empty(2 * int(np.prod(self.dv.pb.box_shape)), dtype=torch.float32, device=self.dv.dev)
         _native.call("fdtd_design_adjoint_passes", self._sets(lam), *self._common(rk), self.dv.n_probe,
                      _ptr(self.probe_ijk), _ptr(g), g.shape[0], n_lo, n_hi, _ptr(hp), _ptr(hd), hist0,
                      hp.numel() // self.ecells, _ptr(acc), _ptr(self._faces), _ptr(self._pb_box), self.ADJ_PLANES,
-                     _ptr(self._pass_scratch(True)), self.dv.stream)
+                     _ptr(self._scratch), self.dv.stream)
 
 
 def history_bytes(pb: DesignProblem, steps: int | None = None) -> int:
@@ -282,7 +282,7 @@ def _pick_history(pb: DesignProblem, history: str, device) -> str:
 
 def _forward_fast(pb, r, kappa, dv, history: str):
     import torch
-    fast = _Fast(dv)
+    fast = _Fast(dv, adjoint=history in ("all", "checkpoint"))
     rk = fast.pack(r, kappa)
     rec = None
     if history == "checkpoint":

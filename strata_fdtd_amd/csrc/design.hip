@@ -371,10 +371,11 @@ __device__ __forceinline__ void design_forward_box_strip(const DesignArgs& a, in
                             a.trace[s * a.n_probe + q] = pnew;
                 if (hist) {
                     if (ei.in && ej[r].in && ek.in)
-                        stx_nt(hp, static_cast<uint32_t>((ei.off * (by + 2) + ej[r].off) * (bz + 2) + ek.off), pr);
+                        stx_nt(hp, static_cast<uint32_t>((ei.off * (by + 2) + ej[r].off) * a.p_nk + (k - a.p_k0)), pr);
                     // the history is read back only by the adjoint, much later:
                     // non-temporal, so it does not evict the fields from the caches
-                    if (di.in && dj[r].in && dk.in) stx_nt(hd, static_cast<uint32_t>(boff(di, dj[r], dk)), div);
+                    if (di.in && dj[r].in && dk.in)
+                        stx_nt(hd, static_cast<uint32_t>((di.off * by + dj[r].off) * a.d_nk + (k - a.d_k0)), div);
                 }
             }
             vxm[r] = vxn;
@@ -941,8 +942,9 @@ __global__ __launch_bounds__(256) void k_design_grad(const DesignArgs a, int64_t
     const uint32_t sx = static_cast<uint32_t>(ny) * static_cast<uint32_t>(nz);
     const uint32_t c = cix(i, j, k, ny, nz);
     GMEM f4v* __restrict__ ACC = gm(a.acc);
-    const int ey = by + 2, ez = bz + 2;
-    const uint32_t e = static_cast<uint32_t>(((bi + 1) * ey + (bj + 1)) * ez + (bk + 1));
+    const int ey = by + 2, ez = a.p_nk;
+    const uint32_t e = static_cast<uint32_t>(((bi + 1) * ey + (bj + 1)) * ez + (k - a.p_k0));
+    const uint32_t d = static_cast<uint32_t>((bi * by + bj) * a.d_nk + (k - a.d_k0));
     // gradient factors of the six faces (below: the face's own cell; above:
     // the +d neighbour's index in the axis' array)
     const GMEM float* __restrict__ EX = gm(a.face_e);
@@ -972,7 +974,7 @@ __global__ __launch_bounds__(256) void k_design_grad(const DesignArgs a, int64_t
         const float wx = ldo(WX, c), wy = ldo(WY, c), wz = ldo(WZ, c);
         const float wxm = ldo(WX, c - sx), wym = ldo(WY, c - static_cast<uint32_t>(nz)), wzm = ldo(WZ, c - 1u);
         const float pb = ldo(gm(a.pbb[par]), b);
-        const float dv = ldo(hd, b);
+        const float dv = ldo(hd, d);
         float gr = 0.f;
         gr += wx * (hxp - hpc) * exp_;
         gr += wy * (hyp - hpc) * eyp;
@@ -1062,18 +1064,17 @@ hipError_t launch_design_adjoint_pass(const DesignArgs& a, const PassTile& m, in
 // floats; each part starts on 16 bytes.
 static int64_t pass_layout(const DesignArgs& a, int64_t off[3]) {
     auto round4 = [](int64_t n) { return (n + 3) & ~int64_t(3); };
-    const int64_t box = static_cast<int64_t>(a.hi[0] - a.lo[0]) * (a.hi[1] - a.lo[1]) * (a.hi[2] - a.lo[2]);
     off[0] = 0;
     off[1] = round4(4 * coef_cells(a));
-    off[2] = off[1] + round4(3 * (kPassSteps - 1) * wall_cells(a));
-    return off[2] + round4(kPassSteps * box);
+    off[2] = off[1] + round4(3 * (kPassSteps - 1) * coef_cells(a));
+    return off[2] + round4(kPassSteps * dbox_cells(a));
 }
 
 // The split of the grid and the coefficients for a call's passes; false where the
-// grid has no passes (the call then steps one by one). 32-bit offsets: four
-// coefficients and three velocities per cell of boxes below 2^26 cells.
+// grid has no passes (the call then steps one by one). 32-bit byte offsets: boxes
+// below 2^26 cells.
 static bool pass_ready(DesignArgs& a, float* scratch, PassTile& tile, hipStream_t st) {
-    if (coef_cells(a) >= (1ll << 26) || wall_cells(a) >= (1ll << 26) || !design_pass_tile(a, tile)) return false;
+    if (coef_cells(a) >= (1ll << 26) || !design_pass_tile(a, tile)) return false;
     int64_t off[3];
     pass_layout(a, off);
     a.pass_w = scratch + off[1];
@@ -1163,9 +1164,24 @@ int64_t fdtd_design_pass_floats(const int32_t* box_lo, const int32_t* box_hi, in
         a.hi[d] = box_hi[d];
         if (a.lo[d] < 1 || a.hi[d] <= a.lo[d]) return -3;
     }
+    history_rows(a, true);
     int64_t off[3];
     const int64_t all = pass_layout(a, off);
     return adjoint ? all : off[1];
+}
+
+int fdtd_design_pass_history(const int32_t* box_lo, const int32_t* box_hi, int64_t* p_floats, int64_t* div_floats) {
+    if (!box_lo || !box_hi || !p_floats || !div_floats) return -2;
+    DesignArgs a{};
+    for (int d = 0; d < 3; ++d) {
+        a.lo[d] = box_lo[d];
+        a.hi[d] = box_hi[d];
+        if (a.lo[d] < 1 || a.hi[d] <= a.lo[d]) return -3;
+    }
+    history_rows(a, true);
+    *p_floats = ebox_cells(a);
+    *div_floats = dbox_cells(a);
+    return 0;
 }
 
 int fdtd_design_forward(float* const* fields, const uint8_t* flags, const float* const* dec, int nx, int ny, int nz,
@@ -1197,6 +1213,7 @@ int fdtd_design_forward_passes(float* const* fields, const uint8_t* flags, const
     a.hist_div = hist_div;
     a.hist0 = hist0;
     a.hist_steps = hist_p ? hist_steps : 0;
+    history_rows(a, scratch != nullptr);
     const int blocks = design_grid(a, planes, kDesignRows, kDesignRows);
     hipStream_t st = static_cast<hipStream_t>(stream);
     const bool nts = static_cast<int64_t>(nx) * ny * nz > kCacheResidentCells;
@@ -1246,6 +1263,7 @@ int fdtd_design_adjoint_passes(float* const* lam, const uint8_t* flags, const fl
     a.hist_div = const_cast<float*>(hist_div);
     a.hist0 = hist0;
     a.hist_steps = hist_steps;
+    history_rows(a, scratch != nullptr);
     a.acc = reinterpret_cast<f4v*>(acc);
     a.face_e = face_e;
     const int blocks = design_grid(a, planes, kDesignAdjRows, kDesignAdjBoxRows);

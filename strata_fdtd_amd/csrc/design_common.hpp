@@ -34,6 +34,11 @@ struct DesignArgs {
     float* hist_div;
     int64_t hist0;
     int64_t hist_steps;
+    // their rows along k: p_nk elements from cell p_k0 on (d_nk, d_k0: div). As
+    // long as the boxes, or whole 4-cell lanes for passes (a lane cut by the box's
+    // edge takes five stores instead of one: with 9 of them per plane they were a
+    // third of a pass)
+    int p_k0, p_nk, d_k0, d_nk;
     // gradient accumulators on the box: Kahan (sum, compensation) of dL/dr,
     // then of dL/dkappa, per voxel
     f4v* acc;
@@ -52,7 +57,7 @@ struct DesignArgs {
     // multi-step passes: face coefficients along x, y, z and the cell coefficient
     // of the box grown by one cell below, its lanes whole ([4][coef_cells()]), the
     // updated velocities of an adjoint pass's first steps there ([steps - 1][3]
-    // [wall_cells()]) and the pb of its steps ([steps][box])
+    // [coef_cells()]) and the pb of its steps ([steps][dbox_cells()])
     const float* coef;
     float* pass_w;
     float* pass_pb;
@@ -60,12 +65,12 @@ struct DesignArgs {
     int box_planes, b_i0, b_i1, nb_i;
 };
 
-__device__ __forceinline__ int64_t ebox_cells(const DesignArgs& a) {
-    return static_cast<int64_t>(a.hi[0] - a.lo[0] + 2) * (a.hi[1] - a.lo[1] + 2) * (a.hi[2] - a.lo[2] + 2);
+__host__ __device__ inline int64_t ebox_cells(const DesignArgs& a) {
+    return static_cast<int64_t>(a.hi[0] - a.lo[0] + 2) * (a.hi[1] - a.lo[1] + 2) * a.p_nk;
 }
 
-__device__ __forceinline__ int64_t dbox_cells(const DesignArgs& a) {
-    return static_cast<int64_t>(a.hi[0] - a.lo[0]) * (a.hi[1] - a.lo[1]) * (a.hi[2] - a.lo[2]);
+__host__ __device__ inline int64_t dbox_cells(const DesignArgs& a) {
+    return static_cast<int64_t>(a.hi[0] - a.lo[0]) * (a.hi[1] - a.lo[1]) * a.d_nk;
 }
 
 __device__ __forceinline__ float cvf(const DesignArgs& a, float r_lo, float r_hi) {
@@ -112,9 +117,19 @@ __host__ __device__ inline int coef_nk(const DesignArgs& a) { return ((a.hi[2] +
 __host__ __device__ inline int64_t coef_cells(const DesignArgs& a) {
     return static_cast<int64_t>(a.hi[0] - a.lo[0] + 1) * (a.hi[1] - a.lo[1] + 1) * coef_nk(a);
 }
-// The box and the cells whose upper faces are its lower ones.
-__host__ __device__ inline int64_t wall_cells(const DesignArgs& a) {
-    return static_cast<int64_t>(a.hi[0] - a.lo[0] + 1) * (a.hi[1] - a.lo[1] + 1) * (a.hi[2] - a.lo[2] + 1);
+// The history's rows: the boxes' own, or whole lanes.
+inline void history_rows(DesignArgs& a, bool lanes) {
+    a.p_k0 = a.lo[2] - 1;
+    a.d_k0 = a.lo[2];
+    int p_end = a.hi[2] + 1, d_end = a.hi[2];
+    if (lanes) {
+        a.p_k0 &= ~3;
+        a.d_k0 &= ~3;
+        p_end = (p_end + 3) & ~3;
+        d_end = (d_end + 3) & ~3;
+    }
+    a.p_nk = p_end - a.p_k0;
+    a.d_nk = d_end - a.d_k0;
 }
 
 }  // namespace fdtd_amd

@@ -5,10 +5,10 @@
 // sweeps in design.hip, so the results are the same bit for bit.
 //
 // A voxel's face and cell coefficients (k_design_coefs, formed once per call by the
-// same division of the same two r values) are loaded with its plane and travel
-// from stage to stage with it in registers, which takes about 200 of them: one
-// workgroup of 512 threads per CU, 2 waves per SIMD. Recomputing them in each
-// stage would cost three IEEE divisions per cell and step.
+// same division of the same two r values; in the stages it would be three IEEE
+// divisions per cell and step) are loaded with its plane and stay in LDS, a slot
+// per plane in flight, until the last stage has used them. With the stages'
+// exchange that is the LDS of a CU for one workgroup of 512 threads.
 //
 // What bounds them at 192^3 with a 128^3 box (both sets, coefficients and flags in
 // the Infinity Cache): the latency of a plane's two LDS phases and its vector
@@ -72,21 +72,20 @@ __device__ __forceinline__ f4v coef_at(const CoefLane& c, int q, int i, float ai
     return v;
 }
 
-// Elements of a lane's value whose k lies in [lo, lo + n): row[k - lo] = v,
-// non-temporal (NT) for what is read much later.
+// A thread's place in the planes of a box array whose rows are whole lanes, n cells
+// from cell k0 (a multiple of 4) on: row `row` of `rows`.
+struct BoxLane {
+    uint32_t off;
+    bool in;
+};
+__device__ __forceinline__ BoxLane box_lane(const PassWindow& w, int row, int rows, int k0, int n) {
+    BoxLane b{0u, w.out && row >= 0 && row < rows && w.k >= k0 && w.k < k0 + n};
+    if (b.in) b.off = static_cast<uint32_t>(row * n + (w.k - k0));
+    return b;
+}
 template <bool NT>
-__device__ __forceinline__ void st_range(GMEM float* row, int k, int lo, int n, f4v v) {
-    const int b = k - lo;
-    if (b >= 0 && b + 4 <= n) {
-        st4<NT>(row, static_cast<uint32_t>(b), v);
-    } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (static_cast<unsigned>(b + e) < static_cast<unsigned>(n)) {
-                if constexpr (NT) stx_nt(row, static_cast<uint32_t>(b + e), v[e]);
-                else stx(row, static_cast<uint32_t>(b + e), v[e]);
-            }
-    }
+__device__ __forceinline__ void st_box(GMEM float* plane, const BoxLane& b, f4v v) {
+    if (b.in) st4<NT>(plane, b.off, v);
 }
 
 // Lane q of a wave holds probe q's plane if the probe lies in the given rows and
@@ -99,7 +98,6 @@ __device__ __forceinline__ int probe_plane(const DesignArgs& a, int lane, int j0
 
 struct ForwardStage {
     f4v vx, vy, vz, vxp;
-    f4v cx, cy, cz, cp;
     uint32_t f;
 };
 
@@ -112,6 +110,8 @@ __global__ __launch_bounds__(kDesignPassThreads) __attribute__((amdgpu_waves_per
     __shared__ f4v sY[T][NT + 1];
     __shared__ float sX[T][NT];
     __shared__ float sZ[T][NT + 1];
+    // the coefficients of the stages' planes (plane i in slot i mod T), each thread's own
+    __shared__ f4v sC[T][4][NT];
     const int lb = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
     if (lb >= mt.nwg) return;
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
@@ -136,14 +136,15 @@ __global__ __launch_bounds__(kDesignPassThreads) __attribute__((amdgpu_waves_per
     for (int e = 0; e < 4; ++e)
         if (w.ld && w.k + e < nz) dz[e] = a.dec[2][w.k + e];
     const int probe_i = probe_plane(a, lane, w.jlo, w.jhi, w.klo, w.khi);
-    // history: rows of p on the box grown by one cell, of div on the box
+    // history: p on the box grown by one cell, div on the box
     const int bx = a.hi[0] - a.lo[0], by = a.hi[1] - a.lo[1], bz = a.hi[2] - a.lo[2];
-    const int ej = w.j - a.lo[1] + 1;
-    const bool hist_j = a.hist_p && w.out && ej >= 0 && ej < by + 2 && w.k + 3 >= a.lo[2] - 1 && w.k < a.hi[2] + 1;
+    const uint32_t p_plane = static_cast<uint32_t>((by + 2) * a.p_nk), d_plane = static_cast<uint32_t>(by * a.d_nk);
+    const BoxLane pl = box_lane(w, w.j - a.lo[1] + 1, by + 2, a.p_k0, a.p_nk);
+    const BoxLane dl = box_lane(w, w.j - a.lo[1], by, a.d_k0, a.d_nk);
 
     ForwardStage st[T];
 #pragma unroll
-    for (int t = 0; t < T; ++t) st[t] = ForwardStage{zero, zero, zero, zero, zero, zero, zero, zero, 0u};
+    for (int t = 0; t < T; ++t) st[t] = ForwardStage{zero, zero, zero, zero, 0u};
     const int m0 = max(w.i0 - T, 0), m1 = w.i1 + T - 1;
     auto at = [&](int i) { return static_cast<uint32_t>(i) * sx + w.c0; };
     auto flags = [&](uint32_t c) -> uint32_t { return *reinterpret_cast<const GMEM u32u*>(at32(FL, c)); };
@@ -157,10 +158,26 @@ __global__ __launch_bounds__(kDesignPassThreads) __attribute__((amdgpu_waves_per
         st[0].f = flags(c);
         if (m0 + 1 < nx) pn = ld4(P, c + sx);
     }
-    st[0].cx = coef_at(cl, 0, m0, a.cv0);
-    st[0].cy = coef_at(cl, 1, m0, a.cv0);
-    st[0].cz = coef_at(cl, 2, m0, a.cv0);
-    st[0].cp = coef_at(cl, 3, m0, a.cp0);
+    int slot[T];  // of the stages' planes
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        slot[t] = (T - t) % T;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) sC[slot[t]][q][tid] = t ? zero : coef_at(cl, q, m0, q < 3 ? a.cv0 : a.cp0);
+    }
+    float dxs[T], dxn;
+#pragma unroll
+    for (int t = 1; t < T; ++t) dxs[t] = 1.f;
+    dxs[0] = uni(a.dec[0], m0);
+    // history of the pass's steps that are recorded (null: none)
+    GMEM float *hps[T], *hds[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        const int64_t h = s + t - a.hist0;
+        const bool on = a.hist_p && h >= 0 && h < a.hist_steps;
+        hps[t] = on ? gmem(a.hist_p + h * ebox_cells(a)) : nullptr;
+        hds[t] = on ? gmem(a.hist_div + h * dbox_cells(a)) : nullptr;
+    }
 #pragma unroll
     for (int t = 0; t < T; ++t) {
         sP[t][tid] = t ? zero : p0;
@@ -180,8 +197,10 @@ __global__ __launch_bounds__(kDesignPassThreads) __attribute__((amdgpu_waves_per
             qz = ld4(VZ, c);
             qf = flags(c);
         }
-        f4v ccx = coef_at(cl, 0, m + 1, a.cv0), ccy = coef_at(cl, 1, m + 1, a.cv0);
-        f4v ccz = coef_at(cl, 2, m + 1, a.cv0), ccp = coef_at(cl, 3, m + 1, a.cp0);
+        f4v qc[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) qc[q] = coef_at(cl, q, m + 1, q < 3 ? a.cv0 : a.cp0);
+        dxn = uni(a.dec[0], min(m + 1, nx - 1));
         // ---- y and z faces of every stage's plane
 #pragma unroll
         for (int t = 0; t < T; ++t) {
@@ -189,9 +208,9 @@ __global__ __launch_bounds__(kDesignPassThreads) __attribute__((amdgpu_waves_per
             const f4v p = sP[t][tid];
             const f4v pu = sP[t][w.iu];
             const float pr = sX[t][w.ir];
-            f4v vy = keep(S.vy + S.cy * (pu - p), S.f, 2);
+            f4v vy = keep(S.vy + sC[slot[t]][1][tid] * (pu - p), S.f, 2);
             const f4v pk = {p.y, p.z, p.w, pr};
-            f4v vz = keep(S.vz + S.cz * (pk - p), S.f, 3);
+            f4v vz = keep(S.vz + sC[slot[t]][2][tid] * (pk - p), S.f, 3);
             // the last faces keep their velocity
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -207,6 +226,7 @@ __global__ __launch_bounds__(kDesignPassThreads) __attribute__((amdgpu_waves_per
         f4v cpn = pn, cx = qx, cy = qy, cz = qz;
         uint32_t cf = qf;
         f4v p = sP[0][tid];
+        f4v hp[T], hd[T];  // the history's p and div
 #pragma unroll
         for (int t = 0; t < T; ++t) {
             ForwardStage& S = st[t];
@@ -214,12 +234,12 @@ __global__ __launch_bounds__(kDesignPassThreads) __attribute__((amdgpu_waves_per
             const f4v vy = sY[t][tid];
             const f4v yb = sY[t][w.id];
             const float zb = sZ[t][w.il];
-            const float dx = uni(a.dec[0], min(max(i, 0), nx - 1));
+            const float dx = dxs[t];
             f4v vx = S.vx;
-            if (i < nx - 1) vx = keep(S.vx + S.cx * (cpn - p), S.f, 1);
+            if (i < nx - 1) vx = keep(S.vx + sC[slot[t]][0][tid] * (cpn - p), S.f, 1);
             const f4v zl = {zb, S.vz.x, S.vz.y, S.vz.z};
             const f4v div = ((vx - S.vxp) + (vy - yb)) + (S.vz - zl);
-            f4v ps = ((keep(p + S.cp * div, S.f, 0) * dx) * dy) * dz;
+            f4v ps = ((keep(p + sC[slot[t]][3][tid] * div, S.f, 0) * dx) * dy) * dz;
             if (i == a.src_i && w.j == a.src_j && a.src_k >= w.k && a.src_k < w.k + 4) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
@@ -236,27 +256,11 @@ __global__ __launch_bounds__(kDesignPassThreads) __attribute__((amdgpu_waves_per
                     a.trace[(s + t) * a.n_probe + q] = e == 0 ? ps.x : (e == 1 ? ps.y : (e == 2 ? ps.z : ps.w));
                 }
             }
-            const int64_t slot = s + t - a.hist0;
-            const int ei = i - a.lo[0] + 1;
-            if (hist_j && mine && slot >= 0 && slot < a.hist_steps && ei >= 0 && ei < bx + 2) {
-                GMEM float* hp = gmem(a.hist_p + slot * ebox_cells(a)) + (static_cast<uint32_t>(ei * (by + 2) + ej) * (bz + 2));
-                st_range<true>(hp, w.k, a.lo[2] - 1, bz + 2, p);
-                if (ei > 0 && ei <= bx && ej > 0 && ej <= by) {
-                    GMEM float* hd = gmem(a.hist_div + slot * dbox_cells(a)) +
-                                     (static_cast<uint32_t>((ei - 1) * by + ej - 1) * bz);
-                    st_range<true>(hd, w.k, a.lo[2], bz, div);
-                }
-            }
-            if (t == T - 1 && w.out && i >= w.i0) {
-                const uint32_t c = at(i);
-                st_lane<NTS>(gmem(a.f[par ^ 1][0]), c, ps, w.nv);
-                st_lane<NTS>(gmem(a.f[par ^ 1][1]), c, ox, w.nv);
-                st_lane<NTS>(gmem(a.f[par ^ 1][2]), c, oy, w.nv);
-                st_lane<NTS>(gmem(a.f[par ^ 1][3]), c, oz, w.nv);
-            }
+            hp[t] = p;
+            hd[t] = div;
             // this stage's next plane: what came in (loads, or the stage before)
-            const ForwardStage old = S;
-            S = ForwardStage{cx, cy, cz, vx, ccx, ccy, ccz, ccp, cf};
+            const uint32_t f = S.f;
+            S = ForwardStage{cx, cy, cz, vx, cf};
             if (t + 1 < T) p = sP[t + 1][tid];  // read before the next stage's p is posted
             sP[t][tid] = cpn;
             sX[t][tid] = cpn.x;
@@ -264,13 +268,41 @@ __global__ __launch_bounds__(kDesignPassThreads) __attribute__((amdgpu_waves_per
             cx = ox;
             cy = oy;
             cz = oz;
-            ccx = old.cx;
-            ccy = old.cy;
-            ccz = old.cz;
-            ccp = old.cp;
-            cf = old.f;
+            cf = f;
         }
         pn = qp;
+        // Every store of the plane comes after the wait for the next one's loads:
+        // a wait behind them would be for the stores as well (with the history
+        // stored stage by stage, box or not, a step took 10 us longer).
+        __builtin_amdgcn_s_waitcnt(kWaitLoads);
+        {
+            const int i = m - (T - 1);
+            if (w.out && i >= w.i0) {
+                const uint32_t c = at(i);
+                st_lane<NTS>(gmem(a.f[par ^ 1][0]), c, cpn, w.nv);
+                st_lane<NTS>(gmem(a.f[par ^ 1][1]), c, cx, w.nv);
+                st_lane<NTS>(gmem(a.f[par ^ 1][2]), c, cy, w.nv);
+                st_lane<NTS>(gmem(a.f[par ^ 1][3]), c, cz, w.nv);
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            const int i = m - t, ei = i - a.lo[0] + 1;
+            if (!hps[t] || i < w.i0 || i >= w.i1 || ei < 0 || ei >= bx + 2) continue;  // uniform
+            st_box<true>(hps[t] + ei * p_plane, pl, hp[t]);
+            if (ei > 0 && ei <= bx) st_box<true>(hds[t] + (ei - 1) * d_plane, dl, hd[t]);
+        }
+        // the slot of the plane that left the last stage takes the next plane's
+        const int free_slot = slot[T - 1];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) sC[free_slot][q][tid] = qc[q];
+#pragma unroll
+        for (int t = T - 1; t > 0; --t) {
+            slot[t] = slot[t - 1];
+            dxs[t] = dxs[t - 1];
+        }
+        slot[0] = free_slot;
+        dxs[0] = dxn;
     }
 }
 
@@ -278,7 +310,6 @@ struct AdjointStage {
     f4v vx, vy, vz;                 // lambda's velocities at the stage's plane
     f4v cwx;                        // cv w of the x face below it
     f4v pb;                         // its pb (q is in LDS)
-    f4v cx, cy, cz, cp;
     uint32_t f;
 };
 
@@ -295,6 +326,9 @@ __global__ __launch_bounds__(kDesignPassThreads) __attribute__((amdgpu_waves_per
     __shared__ f4v sY[T][NT + 1];
     __shared__ float sX[T][NT];
     __shared__ float sZ[T][NT + 1];
+    // the coefficients of the stages' planes (plane i in slot i mod T), each
+    // thread's own; a cell's own coefficient was used a plane ahead
+    __shared__ f4v sC[T][4][NT];
     const int lb = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
     if (lb >= mt.nwg) return;
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
@@ -320,13 +354,14 @@ __global__ __launch_bounds__(kDesignPassThreads) __attribute__((amdgpu_waves_per
         if (w.ld && w.k + e < nz) dz[e] = a.dec[2][w.k + e];
     const int probe_i = probe_plane(a, lane, w.w0, w.w0 + mt.rows, w.k0, w.k0 + 4 * mt.kt);
     const int bx = a.hi[0] - a.lo[0], by = a.hi[1] - a.lo[1], bz = a.hi[2] - a.lo[2];
-    const int wj = w.j - a.lo[1] + 1;  // row in the box grown by one cell below
-    const bool box_j = w.out && wj >= 0 && wj <= by && w.k + 3 >= a.lo[2] - 1 && w.k < a.hi[2];
+    const uint32_t b_plane = static_cast<uint32_t>(by * a.d_nk), w_plane = static_cast<uint32_t>((by + 1) * coef_nk(a));
+    const BoxLane pl = box_lane(w, w.j - a.lo[1], by, a.d_k0, a.d_nk);
+    const BoxLane wl = box_lane(w, w.j - a.lo[1] + 1, by + 1, coef_k0(a), coef_nk(a));
 
     auto at = [&](int i) { return static_cast<uint32_t>(i) * sx + w.c0; };
     auto flags = [&](uint32_t c) -> uint32_t { return *reinterpret_cast<const GMEM u32u*>(at32(FL, c)); };
     // pb of plane i from its pressure at adjoint step n - t
-    auto pb_of = [&](f4v p, int i, int t) -> f4v {
+    auto pb_of = [&](f4v p, int i, int t, float dx) -> f4v {
         for (uint64_t pm = __builtin_amdgcn_ballot_w64(probe_i == i); pm; pm &= pm - 1) {
             const int q = __builtin_ctzll(pm);
             const int pj = a.probe[3 * q + 1], pk = a.probe[3 * q + 2];
@@ -335,13 +370,12 @@ __global__ __launch_bounds__(kDesignPassThreads) __attribute__((amdgpu_waves_per
                 for (int e = 0; e < 4; ++e)
                     if (w.k + e == pk) p[e] += a.g[(n - t) * a.n_probe + q];
         }
-        const float dxy = uni(a.dec[0], min(max(i, 0), nx - 1)) * dy;
-        return (dxy * dz) * p;
+        return ((dx * dy) * dz) * p;
     };
 
     AdjointStage st[T];
 #pragma unroll
-    for (int t = 0; t < T; ++t) st[t] = AdjointStage{zero, zero, zero, zero, zero, zero, zero, zero, zero, 0u};
+    for (int t = 0; t < T; ++t) st[t] = AdjointStage{zero, zero, zero, zero, zero, 0u};
     const int m0 = max(w.i0 - T, 0), m1 = w.i1 + T - 1;
     f4v p0 = zero, pn = zero, cpl = zero;   // cpl: cp of plane m + 1
     uint32_t fn = 0;                        // flags of plane m + 1
@@ -357,14 +391,23 @@ __global__ __launch_bounds__(kDesignPassThreads) __attribute__((amdgpu_waves_per
             fn = flags(c + sx);
         }
     }
-    st[0].cx = coef_at(cl, 0, m0, a.cv0);
-    st[0].cy = coef_at(cl, 1, m0, a.cv0);
-    st[0].cz = coef_at(cl, 2, m0, a.cv0);
-    st[0].cp = coef_at(cl, 3, m0, a.cp0);
+    int slot[T];  // of the stages' planes
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        slot[t] = (T - t) % T;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) sC[slot[t]][q][tid] = t ? zero : coef_at(cl, q, m0, q < 3 ? a.cv0 : a.cp0);
+    }
     cpl = coef_at(cl, 3, m0 + 1, a.cp0);
-    st[0].pb = pb_of(p0, m0, 0);
+    // the damping of the stages' planes along x, and of the plane ahead of stage 0
+    float dxs[T + 1], dxn;
+#pragma unroll
+    for (int t = 2; t <= T; ++t) dxs[t] = 1.f;
+    dxs[1] = uni(a.dec[0], m0);
+    dxs[0] = uni(a.dec[0], min(m0 + 1, nx - 1));
+    st[0].pb = pb_of(p0, m0, 0, dxs[1]);
     {
-        const f4v q0 = keep(st[0].cp * st[0].pb, st[0].f, 0);
+        const f4v q0 = keep(sC[slot[0]][3][tid] * st[0].pb, st[0].f, 0);
 #pragma unroll
         for (int t = 0; t < T; ++t) {
             sQ[t][tid] = t ? zero : q0;
@@ -387,9 +430,11 @@ __global__ __launch_bounds__(kDesignPassThreads) __attribute__((amdgpu_waves_per
             qy = ld4(VY, c);
             qz = ld4(VZ, c);
         }
-        f4v ccx = coef_at(cl, 0, m + 1, a.cv0), ccy = coef_at(cl, 1, m + 1, a.cv0);
-        f4v ccz = coef_at(cl, 2, m + 1, a.cv0);
-        const f4v qc = coef_at(cl, 3, m + 2, a.cp0);
+        f4v qc[4];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) qc[q] = coef_at(cl, q, m + 1, a.cv0);
+        qc[3] = coef_at(cl, 3, m + 2, a.cp0);
+        dxn = uni(a.dec[0], min(m + 2, nx - 1));
         // ---- y and z faces of every stage's plane
 #pragma unroll
         for (int t = 0; t < T; ++t) {
@@ -408,31 +453,32 @@ __global__ __launch_bounds__(kDesignPassThreads) __attribute__((amdgpu_waves_per
             }
             S.vy = wy;
             S.vz = wz;
-            sY[t][tid] = S.cy * wy;
-            sZ[t][tid] = S.cz.w * wz.w;
+            sY[t][tid] = sC[slot[t]][1][tid] * wy;
+            sZ[t][tid] = sC[slot[t]][2][tid].w * wz.w;
         }
         lds_barrier();
         // ---- x faces and pressures, stage by stage
         f4v cpn = pn, cx = qx, cy = qy, cz = qz, ccp = cpl;
         uint32_t cf = fn;
         f4v q = sQ[0][tid];
+        f4v pbs[T], ws[T - 1][3];  // what the gradient needs of the stages' planes
 #pragma unroll
         for (int t = 0; t < T; ++t) {
             AdjointStage& S = st[t];
             const int i = m - t;
             const f4v yo = sY[t][tid], yb = sY[t][w.id];
             const float zb = sZ[t][w.il];
-            const float dx = uni(a.dec[0], min(max(i, 0), nx - 1));
-            const f4v pbn = pb_of(cpn, i + 1, t);
+            const float dx = dxs[t + 1];
+            const f4v pbn = pb_of(cpn, i + 1, t, dxs[t]);
             const f4v qn = keep(ccp * pbn, cf, 0);
             f4v wx = dx * S.vx + q;
             f4v acc = keep(S.pb, S.f, 0), cwx = zero;
             if (i < nx - 1) {
                 wx = keep(wx - qn, S.f, 1);
-                cwx = S.cx * wx;
+                cwx = sC[slot[t]][0][tid] * wx;
                 acc -= cwx;
             }
-            const f4v zo = S.cz * S.vz;
+            const f4v zo = sC[slot[t]][2][tid] * S.vz;
             const f4v zl = {zb, zo.x, zo.y, zo.z};
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -446,31 +492,17 @@ __global__ __launch_bounds__(kDesignPassThreads) __attribute__((amdgpu_waves_per
             acc.y += zl.y;
             acc.z += zl.z;
             acc.w += zl.w;
-            const int wi = i - a.lo[0] + 1;
-            if (box_j && i >= w.i0 && i < w.i1 && wi >= 0 && wi <= bx) {
-                if (wi > 0 && wj > 0) {
-                    GMEM float* row = gmem(a.pass_pb) + t * dbox_cells(a) +
-                                      (static_cast<uint32_t>((wi - 1) * by + wj - 1) * bz);
-                    st_range<false>(row, w.k, a.lo[2], bz, S.pb);
-                }
-                if (t < T - 1) {
-                    GMEM float* row = gmem(a.pass_w) + 3 * t * wall_cells(a) +
-                                      (static_cast<uint32_t>(wi * (by + 1) + wj) * (bz + 1));
-                    st_range<false>(row, w.k, a.lo[2] - 1, bz + 1, wx);
-                    st_range<false>(row + wall_cells(a), w.k, a.lo[2] - 1, bz + 1, S.vy);
-                    st_range<false>(row + 2 * wall_cells(a), w.k, a.lo[2] - 1, bz + 1, S.vz);
-                }
-            }
-            if (t == T - 1 && w.out && i >= w.i0) {
-                const uint32_t c = at(i);
-                st_lane<NTS>(gmem(a.f[src ^ 1][0]), c, acc, w.nv);
-                st_lane<NTS>(gmem(a.f[src ^ 1][1]), c, wx, w.nv);
-                st_lane<NTS>(gmem(a.f[src ^ 1][2]), c, S.vy, w.nv);
-                st_lane<NTS>(gmem(a.f[src ^ 1][3]), c, S.vz, w.nv);
+            pbs[t] = S.pb;
+            if (t < T - 1) {
+                ws[t][0] = wx;
+                ws[t][1] = S.vy;
+                ws[t][2] = S.vz;
             }
             // this stage's next plane: what came in (loads, or the stage before)
             const AdjointStage old = S;
-            S = AdjointStage{cx, cy, cz, cwx, pbn, ccx, ccy, ccz, ccp, cf};
+            S = AdjointStage{cx, cy, cz, cwx, pbn, cf};
+            // the next stage's plane ahead is this one's own
+            if (t + 1 < T) ccp = sC[slot[t]][3][tid];
             if (t + 1 < T) q = sQ[t + 1][tid];  // read before the next stage's q is posted
             sQ[t][tid] = qn;
             sX[t][tid] = qn.x;
@@ -478,15 +510,45 @@ __global__ __launch_bounds__(kDesignPassThreads) __attribute__((amdgpu_waves_per
             cx = wx;
             cy = old.vy;
             cz = old.vz;
-            ccx = old.cx;
-            ccy = old.cy;
-            ccz = old.cz;
-            ccp = old.cp;
             cf = old.f;
         }
         pn = qp;
         fn = qf;
-        cpl = qc;
+        // every store of the plane comes after the wait for the next one's loads
+        __builtin_amdgcn_s_waitcnt(kWaitLoads);
+        {
+            const int i = m - (T - 1);
+            if (w.out && i >= w.i0) {
+                const uint32_t c = at(i);
+                st_lane<NTS>(gmem(a.f[src ^ 1][0]), c, cpn, w.nv);
+                st_lane<NTS>(gmem(a.f[src ^ 1][1]), c, cx, w.nv);
+                st_lane<NTS>(gmem(a.f[src ^ 1][2]), c, cy, w.nv);
+                st_lane<NTS>(gmem(a.f[src ^ 1][3]), c, cz, w.nv);
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            const int i = m - t, wi = i - a.lo[0] + 1;
+            if (i < w.i0 || i >= w.i1 || wi < 0 || wi > bx) continue;  // uniform
+            if (wi > 0) st_box<false>(gmem(a.pass_pb) + (t * dbox_cells(a) + (wi - 1) * b_plane), pl, pbs[t]);
+            if (t < T - 1)
+#pragma unroll
+                for (int x = 0; x < 3; ++x)
+                    st_box<false>(gmem(a.pass_w) + ((3 * t + x) * coef_cells(a) + wi * w_plane), wl, ws[t][x]);
+        }
+        // The slot of the plane that left the last stage takes the next plane's:
+        // its cell coefficient is the one read a plane ahead.
+        const int free_slot = slot[T - 1];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) sC[free_slot][q][tid] = qc[q];
+        sC[free_slot][3][tid] = cpl;
+        cpl = qc[3];
+#pragma unroll
+        for (int t = T - 1; t > 0; --t) slot[t] = slot[t - 1];
+        slot[0] = free_slot;
+#pragma unroll
+        for (int t = T; t > 0; --t) dxs[t] = dxs[t - 1];
+        dxs[0] = dxn;
     }
 }
 
@@ -502,10 +564,11 @@ __global__ __launch_bounds__(256) void k_design_grad3(const DesignArgs a, int64_
     const uint32_t sx = static_cast<uint32_t>(a.ny) * static_cast<uint32_t>(nz);
     const uint32_t c = cix(a.lo[0] + bi, a.lo[1] + bj, a.lo[2] + bk, a.ny, nz);
     GMEM f4v* __restrict__ ACC = gm(a.acc);
-    const int ey = by + 2, ez = bz + 2;
-    const uint32_t e = static_cast<uint32_t>(((bi + 1) * ey + (bj + 1)) * ez + (bk + 1));
-    const uint32_t wy = static_cast<uint32_t>(by + 1), wz = static_cast<uint32_t>(bz + 1);
-    const uint32_t cw = ((bi + 1) * wy + (bj + 1)) * wz + (bk + 1);
+    const int ey = by + 2, ez = a.p_nk, k = a.lo[2] + bk;
+    const uint32_t e = static_cast<uint32_t>(((bi + 1) * ey + (bj + 1)) * ez + (k - a.p_k0));
+    const uint32_t d = static_cast<uint32_t>((bi * by + bj) * a.d_nk + (k - a.d_k0));
+    const uint32_t wy = static_cast<uint32_t>(by + 1), wz = static_cast<uint32_t>(coef_nk(a));
+    const uint32_t cw = ((bi + 1) * wy + (bj + 1)) * wz + static_cast<uint32_t>(k - coef_k0(a));
     const GMEM float* __restrict__ EX = gm(a.face_e);
     const GMEM float* __restrict__ EY = EX + face_count(bx, by, bz, 0);
     const GMEM float* __restrict__ EZ = EY + face_count(bx, by, bz, 1);
@@ -522,7 +585,7 @@ __global__ __launch_bounds__(256) void k_design_grad3(const DesignArgs a, int64_
         const int64_t m = n - q;
         // the last step's velocities are in the fields, the others' beside them
         const bool last = q == kPassSteps - 1;
-        const int64_t wc = wall_cells(a);
+        const int64_t wc = coef_cells(a);
         const GMEM float* __restrict__ WX = gm(last ? a.f[m & 1][1] : a.pass_w + 3 * q * wc);
         const GMEM float* __restrict__ WY = gm(last ? a.f[m & 1][2] : a.pass_w + (3 * q + 1) * wc);
         const GMEM float* __restrict__ WZ = gm(last ? a.f[m & 1][3] : a.pass_w + (3 * q + 2) * wc);
@@ -533,8 +596,8 @@ __global__ __launch_bounds__(256) void k_design_grad3(const DesignArgs a, int64_
                     hzp = ldo(hp, e + 1u);
         const float hxm = ldo(hp, e - static_cast<uint32_t>(ey * ez)), hym = ldo(hp, e - static_cast<uint32_t>(ez)),
                     hzm = ldo(hp, e - 1u);
-        const float pb = ldo(gm(a.pass_pb + q * dbox_cells(a)), b);
-        const float dv = ldo(gm(a.hist_div + (m - a.hist0) * dbox_cells(a)), b);
+        const float pb = ldo(gm(a.pass_pb + q * dbox_cells(a)), d);
+        const float dv = ldo(gm(a.hist_div + (m - a.hist0) * dbox_cells(a)), d);
         float gr = 0.f;
         gr += ldo(WX, o) * (hxp - hpc) * exp_;
         gr += ldo(WY, o) * (hyp - hpc) * eyp;
