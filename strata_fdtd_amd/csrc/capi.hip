@@ -563,8 +563,13 @@ int fdtd_ctx_set_ade(fdtd_ctx* c, int n_pole, const int32_t* mat_id, const int32
         if (target[q] != 0 && target[q] != 1) return fail(-2, "pole %d: target %d", q, target[q]);
         if (lorentz[q] != 0 && lorentz[q] != 1) return fail(-2, "pole %d: kind %d", q, lorentz[q]);
         if (lorentz[q] && !Jprev) return fail(-2, "Lorentz pole without a history array");
-        poles[q] = AdePole{mat_id[q], target[q], lorentz[q], 0, pa[q], pb[q], pd[q], corr[q]};
+        poles[q] = AdePole{mat_id[q], target[q], lorentz[q], q, pa[q], pb[q], pd[q], corr[q]};
     }
+    // Debye poles come before the Lorentz ones of a face's corrections and of a
+    // cell's (ade.cpp:240-401)
+    std::stable_sort(poles.begin(), poles.end(), [](const AdePole& x, const AdePole& y) {
+        return x.target != y.target ? x.target < y.target : x.lorentz < y.lorentz;
+    });
     a.material = material;
     a.J = J;
     a.Jprev = Jprev;
@@ -614,7 +619,9 @@ int fdtd_ctx_set_ade(fdtd_ctx* c, int n_pole, const int32_t* mat_id, const int32
         if (floats > 0 && reserve(c->patch_buf, sizeof(float) * static_cast<size_t>(floats)) != 0) (void)hipGetLastError();
         else if (floats > 0) {
             float* base = static_cast<float*>(c->patch_buf.p);
-            c->patch = PatchArgs{{base + off[0], base + off[1]}, base + off[2]};
+            const bool density = std::any_of(poles.begin(), poles.end(),
+                                             [](const AdePole& q) { return q.target == 0 && q.lorentz; });
+            c->patch = PatchArgs{{base + off[0], base + off[1]}, base + off[2], density};
             c->have_patch = true;
         }
     }

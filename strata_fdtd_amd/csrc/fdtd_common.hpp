@@ -86,7 +86,7 @@ struct AdePole {
     int32_t mat;                    // material id 1..255
     int32_t target;                 // 0 density, 1 modulus
     int32_t lorentz;                // 0 Debye, 1 Lorentz
-    int32_t pad;
+    int32_t slot;                   // its index in J and Jprev (registration order)
     float a, b, d;                  // recurrence coefficients
     float corr;                     // correction coefficient
 };
@@ -173,7 +173,7 @@ struct FusedArgs {
 
     // ADE (materials with poles)
     int n_pole;
-    const AdePole* poles;           // device [n_pole], registration order
+    const AdePole* poles;           // device [n_pole]: by target, Debye first, then as registered
     const uint8_t* material;        // per cell
     int box_lo[3], box_hi[3];       // ADE box [lo, hi)
     float* J;                       // [n_pole][box cells]
@@ -205,6 +205,7 @@ struct PassTile {
 struct PatchArgs {
     float* box[kPassSteps - 1];     // [4][cells] of the material box grown after steps 1 and 2
     float* J;                       // [n_pole][box cells]: the density poles' J of step 2
+    int density;                    // step 1's J is updated by a launch of its own (Lorentz)
 };
 
 // The boundary planes of a context (host side of a launch).

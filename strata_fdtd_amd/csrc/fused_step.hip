@@ -495,8 +495,8 @@ __device__ __forceinline__ void ade_density_part(const FusedArgs& a, int64_t fir
         for (int q = 0; q < a.n_pole; ++q) {
             const AdePole pl = pole_at(a.poles, q);
             if (pl.target != 0 || pl.mat != m) continue;
-            float* Jq = a.J + q * box_n + b;
-            *Jq = ade_recur(pl, *Jq, pl.lorentz ? a.Jprev + q * box_n + b : nullptr, pv);
+            float* Jq = a.J + pl.slot * box_n + b;
+            *Jq = ade_recur(pl, *Jq, pl.lorentz ? a.Jprev + pl.slot * box_n + b : nullptr, pv);
         }
     }
 }
@@ -508,12 +508,12 @@ __global__ void k_ade_density(const FusedArgs a) {
 
 // Full ADE update of every pole-material cell in the box, from the input set,
 // overwriting what the plain sweep wrote for those cells (see file comment).
-template <bool NU>
-__global__ void k_ade_fixup(const FusedArgs a) {
+template <bool NU, typename IX>
+__global__ __launch_bounds__(256) void k_ade_fixup(const FusedArgs a) {
     const int by = a.box_hi[1] - a.box_lo[1], bz = a.box_hi[2] - a.box_lo[2];
     const int64_t s = *a.step_ptr + a.koff;
     if (s >= a.step_limit) return;
-    const int par = static_cast<int>(s & 1);
+    const int par = __builtin_amdgcn_readfirstlane(static_cast<int>(s & 1));
     FieldView S{{}, 0, 0, 0, a.ny, a.nz};
     for (int g = 0; g < 4; ++g) S.f[g] = a.f[par][g];
     float* __restrict__ Po = a.f[par ^ 1][0];
@@ -521,6 +521,8 @@ __global__ void k_ade_fixup(const FusedArgs a) {
     float* __restrict__ VYo = a.f[par ^ 1][2];
     float* __restrict__ VZo = a.f[par ^ 1][3];
     const int64_t n_visit = a.ade_cells ? a.n_ade_cells : box_cells(a);
+    CellPoles cp;
+    fetch_poles(a, 0, cp);
     for (int64_t e = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; e < n_visit;
          e += static_cast<int64_t>(gridDim.x) * blockDim.x) {
         const int64_t b = a.ade_cells ? static_cast<int64_t>(a.ade_cells[e]) : e;
@@ -529,9 +531,10 @@ __global__ void k_ade_fixup(const FusedArgs a) {
         const int i = static_cast<int>(b / (static_cast<int64_t>(by) * bz)) + a.box_lo[0];
         const int64_t c = lin(i, j, k, a.ny, a.nz);
         const int m = a.material[c];
-        if (!has_pole(a, m)) continue;
+        if (!has_pole(a, cp, m)) continue;
         float o[4];
-        ade_cell<NU>(a, S, a.J, i, j, k, m, o);
+        ade_cell<NU, true, IX>(a, S, a.J, false, i, j, k, m, static_cast<IX>(b), cp, o);
+        if (a.n_pole > kFewPoles) fetch_poles(a, 0, cp);
         if (s < a.wave_len && (a.flags[c] & FDTD_FLAG_AIR)) o[0] = ade_sources(a, i, j, k, s, o[0]);
         Po[c] = o[0];
         VXo[c] = o[1];
@@ -786,8 +789,10 @@ hipError_t launch_fused(const FusedArgs& a_in, int rows, int stack, bool nu, boo
     if (e != hipSuccess) return e;
     if (ev_after && (e = hipEventRecord(ev_after, st)) != hipSuccess) return e;
     if (ade) {
-        if (nu) hipLaunchKernelGGL(k_ade_fixup<true>, dim3(box_blocks), dim3(256), 0, st, a);
-        else hipLaunchKernelGGL(k_ade_fixup<false>, dim3(box_blocks), dim3(256), 0, st, a);
+        const bool small = static_cast<int64_t>(a.nx) * a.ny * a.nz < kMaxCells32;
+        const auto run = [&](auto k) { hipLaunchKernelGGL(k, dim3(box_blocks), dim3(256), 0, st, a); };
+        if (small) nu ? run(k_ade_fixup<true, uint32_t>) : run(k_ade_fixup<false, uint32_t>);
+        else nu ? run(k_ade_fixup<true, int64_t>) : run(k_ade_fixup<false, int64_t>);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     if (bnd) {

@@ -489,8 +489,93 @@ __global__ __launch_bounds__(kBatchPassThreads) __attribute__((amdgpu_waves_per_
 // four cells into dense scratch, step 2 on it grown by three, step 3 on it grown by
 // two into the output, over what the pass wrote. The scratch stays in the caches
 // (the 512^3 enclosure's 81^3 box: 23 MB per step).
+//
+// A launch's first workgroups take the listed cells with poles, a thread each, the
+// others the rows of the grown box without those cells, four cells a lane. With a
+// thread for every cell of the box, those with poles scattered over its waves, a
+// step of the 81^3 box took 20.2 us and of a lined room's 86 x 102 x 130 (a fifth of
+// the cells with poles) 31; this way 16.4 and 23.4, the latter bound by the poles'
+// lanes, whose rows are pieces of a few cells: 1.7 times the L1 accesses.
+
+// The four cells from (i, j, k) of a step's input state as plain air, their sources
+// among them; nk of them lie in the row.
 template <bool NU>
-__global__ __launch_bounds__(256) void k_patch_step(const FusedArgs a, const PatchArgs pt, int t) {
+__device__ __forceinline__ void air_cells(const FusedArgs& a, const FieldView& S, int i, int j, int k, int nk,
+                                          int64_t s, f4v o[4]) {
+    const int nx = a.nx, ny = a.ny, nz = a.nz;
+    const uint32_t sy = S.nz, sx = static_cast<uint32_t>(S.ny) * S.nz;
+    const uint32_t gy = nz, gx = static_cast<uint32_t>(ny) * nz;
+    const uint32_t c = lidx<uint32_t>(i - S.oi, j - S.oj, k - S.ok, S.ny, S.nz), g = lidx<uint32_t>(i, j, k, ny, nz);
+    const GMEM float *P = gmem(S.f[0]), *VX = gmem(S.f[1]), *VY = gmem(S.f[2]), *VZ = gmem(S.f[3]);
+    const GMEM uint8_t* FL = gmem(a.flags);
+    const auto ldf = [&](uint32_t at) { return *reinterpret_cast<const GMEM u32u*>(at32(FL, at)); };
+    const f4v zero = {0.f, 0.f, 0.f, 0.f};
+    const bool ux = i + 1 < nx, uy = j + 1 < ny, dx = i > 0, dy = j > 0, dz = k > 0;
+    const f4v p = ld4(P, c), vx = ld4(VX, c), vy = ld4(VY, c), vz = ld4(VZ, c);
+    // where there is no neighbour its loads read the cell itself
+    const uint32_t cxl = dx ? c - sx : c, cyl = dy ? c - sy : c, czl = dz ? c - 1u : c;
+    const f4v pxh = ld4(P, ux ? c + sx : c), pxl = ld4(P, cxl), pyh = ld4(P, uy ? c + sy : c), pyl = ld4(P, cyl);
+    const f4v vxl = ld4(VX, cxl), vyl = ld4(VY, cyl);
+    const float pzh = ldx(P, nk == 4 && k + 4 < nz ? c + 4u : c), pzl = ldx(P, czl), vzl = ldx(VZ, czl);
+    const uint32_t f = ldf(g), fx = ldf(dx ? g - gx : g), fy = ldf(dy ? g - gy : g), fz = ldx(FL, dz ? g - 1u : g);
+    const auto tab = [&](const float* v, int at) { return ldx(gmem(v), static_cast<uint32_t>(at)); };
+    const float dxi = tab(a.dec[0], i), dyj = tab(a.dec[1], j);
+    float dzk[4], iz[4], cz[5];
+    const auto face = [&](int ax, int at, bool on) { return NU ? a.cv * (on ? tab(a.ifc[ax], at) : 1.f) : a.cv; };
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int ke = min(k + e, nz - 1);
+        dzk[e] = tab(a.dec[2], ke);
+        iz[e] = NU ? tab(a.icl[2], ke) : 1.f;
+        cz[e + 1] = face(2, ke, ke + 1 < nz);
+    }
+    cz[0] = face(2, k - 1, dz);
+    const float fxh = face(0, i, ux), fxl = face(0, i - 1, dx), fyh = face(1, j, uy), fyl = face(1, j - 1, dy);
+    const float ix = NU ? tab(a.icl[0], i) : 1.f, iy = NU ? tab(a.icl[1], j) : 1.f;
+    constexpr int bx = __builtin_ctz(FDTD_FLAG_OPEN_X), by = __builtin_ctz(FDTD_FLAG_OPEN_Y),
+                  bz = __builtin_ctz(FDTD_FLAG_OPEN_Z);
+    // the last face of an axis is neither updated nor masked
+    const f4v hx = ux ? keep(vx + fxh * (pxh - p), f, bx) : vx, lx = dx ? keep(vxl + fxl * (p - pxl), fx, bx) : zero;
+    const f4v hy = uy ? keep(vy + fyh * (pyh - p), f, by) : vy, ly = dy ? keep(vyl + fyl * (p - pyl), fy, by) : zero;
+    f4v hz, lz;
+    lz[0] = dz && (fz & FDTD_FLAG_OPEN_Z) ? vzl + cz[0] * (p[0] - pzl) : 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float up = e < 3 ? p[e < 3 ? e + 1 : 3] : pzh;
+        const float v = vz[e] + cz[e + 1] * (up - p[e]);
+        hz[e] = k + e + 1 < nz ? ((f >> (8 * e + bz)) & 1u ? v : 0.f) : vz[e];
+        if (e < 3) lz[e < 3 ? e + 1 : 3] = hz[e];
+    }
+    const f4v ax = hx - lx, ay = hy - ly, az = hz - lz;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        float q;
+        if (NU) q = p[e] + a.cp * (((ix * ax[e]) + (iy * ay[e])) + (iz[e] * az[e]));
+        else q = p[e] + a.cp * ((ax[e] + ay[e]) + az[e]);
+        const bool air = (f >> (8 * e)) & FDTD_FLAG_AIR;
+        if (!air) q = 0.f;
+        o[0][e] = ((q * dxi) * dyj) * dzk[e];
+        o[3][e] = hz[e] * dzk[e];
+    }
+    o[1] = hx * dxi;
+    o[2] = hy * dyj;
+    if (s < a.wave_len)
+        for (int q = 0; q < a.n_src; ++q) {
+            const int kind = a.src_kind[q], si = a.src_i[q], sj = a.src_j[q], sk = a.src_k[q];
+            // from k: the source's cells, all four or one
+            const int z = kind == 0 ? sk : si == 2 ? sj : -1;
+            const bool row = kind == 0 ? (si == i) & (sj == j) : (si == 2) | (sj == (si == 0 ? i : j));
+            if (!row) continue;
+            const double w = a.wave[q * a.wave_len + s];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if ((z < 0 || z == k + e) && ((f >> (8 * e)) & FDTD_FLAG_AIR))
+                    o[0][e] = static_cast<float>(static_cast<double>(o[0][e]) + w);
+        }
+}
+
+template <bool NU>
+__global__ __launch_bounds__(256) void k_patch_step(const FusedArgs a, const PatchArgs pt, int t, int pole_wgs) {
     const int64_t s = uni(a.step_ptr, 0) + a.koff + t;
     const int par = static_cast<int>((s - t) & 1);
     const int grow = 2 * kPassSteps - 2 - t;
@@ -515,57 +600,111 @@ __global__ __launch_bounds__(256) void k_patch_step(const FusedArgs a, const Pat
         const int64_t cells = static_cast<int64_t>(min(a.box_hi[0] + from, a.nx) - S.oi) * S.ny * S.nz;
         for (int g = 0; g < 4; ++g) S.f[g] = pt.box[t - 1] + g * cells;
     }
+    const int64_t cells = static_cast<int64_t>(n[0]) * n[1] * n[2];
+    const auto out = [&](int g) { return gmem(t == kPassSteps - 1 ? a.f[par ^ 1][g] : pt.box[t] + g * cells); };
+    const auto out_at = [&](int i, int j, int k) {
+        return t == kPassSteps - 1 ? lidx<uint32_t>(i, j, k, a.ny, a.nz)
+                                   : lidx<uint32_t>(i - lo[0], j - lo[1], k - lo[2], n[1], n[2]);
+    };
     // probes in the region (the pass recorded what it made of them)
     const GMEM int32_t* __restrict__ PIJK = gmem(a.probe_ijk);
     const int lane = threadIdx.x & (kWave - 1);
-    bool in = lane < a.n_sweep_probe;
-    if (in)
+    int at[3] = {kNowhere, kNowhere, kNowhere};
+    if (lane < a.n_sweep_probe)
 #pragma unroll
-        for (int x = 0; x < 3; ++x) {
-            const int v = PIJK[3 * lane + x];
-            in = in && v >= lo[x] && v < lo[x] + n[x];
+        for (int x = 0; x < 3; ++x) at[x] = PIJK[3 * lane + x];
+    int i, j, k, nk = 0;            // nk: cells from (i, j, k); bit e of own: cell k + e is this lane's
+    uint32_t own = 0;
+    f4v o[4];
+    if (static_cast<int>(blockIdx.x) < pole_wgs) {
+        const int64_t q = blockIdx.x * int64_t(256) + threadIdx.x;
+        const bool live = q < a.n_ade_cells;
+        const uint32_t b = static_cast<uint32_t>(a.ade_cells[live ? q : 0]);
+        const uint32_t by = a.box_hi[1] - a.box_lo[1], bz = a.box_hi[2] - a.box_lo[2], row = b / bz;
+        k = a.box_lo[2] + static_cast<int>(b - row * bz);
+        i = a.box_lo[0] + static_cast<int>(row / by);
+        j = a.box_lo[1] + static_cast<int>(row % by);
+        if (live) {
+            const uint32_t c = lidx<uint32_t>(i, j, k, a.ny, a.nz);
+            const int m = ldx(gmem(a.material), c);
+            const bool air = ldx(gmem(a.flags), c) & FDTD_FLAG_AIR;
+            const float p0 = ldx(gmem(S.f[0]), lidx<uint32_t>(i - S.oi, j - S.oj, k - S.ok, S.ny, S.nz));
+            const bool fresh = t == 0 && !pt.density;
+            const float* Jd = t == 1 ? pt.J : a.J;
+            float v[4];
+            CellPoles cp;
+            fetch_poles(a, 0, cp);
+            ade_cell<NU, true, uint32_t>(a, S, Jd, fresh, i, j, k, m, b, cp, v);
+            if (s < a.wave_len && air) v[0] = ade_sources(a, i, j, k, s, v[0]);
+            const uint32_t d = out_at(i, j, k);
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                stx(out(g), d, v[g]);
+                o[g][0] = v[g];
+            }
+            // density poles' J of the next step, from this step's pressure: from
+            // a.J into pt.J and back, since neighbours still read this step's
+            if (t < kPassSteps - 1)
+                ade_density_next(a, Jd, fresh, b, m, p0, v[0], cp, t == 1 ? a.J : pt.J);
+            nk = 1;
+            own = 1;
         }
-    const uint64_t probes = __builtin_amdgcn_ballot_w64(in);
-    const int64_t cells = static_cast<int64_t>(n[0]) * n[1] * n[2];
-    const uint32_t e = blockIdx.x * 256u + threadIdx.x;
-    if (e >= cells) return;
-    const uint32_t row = e / static_cast<uint32_t>(n[2]);
-    const int k = lo[2] + static_cast<int>(e - row * static_cast<uint32_t>(n[2]));
-    const int i = lo[0] + static_cast<int>(row / static_cast<uint32_t>(n[1]));
-    const int j = lo[1] + static_cast<int>(row % static_cast<uint32_t>(n[1]));
-    const int64_t c = lin(i, j, k, a.ny, a.nz);
-    int m = a.material[c];
-    if (!has_pole(a, m)) m = 0;
-    float o[4];
-    ade_cell<NU>(a, S, t == 1 ? pt.J : a.J, i, j, k, m, o);
-    if (s < a.wave_len && (a.flags[c] & FDTD_FLAG_AIR)) o[0] = ade_sources(a, i, j, k, s, o[0]);
-    if (t == kPassSteps - 1) {
-#pragma unroll
-        for (int g = 0; g < 4; ++g) a.f[par ^ 1][g][c] = o[g];
     } else {
+        const uint32_t lanes = static_cast<uint32_t>(n[2] + 3) >> 2;
+        const uint32_t e = (blockIdx.x - pole_wgs) * 256u + threadIdx.x, row = e / lanes;
+        const int in_row = 4 * static_cast<int>(e - row * lanes);
+        i = lo[0] + static_cast<int>(row / static_cast<uint32_t>(n[1]));
+        j = lo[1] + static_cast<int>(row % static_cast<uint32_t>(n[1]));
+        k = lo[2] + in_row;
+        if (row < static_cast<uint32_t>(n[0]) * static_cast<uint32_t>(n[1])) {
+            nk = min(4, n[2] - in_row);
+            own = (1u << nk) - 1u;
+            if (i >= a.box_lo[0] && i < a.box_hi[0] && j >= a.box_lo[1] && j < a.box_hi[1]) {
+                // the four cells' materials, those outside the box as 0; the array
+                // ends with the grid
+                const uint32_t c = lidx<uint32_t>(i, j, k, a.ny, a.nz);
+                const uint32_t last = static_cast<uint32_t>(a.nx) * a.ny * a.nz - 4u, at4 = min(c, last);
+                uint32_t m = *reinterpret_cast<const GMEM u32u*>(at32(gmem(a.material), at4)) >> (8u * (c - at4));
+                const int skip = min(max(a.box_lo[2] - k, 0), 4), stop = min(max(a.box_hi[2] - k, 0), nk);
+                m &= static_cast<uint32_t>((uint64_t(1) << (8 * stop)) - 1u) & static_cast<uint32_t>(~uint64_t(0) << (8 * skip));
+                if (m) {
+                    CellPoles cp;
+                    fetch_poles(a, 0, cp);
 #pragma unroll
-        for (int g = 0; g < 4; ++g) pt.box[t][g * cells + e] = o[g];
-        // density poles' J of the next step, from this step's pressure: from a.J
-        // into pt.J and back, since neighbours still read this step's
-        if (m) {
-            const int64_t box_n = box_cells(a), b = box_index(a, i, j, k);
-            const float* from = t == 1 ? pt.J : a.J;
-            float* to = t == 1 ? a.J : pt.J;
-            for (int q = 0; q < a.n_pole; ++q) {
-                const AdePole po = pole_at(a.poles, q);
-                if (po.target != 0 || po.mat != m) continue;
-                to[q * box_n + b] = ade_recur(po, from[q * box_n + b],
-                                              po.lorentz ? a.Jprev + q * box_n + b : nullptr, o[0]);
+                    for (int x = 0; x < 4; ++x) {
+                        const int mx = (m >> (8 * x)) & 255u;
+                        if (mx && has_pole(a, cp, mx)) own &= ~(1u << x);
+                    }
+                }
+            }
+            if (own) {
+                air_cells<NU>(a, S, i, j, k, nk, s, o);
+                const uint32_t d = out_at(i, j, k);
+                if (own == 15u) {
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) st4<false>(out(g), d, o[g]);
+                } else {
+#pragma unroll
+                    for (int g = 0; g < 4; ++g)
+#pragma unroll
+                        for (int x = 0; x < 4; ++x)
+                            if ((own >> x) & 1u) stx(out(g), d + static_cast<uint32_t>(x), o[g][x]);
+                }
             }
         }
     }
-    for (uint64_t pm = probes; pm; pm &= pm - 1) {
+    bool in = lane < a.n_sweep_probe;
+#pragma unroll
+    for (int x = 0; x < 3; ++x) in = in && at[x] >= lo[x] && at[x] < lo[x] + n[x];
+    for (uint64_t pm = __builtin_amdgcn_ballot_w64(in); pm; pm &= pm - 1) {
         const int q = __builtin_ctzll(pm);
-        if (uni(a.probe_ijk, 3 * q) == i && uni(a.probe_ijk, 3 * q + 1) == j && uni(a.probe_ijk, 3 * q + 2) == k &&
-            s < a.trace_len) {
-            a.trace[s * a.n_probe + q] = o[0];
-            if (!isfinite(o[0])) atomicOr(a.health, 1u);
-        }
+        const int x = uni(a.probe_ijk, 3 * q + 2) - k;
+        if (uni(a.probe_ijk, 3 * q) != i || uni(a.probe_ijk, 3 * q + 1) != j || x < 0 || x >= nk || s >= a.trace_len)
+            continue;
+        if (!((own >> x) & 1u)) continue;
+        const float v = x == 0 ? o[0][0] : x == 1 ? o[0][1] : x == 2 ? o[0][2] : o[0][3];
+        a.trace[s * a.n_probe + q] = v;
+        if (!isfinite(v)) atomicOr(a.health, 1u);
     }
 }
 
@@ -671,19 +810,22 @@ int64_t patch_floats(const FusedArgs& a, int64_t off[3]) {
     off[0] = 0;
     off[1] = 4 * first;
     off[2] = off[1] + 4 * second;
-    return off[2] + a.n_pole * grown_cells(a, 0);
+    return off[2] + a.n_pole * grown_cells(a, 0) + 4;  // a lane reads up to three cells past its row
 }
 
 hipError_t launch_density(const FusedArgs& a, hipStream_t st);
 
 // The cells a pass took wrongly (after it, on the same steps).
 hipError_t launch_patch(const FusedArgs& a, bool nu, const PatchArgs& pt, hipStream_t st) {
-    hipError_t e = launch_density(a, st);
+    hipError_t e = pt.density ? launch_density(a, st) : hipSuccess;
+    const int pole_wgs = static_cast<int>((a.n_ade_cells + 255) / 256);
     for (int t = 0; t < kPassSteps && e == hipSuccess; ++t) {
-        const int64_t cells = grown_cells(a, 2 * kPassSteps - 2 - t);
-        const dim3 grid(static_cast<unsigned>((cells + 255) / 256));
-        if (nu) hipLaunchKernelGGL(k_patch_step<true>, grid, dim3(256), 0, st, a, pt, t);
-        else hipLaunchKernelGGL(k_patch_step<false>, grid, dim3(256), 0, st, a, pt, t);
+        const int grow = 2 * kPassSteps - 2 - t;
+        const int64_t row = std::min(a.box_hi[2] + grow, a.nz) - std::max(a.box_lo[2] - grow, 0);
+        const int64_t lanes = grown_cells(a, grow) / row * ((row + 3) / 4);
+        const dim3 grid(static_cast<unsigned>(pole_wgs + (lanes + 255) / 256));
+        if (nu) hipLaunchKernelGGL(k_patch_step<true>, grid, dim3(256), 0, st, a, pt, t, pole_wgs);
+        else hipLaunchKernelGGL(k_patch_step<false>, grid, dim3(256), 0, st, a, pt, t, pole_wgs);
         e = hipGetLastError();
     }
     return e;

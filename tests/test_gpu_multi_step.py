@@ -141,3 +141,31 @@ def test_pass_ade_patch(oracle_lib, where, nonuniform):
     s.step_n(12, graph_chunk=6)
     s.step_n(n - 20)
     _compare(sc, s, n, st_o, tr_o)
+
+
+@pytest.mark.parametrize("nonuniform", [False, True])
+@pytest.mark.parametrize("poles", [("debye",), ("lorentz",), ("debye", "lorentz", "debye")])
+def test_pass_ade_pole_tables(oracle_lib, poles, nonuniform):
+    """Tables of up to four poles and of more, density Lorentz poles among them or
+    not: a thin layer along the grid's last rows, whose last cell is the grid's,
+    and single cells beside it, so that lanes hold cells with poles and without."""
+    print(f"[pass] poles {poles} nonuniform={nonuniform}", flush=True)
+    shape = (30, 27, 46)
+    sc = seeded_scenario(13, shape=shape, pml=3, nonuniform=nonuniform, geometry=False)
+    sc.material = np.zeros(shape, np.uint8)
+    sc.material[22:, 24:, 37:] = 1
+    sc.material[24, 21:23, 30:34] = 1
+    sc.material[26, 22, 31] = 2
+    sc.materials = {1: sum((POLES[q] for q in poles), [])}
+    if len(poles) > 1:
+        sc.materials[2] = POLES["debye"][:1]
+    else:
+        sc.material[sc.material == 2] = 0
+    sc.probes += [(29, 26, 45), (24, 22, 32), (25, 23, 36), (23, 20, 30)]
+    sc.sources.append(("point", (24, 22, 35), 9000.0))
+    sc.sources.append(("plane", 2, 33, 7000.0))
+    n = 17
+    st_o, tr_o = cpu.run(oracle_problem(sc, n), n)
+    s = make_solver(sc)
+    s.step_n(n)
+    _compare(sc, s, n, st_o, tr_o)
