@@ -90,9 +90,10 @@ int fdtd_ctx_set_sources(fdtd_ctx* ctx, int n, const int32_t* kind, const int64_
 
 /* Multi-step passes (three time steps per sweep over the fields, the same
  * arithmetic). mode 1 lets fdtd_step_n and fdtd_graph_run take them where the
- * solve allows it (no microphones or boundary planes, at most 64 probes, fewer
- * than 2^30 cells, every source a point or plane, materials with poles in at
- * most about a third of the grid; set it before fdtd_ctx_set_ade), mode 2 leaves
+ * solve allows it (no boundary planes, at most 64 probes, fewer than 2^30 cells,
+ * every source a point or plane, materials with poles in at most about a third
+ * of the grid, no microphone at the edge of their box; set it before
+ * fdtd_ctx_set_ade), mode 2 leaves
  * them to a batch the solve is in (a batch takes them when all its solves have
  * mode 1 or 2). Both promise that the field and flag buffers can be read 4 cells
  * past their end. 0 (the default): single steps. No counterpart in the

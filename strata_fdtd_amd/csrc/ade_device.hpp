@@ -252,4 +252,26 @@ __device__ __forceinline__ float ade_sources(const FusedArgs& a, int i, int j, i
     return ps;
 }
 
+// Gather g (0 p, 1..3 velocities) of microphone m: the weighted sum of its 8 corners
+// in the corner order of core/solver.py:962-1003 (acc = 0, then acc += w * f). The
+// reference sums in float32 when its weights are Python floats (numpy rounds the
+// weight to float32 and multiplies in float32) and in float64 when they are numpy
+// float64 scalars; mic_f64 selects which. at(flat grid index): the corner's value.
+template <typename At>
+__device__ __forceinline__ double mic_sum(const FusedArgs& a, int m, int g, At at) {
+    const int64_t row = static_cast<int64_t>(m) * 4 + g;
+    const int32_t* idx = a.mic_idx + row * 8;
+    const double* w = a.mic_w + row * 8;
+    if (a.mic_f64[row]) {
+        double acc = 0.0;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) acc = acc + w[c] * static_cast<double>(at(idx[c]));
+        return acc;
+    }
+    float acc = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) acc = acc + static_cast<float>(w[c]) * at(idx[c]);
+    return acc;
+}
+
 }  // namespace fdtd_amd

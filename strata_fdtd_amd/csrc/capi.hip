@@ -20,6 +20,8 @@ hipError_t launch_fused(const FusedArgs& a, int rows, int stack, bool nu, bool a
                         hipStream_t st, hipEvent_t ev_before, hipEvent_t ev_after, const BoundarySet* bnd);
 bool pick_pass_tile(int nx, int ny, int nz, int only_nt, double share, PassTile& best);
 hipError_t launch_pass(const FusedArgs& a, bool nu, const PassTile& m, hipStream_t st);
+bool mic_in_pass(const FusedArgs& a, const int32_t box[6]);
+hipError_t launch_pass_mics(const FusedArgs& a, bool nu, const PatchArgs& pt, const MicPass& mp, hipStream_t st);
 int64_t patch_floats(const FusedArgs& a, int64_t off[3]);
 hipError_t launch_patch(const FusedArgs& a, bool nu, const PatchArgs& pt, hipStream_t st);
 hipError_t launch_advance(int64_t* step, int n, hipStream_t st);
@@ -138,6 +140,8 @@ struct fdtd_ctx {
     bool have_patch = false;           // scratch for the poles' cells of a pass
     PatchArgs patch{};
     DevBuf patch_buf;
+    std::vector<int32_t> mic_boxes;    // [n_mic][6]: cells of each microphone, and on the device
+    DevBuf mic_box, mic_scratch;
 };
 
 extern "C" {
@@ -179,7 +183,7 @@ int fdtd_ctx_destroy(fdtd_ctx* c) {
     if (c->mic_w_dev) (void)hipFree(c->mic_w_dev);
     if (c->mic_f64_dev) (void)hipFree(c->mic_f64_dev);
     for (fdtd_ctx::DevBuf* b : {&c->ade_cells, &c->m_cell, &c->m_estart, &c->m_esrc, &c->m_efield, &c->m_eweight, &c->m_pstart,
-                                &c->m_pidx, &c->ade_poles, &c->probes, &c->patch_buf})
+                                &c->m_pidx, &c->ade_poles, &c->probes, &c->patch_buf, &c->mic_box, &c->mic_scratch})
         if (b->p) (void)hipFree(b->p);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
@@ -367,6 +371,32 @@ int fdtd_ctx_set_probes(fdtd_ctx* c, int n, const int64_t* idx, float* trace, in
     return 0;
 }
 
+static int reserve(fdtd_ctx::DevBuf& b, size_t bytes);
+
+// The cells of each microphone's gathers and room for a pass's first states there
+// (without room the solve steps one by one).
+static int set_mic_boxes(fdtd_ctx* c, int n, const int32_t* idx) {
+    c->mic_boxes.assign(6 * static_cast<size_t>(n), 0);
+    for (int m = 0; m < n; ++m) {
+        int32_t* b = c->mic_boxes.data() + 6 * static_cast<size_t>(m);
+        for (int q = 0; q < 32; ++q) {
+            const int f = idx[32 * static_cast<int64_t>(m) + q];
+            const int at[3] = {f / c->a.nz / c->a.ny, f / c->a.nz % c->a.ny, f % c->a.nz};
+            for (int x = 0; x < 3; ++x) {
+                b[x] = q ? std::min(b[x], at[x]) : at[x];
+                b[3 + x] = q ? std::max(b[3 + x], at[x] + 1) : at[x] + 1;
+            }
+        }
+    }
+    if (n == 0) return 0;
+    if (reserve(c->mic_scratch, sizeof(float) * kMicScratch * static_cast<size_t>(n)) != 0 ||
+        reserve(c->mic_box, sizeof(int32_t) * c->mic_boxes.size()) != 0) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    return upload(c->mic_box, c->mic_boxes.data(), sizeof(int32_t) * c->mic_boxes.size());
+}
+
 int fdtd_ctx_set_microphones(fdtd_ctx* c, int n, const int32_t* idx, const double* w, const int32_t* f64,
                              double* out, int64_t out_len) {
     if (!c) return fail(-1, "null context");
@@ -406,6 +436,7 @@ int fdtd_ctx_set_microphones(fdtd_ctx* c, int n, const int32_t* idx, const doubl
                            "hipMemcpy"))
             return rc;
     }
+    if (int rc = set_mic_boxes(c, n, idx)) return rc;
     c->a.n_mic = n;
     c->a.mic_idx = c->mic_idx_dev;
     c->a.mic_w = c->mic_w_dev;
@@ -661,9 +692,14 @@ static int ready(fdtd_ctx* c) {
 // step adds around the sweep has to be in the pass as well, or absent.
 static bool pass_allowed(fdtd_ctx* c) {
     const FusedArgs& a = c->a;
-    if (!c->multi_step || a.n_mic > 0 || c->bnd.n > 0 || a.n_probe > kSweepProbes) return false;
+    if (!c->multi_step || c->bnd.n > 0 || a.n_probe > kSweepProbes) return false;
     if (a.n_mcell > 0 && !c->have_pass_src) return false;
     if (a.n_pole > 0 && !c->have_patch) return false;
+    if (a.n_mic > 0) {
+        if (!c->mic_scratch.p || !c->mic_box.p) return false;
+        for (int m = 0; m < a.n_mic; ++m)
+            if (!mic_in_pass(a, c->mic_boxes.data() + 6 * static_cast<size_t>(m))) return false;
+    }
     if (!c->tile_known) {
         c->tile_known = true;
         c->tile_ok = pick_pass_tile(a.nx, a.ny, a.nz, 0, 1.0, c->tile);
@@ -683,6 +719,11 @@ static int enqueue_steps(fdtd_ctx* c, int n) {
             if (int rc = check(launch_pass(pa, c->nonuniform, c->tile, c->stream), "multi-step pass launch")) return rc;
             if (pa.n_pole > 0)
                 if (int rc = check(launch_patch(pa, c->nonuniform, c->patch, c->stream), "patch launch")) return rc;
+            if (pa.n_mic > 0) {
+                const MicPass mp{static_cast<const int32_t*>(c->mic_box.p), static_cast<float*>(c->mic_scratch.p)};
+                if (int rc = check(launch_pass_mics(pa, c->nonuniform, c->patch, mp, c->stream), "microphone launch"))
+                    return rc;
+            }
         }
     }
     for (; s < n; ++s) {

@@ -481,6 +481,10 @@ __global__ __launch_bounds__(kBatchPassThreads) __attribute__((amdgpu_waves_per_
     pass_workgroup<false, kBatchPassThreads, NTS>(ka, mt, s0 + koff, g - uni(offsets, lo));
 }
 
+// a microphone whose cells lie within this of the material box is in the boxes of
+// both of the patch's first steps (grown by 4 and 3 cells)
+constexpr int kPatchMic = kPassSteps;
+
 // ---- ADE patch ------------------------------------------------------------------
 // A pass takes every cell as plain air. Poles change the cells of their material
 // after one step and those up to t - 1 cells around them after t, so the pass is
@@ -708,6 +712,70 @@ __global__ __launch_bounds__(256) void k_patch_step(const FusedArgs a, const Pat
     }
 }
 
+// ---- microphones -----------------------------------------------------------------
+// The samples of a pass's steps, of which it stores the last one's state alone: one
+// workgroup per microphone steps the few cells around it from the pass's input
+// state (step 1 on its cells grown by one, step 2 on them) and gathers; a
+// microphone inside the patch's boxes gathers from those. Latency bounds it: two
+// dependent steps and a gather, 8.1 us a pass for two microphones (three launches of
+// k_mic_gather: 13.8). What it buys is the pass: a lined 131 x 157 x 203 room with
+// two microphones took 48 us a step one by one and takes 42.6.
+template <bool NU>
+__global__ __launch_bounds__(256) void k_mic_pass(const FusedArgs a, const PatchArgs pt, const MicPass mp) {
+    const int m = blockIdx.x, tid = threadIdx.x;
+    const int64_t s = uni(a.step_ptr, 0) + a.koff;
+    const int par = static_cast<int>(s & 1);
+    const int dim[3] = {a.nx, a.ny, a.nz};
+    int lo[3], hi[3];
+    bool patched = a.n_pole > 0;
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+        lo[x] = uni(mp.box, 6 * m + x);
+        hi[x] = uni(mp.box, 6 * m + 3 + x);
+        patched = patched && lo[x] >= a.box_lo[x] - kPatchMic && hi[x] <= a.box_hi[x] + kPatchMic;
+    }
+    float* scratch = mp.scratch + static_cast<int64_t>(m) * kMicScratch;
+    FieldView S{{}, 0, 0, 0, a.ny, a.nz};
+    for (int g = 0; g < 4; ++g) S.f[g] = a.f[par][g];
+    for (int t = 0; t < kPassSteps; ++t) {
+        // the box of the state after this step
+        const int grow = patched ? 2 * kPassSteps - 2 - t : kPassSteps - 2 - t;
+        int b0[3] = {}, n[3] = {dim[0], dim[1], dim[2]};
+        if (t < kPassSteps - 1)
+#pragma unroll
+            for (int x = 0; x < 3; ++x) {
+                b0[x] = max((patched ? a.box_lo[x] : lo[x]) - grow, 0);
+                n[x] = min((patched ? a.box_hi[x] : hi[x]) + grow, dim[x]) - b0[x];
+            }
+        const int64_t cells = static_cast<int64_t>(n[0]) * n[1] * n[2];
+        FieldView D{{}, b0[0], b0[1], b0[2], n[1], n[2]};
+        float* base = patched && t < kPassSteps - 1 ? pt.box[t] : scratch;
+        for (int g = 0; g < 4; ++g) D.f[g] = t == kPassSteps - 1 ? a.f[par ^ 1][g] : base + g * cells;
+        if (!patched && t < kPassSteps - 1) {
+            if (tid < cells) {
+                const int k = b0[2] + tid % n[2], r = tid / n[2];
+                const int j = b0[1] + r % n[1], i = b0[0] + r / n[1];
+                float o[4];
+                CellPoles cp;
+                ade_cell<NU, false, uint32_t>(a, S, nullptr, false, i, j, k, 0, 0u, cp, o);
+                if (s + t < a.wave_len && (a.flags[lin(i, j, k, a.ny, a.nz)] & FDTD_FLAG_AIR))
+                    o[0] = ade_sources(a, i, j, k, s + t, o[0]);
+                for (int g = 0; g < 4; ++g) base[g * cells + tid] = o[g];
+            }
+            __syncthreads();
+            scratch += 4 * cells;
+            S = D;
+        }
+        if (tid < 4 && s + t < a.mic_len) {
+            const float* F = tid == 0 ? D.f[0] : tid == 1 ? D.f[1] : tid == 2 ? D.f[2] : D.f[3];
+            a.mic_out[((s + t) * a.n_mic + m) * 4 + tid] = mic_sum(a, m, tid, [&](int c) {
+                const int row = c / a.nz;
+                return F[D.at(row / a.ny, row % a.ny, c % a.nz)];
+            });
+        }
+    }
+}
+
 // ---- host side -------------------------------------------------------------------
 constexpr int kCUs = 256;
 
@@ -811,6 +879,26 @@ int64_t patch_floats(const FusedArgs& a, int64_t off[3]) {
     off[1] = 4 * first;
     off[2] = off[1] + 4 * second;
     return off[2] + a.n_pole * grown_cells(a, 0) + 4;  // a lane reads up to three cells past its row
+}
+
+// Whether a pass can record a microphone with the cells [lo, hi): it lies in the
+// patch's boxes, or no cell it depends on has poles.
+bool mic_in_pass(const FusedArgs& a, const int32_t box[6]) {
+    bool inside = true, apart = false;
+    for (int x = 0; x < 3; ++x) {
+        const int lo = box[x], hi = box[3 + x];
+        if (hi - lo > kMicCells) return false;
+        inside = inside && lo >= a.box_lo[x] - kPatchMic && hi <= a.box_hi[x] + kPatchMic;
+        apart = apart || hi + kPassSteps - 1 <= a.box_lo[x] || lo - (kPassSteps - 1) >= a.box_hi[x];
+    }
+    return a.n_pole == 0 || inside || apart;
+}
+
+// The microphones' samples of a pass's steps (after it and its patch).
+hipError_t launch_pass_mics(const FusedArgs& a, bool nu, const PatchArgs& pt, const MicPass& mp, hipStream_t st) {
+    if (nu) hipLaunchKernelGGL(k_mic_pass<true>, dim3(a.n_mic), dim3(256), 0, st, a, pt, mp);
+    else hipLaunchKernelGGL(k_mic_pass<false>, dim3(a.n_mic), dim3(256), 0, st, a, pt, mp);
+    return hipGetLastError();
 }
 
 hipError_t launch_density(const FusedArgs& a, hipStream_t st);

@@ -169,3 +169,44 @@ def test_pass_ade_pole_tables(oracle_lib, poles, nonuniform):
     s = make_solver(sc)
     s.step_n(n)
     _compare(sc, s, n, st_o, tr_o)
+
+
+@pytest.mark.parametrize("nonuniform", [False, True])
+@pytest.mark.parametrize("poles", [None, "clear", "edge"])
+def test_pass_microphones(poles, nonuniform):
+    """Microphones recorded from passes against single steps: at the walls, next to
+    a source, and, with poles, in their material, in the boxes of the patch and
+    clear of them; one more at the edge of the boxes makes the solve step singly."""
+    print(f"[pass] microphones poles={poles} nonuniform={nonuniform}", flush=True)
+    shape, c = (36, 44, 60), (15, 20, 30)
+    sc = seeded_scenario(12, shape=shape, pml=4, nonuniform=nonuniform)
+    if poles:
+        g = np.indices(shape)
+        d2 = sum((g[x] - c[x]) ** 2 for x in range(3))
+        sc.material = np.where(d2 <= 20, 1, 0).astype(np.uint8)
+        sc.material[~sc.air] = 0
+        sc.materials = {1: POLES["debye"]}
+    # cells (with an offset inside them); box: [11, 20) x [16, 25) x [26, 35)
+    cells = [(0, 0, 0), (34, 42, 58), (5, 42, 30), (30, 9, 50), (15, 20, 30), (10, 20, 30), (15, 14, 36),
+             (26, 20, 30), (15, 28, 30)]
+    if poles == "edge":
+        cells.append((22, 20, 30))
+    solvers = []
+    for _ in range(2):
+        s = make_solver(sc)
+        for q, ijk in enumerate(cells):
+            pos = tuple((v + 0.3) * s.dx for v in ijk)
+            kw = dict(pattern="cardioid", direction=(1, 2, 3)) if q % 2 else {}
+            s.add_microphone(pos, name=f"m{q}", **kw)
+        solvers.append(s)
+    s, one = solvers
+    s.step_n(7)
+    s.step_n(12, graph_chunk=6)
+    s.step_n(10)
+    for _ in range(29):
+        one.step()
+    for q in range(len(cells)):
+        got, want = (np.asarray(v.microphones[f"m{q}"].get_waveform()) for v in solvers)
+        _same(got, want, f"microphone {cells[q]}")
+    for k in FIELDS:
+        _same(getattr(s, k), np.asarray(getattr(one, k)), k)
