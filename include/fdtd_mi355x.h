@@ -93,9 +93,9 @@ int fdtd_ctx_set_sources(fdtd_ctx* ctx, int n, const int32_t* kind, const int64_
  * solve allows it (no boundary planes, at most 64 probes, fewer than 2^30 cells,
  * every source a point or plane, materials with poles in at most about a third
  * of the grid, no microphone at the edge of their box; set it before
- * fdtd_ctx_set_ade), mode 2 leaves
- * them to a batch the solve is in (a batch takes them when all its solves have
- * mode 1 or 2). Both promise that the field and flag buffers can be read 4 cells
+ * fdtd_ctx_set_ade) and is not so small that single steps are faster, mode 3 on
+ * grids of any size, mode 2 leaves them to a batch the solve is in (a batch takes
+ * them when all its solves have a mode other than 0). All promise that the field and flag buffers can be read 4 cells
  * past their end. 0 (the default): single steps. No counterpart in the
  * reference, which makes one pass per step. */
 int fdtd_ctx_set_multi_step(fdtd_ctx* ctx, int mode);

@@ -131,7 +131,7 @@ struct fdtd_ctx {
         const double* wave = nullptr;
         int64_t wave_len = 0;
     } pass_src;
-    bool multi_step = false, padded = false, have_pass_src = false;
+    bool multi_step = false, every_pass = false, padded = false, have_pass_src = false;
     bool tile_known = false, tile_ok = false;
     PassTile tile{};
     // in a batch: the windows for a share of the chip of 1, 1/2, 1/4 .. 1/64
@@ -323,9 +323,10 @@ int fdtd_ctx_set_pass_sources(fdtd_ctx* c, int n, const int32_t* kind, const int
 
 int fdtd_ctx_set_multi_step(fdtd_ctx* c, int mode) {
     if (!c) return fail(-1, "null context");
-    if (mode < 0 || mode > 2) return fail(-2, "multi-step mode must be 0, 1 or 2");
+    if (mode < 0 || mode > 3) return fail(-2, "multi-step mode must be 0, 1, 2 or 3");
     drop_graph(c);
-    c->multi_step = mode == 1;
+    c->multi_step = mode == 1 || mode == 3;
+    c->every_pass = mode == 3;
     c->padded = mode != 0;
     return 0;
 }
@@ -688,6 +689,21 @@ static int ready(fdtd_ctx* c) {
     return 0;
 }
 
+// Whether a pass takes less than its steps one by one. It costs about a step's
+// launch and the latency of its planes whatever the grid, which three single
+// launches only exceed once there are cells to wait for: with a workgroup
+// marching several planes, 45 x 80 x 99 takes 7.0 us a step (single 6.5), 34 x 74 x
+// 173 7.2 (6.6), 64^3 6.1 (5.6), but 56 x 76 x 113 7.0 (7.8) and 100^3 7.7 (9.5); with
+// one plane each, 74 x 50 x 85 6.0 (6.3), 97 x 40 x 32 5.2 (5.5), and 40^3 5.2 (5.1).
+// Steps of several launches are left for a pass at any size (with a microphone
+// 40^3 takes 8.2 us for 9.0, with poles 11.3 for 12.4).
+static bool pass_pays(const fdtd_ctx* c) {
+    const FusedArgs& a = c->a;
+    if (c->every_pass || a.n_mic > 0 || a.n_pole > 0 || a.n_mcell > 0) return true;
+    const int64_t cells = static_cast<int64_t>(a.nx) * a.ny * a.nz;
+    return cells >= 450000 || (cells >= 100000 && c->tile.units == 1);
+}
+
 // Whether the context's steps can go several to a pass (k_multi_step): what a
 // step adds around the sweep has to be in the pass as well, or absent.
 static bool pass_allowed(fdtd_ctx* c) {
@@ -704,7 +720,7 @@ static bool pass_allowed(fdtd_ctx* c) {
         c->tile_known = true;
         c->tile_ok = pick_pass_tile(a.nx, a.ny, a.nz, 0, 1.0, c->tile);
     }
-    return c->tile_ok;
+    return c->tile_ok && pass_pays(c);
 }
 
 static int enqueue_steps(fdtd_ctx* c, int n) {

@@ -6,7 +6,8 @@ kernels keep the oracle's operations and their order, so the tolerance is 0."""
 import numpy as np
 import pytest
 
-from helpers import make_solver, oracle_problem, seeded_scenario
+import helpers
+from helpers import oracle_problem, seeded_scenario
 from oracle import cpu
 
 pytestmark = pytest.mark.gpu
@@ -16,6 +17,15 @@ FIELDS = ("p", "vx", "vy", "vz")
 # nz of every remainder by 4; one and several k segments; rows that fill their
 # windows exactly and by one more; fewer planes than a pass has steps
 SHAPES = [(26, 37, 70), (13, 41, 33), (9, 25, 130), (3, 20, 31), (12, 61, 1030), (31, 19, 12), (40, 26, 64)]
+
+
+def make_solver(sc, tiling=None):
+    """A solver that takes passes on these small grids too."""
+    from strata_fdtd_amd import _native
+    s = helpers.make_solver(sc, tiling=tiling)
+    if tiling is None:
+        _native.call("fdtd_ctx_set_multi_step", s._ctx, 3)
+    return s
 
 
 def _same(got, want, what):
