@@ -90,7 +90,8 @@ int fdtd_ctx_set_sources(fdtd_ctx* ctx, int n, const int32_t* kind, const int64_
 
 /* Multi-step passes (three time steps per sweep over the fields, the same
  * arithmetic). mode 1 lets fdtd_step_n and fdtd_graph_run take them where the
- * solve allows it (no boundary planes, at most 64 probes, fewer than 2^30 cells,
+ * solve allows it (no boundary planes, at most 1024 microphones and probes past the
+ * first 64, fewer than 2^30 cells,
  * every source a point or plane, materials with poles in at most about a third
  * of the grid, no microphone at the edge of their box; set it before
  * fdtd_ctx_set_ade) and is not so small that single steps are faster, mode 3 on

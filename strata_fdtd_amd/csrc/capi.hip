@@ -21,7 +21,8 @@ hipError_t launch_fused(const FusedArgs& a, int rows, int stack, bool nu, bool a
 bool pick_pass_tile(int nx, int ny, int nz, int only_nt, double share, PassTile& best);
 hipError_t launch_pass(const FusedArgs& a, bool nu, const PassTile& m, hipStream_t st);
 bool mic_in_pass(const FusedArgs& a, const int32_t box[6]);
-hipError_t launch_pass_mics(const FusedArgs& a, bool nu, const PatchArgs& pt, const MicPass& mp, hipStream_t st);
+hipError_t launch_pass_stations(const FusedArgs& a, bool nu, const PatchArgs& pt, const StationPass& mp,
+                                hipStream_t st);
 int64_t patch_floats(const FusedArgs& a, int64_t off[3]);
 hipError_t launch_patch(const FusedArgs& a, bool nu, const PatchArgs& pt, hipStream_t st);
 hipError_t launch_advance(int64_t* step, int n, hipStream_t st);
@@ -141,7 +142,7 @@ struct fdtd_ctx {
     PatchArgs patch{};
     DevBuf patch_buf;
     std::vector<int32_t> mic_boxes;    // [n_mic][6]: cells of each microphone, and on the device
-    DevBuf mic_box, mic_scratch;
+    DevBuf mic_box, station_scratch;
 };
 
 extern "C" {
@@ -183,7 +184,7 @@ int fdtd_ctx_destroy(fdtd_ctx* c) {
     if (c->mic_w_dev) (void)hipFree(c->mic_w_dev);
     if (c->mic_f64_dev) (void)hipFree(c->mic_f64_dev);
     for (fdtd_ctx::DevBuf* b : {&c->ade_cells, &c->m_cell, &c->m_estart, &c->m_esrc, &c->m_efield, &c->m_eweight, &c->m_pstart,
-                                &c->m_pidx, &c->ade_poles, &c->probes, &c->patch_buf, &c->mic_box, &c->mic_scratch})
+                                &c->m_pidx, &c->ade_poles, &c->probes, &c->patch_buf, &c->mic_box, &c->station_scratch})
         if (b->p) (void)hipFree(b->p);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
@@ -343,6 +344,19 @@ int fdtd_pass_tiling(int nx, int ny, int nz, int32_t* out) {
 
 static int upload(fdtd_ctx::DevBuf& b, const void* host, size_t bytes);
 
+static int reserve(fdtd_ctx::DevBuf& b, size_t bytes);
+
+// Microphones and probes that a pass leaves to k_station_pass.
+static int64_t stations(const fdtd_ctx* c, int n_mic) { return int64_t(n_mic) + std::max(0, c->a.n_probe - kSweepProbes); }
+
+// Room for a pass's first states around the stations; without it, and with more of
+// them, the solve steps one by one.
+static void reserve_stations(fdtd_ctx* c, int n_mic) {
+    const int64_t n = stations(c, n_mic);
+    if (n > 0 && n <= kMaxStations && reserve(c->station_scratch, sizeof(float) * kMicScratch * static_cast<size_t>(n)))
+        (void)hipGetLastError();
+}
+
 int fdtd_ctx_set_probes(fdtd_ctx* c, int n, const int64_t* idx, float* trace, int64_t trace_len) {
     if (!c) return fail(-1, "null context");
     if (!c->have_grid) return fail(-3, "set the grid before the probes");
@@ -369,13 +383,11 @@ int fdtd_ctx_set_probes(fdtd_ctx* c, int n, const int64_t* idx, float* trace, in
     c->a.probe_ijk = static_cast<const int32_t*>(c->probes.p);
     c->a.trace = trace;
     c->a.trace_len = n > 0 ? trace_len : 0;
+    reserve_stations(c, c->a.n_mic);
     return 0;
 }
 
-static int reserve(fdtd_ctx::DevBuf& b, size_t bytes);
-
-// The cells of each microphone's gathers and room for a pass's first states there
-// (without room the solve steps one by one).
+// The cells of each microphone's gathers.
 static int set_mic_boxes(fdtd_ctx* c, int n, const int32_t* idx) {
     c->mic_boxes.assign(6 * static_cast<size_t>(n), 0);
     for (int m = 0; m < n; ++m) {
@@ -389,9 +401,9 @@ static int set_mic_boxes(fdtd_ctx* c, int n, const int32_t* idx) {
             }
         }
     }
+    reserve_stations(c, n);
     if (n == 0) return 0;
-    if (reserve(c->mic_scratch, sizeof(float) * kMicScratch * static_cast<size_t>(n)) != 0 ||
-        reserve(c->mic_box, sizeof(int32_t) * c->mic_boxes.size()) != 0) {
+    if (reserve(c->mic_box, sizeof(int32_t) * c->mic_boxes.size()) != 0) {
         (void)hipGetLastError();
         return 0;
     }
@@ -699,7 +711,7 @@ static int ready(fdtd_ctx* c) {
 // 40^3 takes 8.2 us for 9.0, with poles 11.3 for 12.4).
 static bool pass_pays(const fdtd_ctx* c) {
     const FusedArgs& a = c->a;
-    if (c->every_pass || a.n_mic > 0 || a.n_pole > 0 || a.n_mcell > 0) return true;
+    if (c->every_pass || stations(c, a.n_mic) > 0 || a.n_pole > 0 || a.n_mcell > 0) return true;
     const int64_t cells = static_cast<int64_t>(a.nx) * a.ny * a.nz;
     return cells >= 450000 || (cells >= 100000 && c->tile.units == 1);
 }
@@ -708,11 +720,13 @@ static bool pass_pays(const fdtd_ctx* c) {
 // step adds around the sweep has to be in the pass as well, or absent.
 static bool pass_allowed(fdtd_ctx* c) {
     const FusedArgs& a = c->a;
-    if (!c->multi_step || c->bnd.n > 0 || a.n_probe > kSweepProbes) return false;
+    if (!c->multi_step || c->bnd.n > 0) return false;
     if (a.n_mcell > 0 && !c->have_pass_src) return false;
     if (a.n_pole > 0 && !c->have_patch) return false;
+    const int64_t n = stations(c, a.n_mic);
+    if (n > kMaxStations || c->station_scratch.bytes < sizeof(float) * kMicScratch * static_cast<size_t>(n)) return false;
     if (a.n_mic > 0) {
-        if (!c->mic_scratch.p || !c->mic_box.p) return false;
+        if (!c->mic_box.p) return false;
         for (int m = 0; m < a.n_mic; ++m)
             if (!mic_in_pass(a, c->mic_boxes.data() + 6 * static_cast<size_t>(m))) return false;
     }
@@ -735,9 +749,10 @@ static int enqueue_steps(fdtd_ctx* c, int n) {
             if (int rc = check(launch_pass(pa, c->nonuniform, c->tile, c->stream), "multi-step pass launch")) return rc;
             if (pa.n_pole > 0)
                 if (int rc = check(launch_patch(pa, c->nonuniform, c->patch, c->stream), "patch launch")) return rc;
-            if (pa.n_mic > 0) {
-                const MicPass mp{static_cast<const int32_t*>(c->mic_box.p), static_cast<float*>(c->mic_scratch.p)};
-                if (int rc = check(launch_pass_mics(pa, c->nonuniform, c->patch, mp, c->stream), "microphone launch"))
+            if (stations(c, pa.n_mic) > 0) {
+                const StationPass mp{static_cast<const int32_t*>(c->mic_box.p),
+                                     static_cast<float*>(c->station_scratch.p)};
+                if (int rc = check(launch_pass_stations(pa, c->nonuniform, c->patch, mp, c->stream), "station launch"))
                     return rc;
             }
         }

@@ -208,14 +208,16 @@ struct PatchArgs {
     int density;                    // step 1's J is updated by a launch of its own (Lorentz)
 };
 
-// What the microphones of a pass need: each one's cells [lo, hi) per axis (at most
-// kMicCells of them), and scratch for them after step 2 and, grown by one cell,
-// after step 1.
+// What the stations of a pass need, its microphones and the probes past the
+// sweep's: a microphone's cells [lo, hi) per axis (at most kMicCells of them; a
+// probe's is one), and scratch for them after step 2 and, grown by one cell, after
+// step 1.
+constexpr int kMaxStations = 1024;
 constexpr int kMicCells = 4;
 constexpr int kMicScratch = 4 * ((kMicCells + 2) * (kMicCells + 2) * (kMicCells + 2) + kMicCells * kMicCells * kMicCells);
-struct MicPass {
+struct StationPass {
     const int32_t* box;             // device [n_mic][6]
-    float* scratch;                 // device [n_mic][kMicScratch]
+    float* scratch;                 // device [stations][kMicScratch]
 };
 
 // The boundary planes of a context (host side of a launch).

@@ -712,26 +712,29 @@ __global__ __launch_bounds__(256) void k_patch_step(const FusedArgs a, const Pat
     }
 }
 
-// ---- microphones -----------------------------------------------------------------
-// The samples of a pass's steps, of which it stores the last one's state alone: one
-// workgroup per microphone steps the few cells around it from the pass's input
+// ---- stations --------------------------------------------------------------------
+// The samples of a pass's steps, of which it stores the last one's state alone, of
+// the microphones and of the probes past the 64 that the pass records itself: one
+// workgroup per station steps the few cells around it from the pass's input
 // state (step 1 on its cells grown by one, step 2 on them) and gathers; a
-// microphone inside the patch's boxes gathers from those. Latency bounds it: two
+// station inside the patch's boxes gathers from those. Latency bounds it: two
 // dependent steps and a gather, 8.1 us a pass for two microphones (three launches of
 // k_mic_gather: 13.8). What it buys is the pass: a lined 131 x 157 x 203 room with
 // two microphones took 48 us a step one by one and takes 42.6.
 template <bool NU>
-__global__ __launch_bounds__(256) void k_mic_pass(const FusedArgs a, const PatchArgs pt, const MicPass mp) {
+__global__ __launch_bounds__(256) void k_station_pass(const FusedArgs a, const PatchArgs pt, const StationPass mp) {
     const int m = blockIdx.x, tid = threadIdx.x;
     const int64_t s = uni(a.step_ptr, 0) + a.koff;
     const int par = static_cast<int>(s & 1);
     const int dim[3] = {a.nx, a.ny, a.nz};
+    const bool probe = m >= a.n_mic;
+    const int pq = a.n_sweep_probe + m - a.n_mic;
     int lo[3], hi[3];
     bool patched = a.n_pole > 0;
 #pragma unroll
     for (int x = 0; x < 3; ++x) {
-        lo[x] = uni(mp.box, 6 * m + x);
-        hi[x] = uni(mp.box, 6 * m + 3 + x);
+        lo[x] = probe ? uni(a.probe_ijk, 3 * pq + x) : uni(mp.box, 6 * m + x);
+        hi[x] = probe ? lo[x] + 1 : uni(mp.box, 6 * m + 3 + x);
         patched = patched && lo[x] >= a.box_lo[x] - kPatchMic && hi[x] <= a.box_hi[x] + kPatchMic;
     }
     float* scratch = mp.scratch + static_cast<int64_t>(m) * kMicScratch;
@@ -766,7 +769,16 @@ __global__ __launch_bounds__(256) void k_mic_pass(const FusedArgs a, const Patch
             scratch += 4 * cells;
             S = D;
         }
-        if (tid < 4 && s + t < a.mic_len) {
+        if (probe) {
+            if (tid > 0) continue;
+            if (s + t < a.trace_len) {
+                const float v = D.f[0][D.at(lo[0], lo[1], lo[2])];
+                a.trace[(s + t) * a.n_probe + pq] = v;
+                if (!isfinite(v)) atomicOr(a.health, 1u);
+            } else {
+                atomicOr(a.health, 2u);
+            }
+        } else if (tid < 4 && s + t < a.mic_len) {
             const float* F = tid == 0 ? D.f[0] : tid == 1 ? D.f[1] : tid == 2 ? D.f[2] : D.f[3];
             a.mic_out[((s + t) * a.n_mic + m) * 4 + tid] = mic_sum(a, m, tid, [&](int c) {
                 const int row = c / a.nz;
@@ -882,7 +894,7 @@ int64_t patch_floats(const FusedArgs& a, int64_t off[3]) {
 }
 
 // Whether a pass can record a microphone with the cells [lo, hi): it lies in the
-// patch's boxes, or no cell it depends on has poles.
+// patch's boxes, or no cell it depends on has poles. (A single cell does either.)
 bool mic_in_pass(const FusedArgs& a, const int32_t box[6]) {
     bool inside = true, apart = false;
     for (int x = 0; x < 3; ++x) {
@@ -894,10 +906,12 @@ bool mic_in_pass(const FusedArgs& a, const int32_t box[6]) {
     return a.n_pole == 0 || inside || apart;
 }
 
-// The microphones' samples of a pass's steps (after it and its patch).
-hipError_t launch_pass_mics(const FusedArgs& a, bool nu, const PatchArgs& pt, const MicPass& mp, hipStream_t st) {
-    if (nu) hipLaunchKernelGGL(k_mic_pass<true>, dim3(a.n_mic), dim3(256), 0, st, a, pt, mp);
-    else hipLaunchKernelGGL(k_mic_pass<false>, dim3(a.n_mic), dim3(256), 0, st, a, pt, mp);
+// The stations' samples of a pass's steps (after it and its patch).
+hipError_t launch_pass_stations(const FusedArgs& a, bool nu, const PatchArgs& pt, const StationPass& mp,
+                                hipStream_t st) {
+    const dim3 grid(a.n_mic + a.n_probe - a.n_sweep_probe);
+    if (nu) hipLaunchKernelGGL(k_station_pass<true>, grid, dim3(256), 0, st, a, pt, mp);
+    else hipLaunchKernelGGL(k_station_pass<false>, grid, dim3(256), 0, st, a, pt, mp);
     return hipGetLastError();
 }
 

@@ -220,3 +220,29 @@ def test_pass_microphones(poles, nonuniform):
         _same(got, want, f"microphone {cells[q]}")
     for k in FIELDS:
         _same(getattr(s, k), np.asarray(getattr(one, k)), k)
+
+
+@pytest.mark.parametrize("poles", [False, True])
+@pytest.mark.parametrize("count", [65, 200])
+def test_pass_probes_past_the_sweeps(oracle_lib, count, poles):
+    """More probes than a pass records itself: all over the grid, its corners and
+    the boxes around a material with poles among them."""
+    print(f"[pass] {count} probes poles={poles}", flush=True)
+    shape = (36, 44, 60)
+    sc = seeded_scenario(14, shape=shape, pml=4)
+    rng = np.random.default_rng(14)
+    if poles:
+        sc.material = np.zeros(shape, np.uint8)
+        sc.material[12:18, 18:24, 30:37] = 1
+        sc.material[~sc.air] = 0
+        sc.materials = {1: POLES["debye"]}
+    near = [(i, j, k) for i in (8, 11, 20, 21) for j in (15, 20, 27) for k in (33, 40)]
+    while len(sc.probes) < count - 26:
+        sc.probes.append(tuple(int(rng.integers(0, n)) for n in shape))
+    sc.probes += near + [(0, 0, 0), (35, 43, 59)]
+    sc.probes = sc.probes[-count:]
+    n = 20
+    st_o, tr_o = cpu.run(oracle_problem(sc, n), n)
+    s = make_solver(sc)
+    s.step_n(n)
+    _compare(sc, s, n, st_o, tr_o)
