@@ -93,7 +93,8 @@ def tune_shapes(requests, rows: int = 2, planes=(1, 2, 4, 8), steps: int = 20, d
     finds it. `rows` is the batched sweep's row count, so only the strip
     length along i is chosen per shape. Returns {shape: (tiling, ms per step)}.
 
-    Measured on the 64-request sweep (62 shapes, tuned in 0.2 s): the tuned
+    Measured on the 64-request sweep (62 shapes, tuned in 0.2 s), one step per
+    launch: the tuned
     single-solve strips (planes 2 for 30 shapes, 4 for 26, 8 for 5, 1 for 1)
     served the batch at 11.6 solves/s against 13.2 with the heuristic's
     shorter strips, which keep more waves in flight when many solves share
@@ -206,7 +207,7 @@ class SweepServer:
     captured once per chunk length and wave capacity and stays valid while
     the table of active solves changes between chunks. Enqueueing the kernels
     one by one instead (False) measured the same on the 64-request sweep
-    (13.95-14.00 against 13.88-13.99 solves/s)."""
+    (13.95-14.00 against 13.88-13.99 solves/s, one step per launch)."""
 
     CACHE_RESIDENT_CELLS = 6 << 20
     # batched rate (cell-updates per second) that converts a request's work

@@ -875,9 +875,9 @@ class FDTDSolver:
 
         graph_chunk = 0 (the default) enqueues the steps' kernels one by one;
         graph_chunk = m replays a captured hipGraph of m steps. Measured on
-        MI355X, the graph replay costs about 3.5 us more per step than the
-        same kernels enqueued back to back (100^3: 12.9 against 9.6 us per
-        step; 512^3: 901 against 863 us), so graphs are only worth it where
+        MI355X, the replay is no faster than the same passes enqueued back to
+        back (100^3: 7.7 against 7.3 us per step; 512^3: 320 against 320; of
+        single steps 12.9 against 9.6), so graphs are only worth it where
         the host cannot keep up with the launches."""
         if n <= 0:
             return
