@@ -92,8 +92,8 @@ int fdtd_ctx_set_sources(fdtd_ctx* ctx, int n, const int32_t* kind, const int64_
  * arithmetic). mode 1 lets fdtd_step_n and fdtd_graph_run take them where the
  * solve allows it (no boundary planes, at most 1024 microphones and probes past the
  * first 64, fewer than 2^30 cells,
- * every source a point or plane, materials with poles in at most about a third
- * of the grid, no microphone at the edge of their box; set it before
+ * every source a point or plane, room for a copy of the fields around materials
+ * with poles, no microphone at the edge of their box; set it before
  * fdtd_ctx_set_ade) and is not so small that single steps are faster, mode 3 on
  * grids of any size, mode 2 leaves them to a batch the solve is in (a batch takes
  * them when all its solves have a mode other than 0). All promise that the field and flag buffers can be read 4 cells

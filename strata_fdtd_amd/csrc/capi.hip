@@ -659,9 +659,14 @@ int fdtd_ctx_set_ade(fdtd_ctx* c, int n_pole, const int32_t* mat_id, const int32
     if (c->multi_step) {
         int64_t off[3];
         const int64_t floats = patch_floats(a, off);
-        // without room for the scratch the solve steps one by one
-        if (floats > 0 && reserve(c->patch_buf, sizeof(float) * static_cast<size_t>(floats)) != 0) (void)hipGetLastError();
-        else if (floats > 0) {
+        // without room for the scratch (up to as much as the fields) the solve steps
+        // one by one; a quarter of the free memory leaves others theirs
+        size_t have = 0, all = 0;
+        const size_t need = sizeof(float) * static_cast<size_t>(floats);
+        if (hipMemGetInfo(&have, &all) != hipSuccess || (need > c->patch_buf.bytes && need > have / 4) ||
+            reserve(c->patch_buf, need) != 0) {
+            (void)hipGetLastError();
+        } else {
             float* base = static_cast<float*>(c->patch_buf.p);
             const bool density = std::any_of(poles.begin(), poles.end(),
                                              [](const AdePole& q) { return q.target == 0 && q.lorentz; });

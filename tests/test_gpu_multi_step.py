@@ -124,18 +124,20 @@ POLES = {
 
 
 @pytest.mark.parametrize("nonuniform", [False, True])
-@pytest.mark.parametrize("where", ["inside", "corner"])
+@pytest.mark.parametrize("where", ["inside", "corner", "everywhere"])
 def test_pass_ade_patch(oracle_lib, where, nonuniform):
     """Materials with poles in a pass: a sphere of two materials away from the
-    walls, or in a corner (its grown boxes are cut by the grid), with the source
-    and probes in, next to and away from it, over passes and single steps."""
+    walls, or in a corner (its grown boxes are cut by the grid), or all of the
+    grid, with the source and probes in, next to and away from it, over passes
+    and single steps."""
     print(f"[pass] ade {where} nonuniform={nonuniform}", flush=True)
     shape = (36, 44, 60)
     sc = seeded_scenario(10, shape=shape, pml=4, nonuniform=nonuniform)
-    c = np.array((15, 20, 30) if where == "inside" else (0, 43, 57))
+    c = np.array((0, 43, 57) if where == "corner" else (15, 20, 30))
     g = np.indices(shape)
     d2 = sum((g[x] - c[x]) ** 2 for x in range(3))
-    sc.material = np.where(d2 <= 20, np.where(g[2] > c[2], 2, 1), 0).astype(np.uint8)
+    r2 = 10**6 if where == "everywhere" else 20
+    sc.material = np.where(d2 <= r2, np.where(g[2] > c[2], 2, 1), 0).astype(np.uint8)
     sc.material[~sc.air] = 0
     sc.materials = {1: POLES["debye"], 2: POLES["lorentz"] + POLES["debye"][:1]}
     near = [tuple(int(v) for v in np.clip(c + d, 0, np.array(shape) - 1))
