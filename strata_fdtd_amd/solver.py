@@ -632,9 +632,11 @@ class FDTDSolver:
         srcs = self._sources[:first]
         table = self._sources[first:]
         times = accumulated_times(self.dt, cap) if self._sources else None
+        waves = []
         if srcs:
             wave = np.stack([_fast_waveform(s, times, self.dt) for s in srcs]).astype(np.float64)
             self._wave = torch.from_numpy(np.ascontiguousarray(wave)).to(self._device)
+            waves.append(wave)
         else:
             self._wave = None
         if table:
@@ -643,6 +645,7 @@ class FDTDSolver:
             wave = np.stack([_fast_waveform(m.waveform if m.source_type == "membrane" else m, times, self.dt)
                              for m in table]).astype(np.float64)
             self._mwave = torch.from_numpy(np.ascontiguousarray(wave)).to(self._device)
+            waves.append(wave)
         else:
             self._mwave = None
         names = list(self._probes)
@@ -683,7 +686,7 @@ class FDTDSolver:
         _native.call("fdtd_ctx_set_probes", self._ctx, len(names), flat.ctypes.data,
                      _native.ptr(self._trace), cap)
         self._set_table_sources(table, names, cap)
-        self._set_pass_sources(table, cap)
+        self._set_pass_sources(table, waves, cap)
         self._cap = cap
         self._dirty_sources = False
 
@@ -703,16 +706,19 @@ class FDTDSolver:
         return (np.array(kind or [0], dtype=np.int32), np.array(a or [0], dtype=np.int64),
                 np.array(b or [0], dtype=np.int64))
 
-    def _set_pass_sources(self, table: list, cap: int) -> None:
+    def _set_pass_sources(self, table: list, waves: list, cap: int) -> None:
         """The whole source list for multi-step passes when some of it is in the
         per-cell tables (z planes): a pass adds up to SWEEP_SOURCES point and
-        plane sources of any axis itself, in list order."""
+        plane sources of any axis itself, in list order. Its waveforms are joined
+        on the host: the copy has ended when it returns, whatever stream is current,
+        where a device-side join would run on the current stream while the passes
+        read it on the solver's."""
         self._pwave = None
         if (not table or len(self._sources) > SWEEP_SOURCES
                 or any(s.source_type == "membrane" for s in self._sources)):
             return
         torch = _torch()
-        self._pwave = torch.cat([w for w in (self._wave, self._mwave) if w is not None]).contiguous()
+        self._pwave = torch.from_numpy(np.ascontiguousarray(np.concatenate(waves))).to(self._device)
         kind, a, b = self._source_arrays(self._sources)
         _native.call("fdtd_ctx_set_pass_sources", self._ctx, len(self._sources), kind.ctypes.data, a.ctypes.data,
                      b.ctypes.data, _native.ptr(self._pwave), cap)
