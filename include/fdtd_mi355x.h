@@ -223,6 +223,10 @@ int fdtd_step_n(fdtd_ctx* ctx, int n_steps);
  * the context and replay it `replays` times. */
 int fdtd_graph_run(fdtd_ctx* ctx, int n_steps, int replays);
 
+/* How the steps of fdtd_step_n and fdtd_graph_run have gone to the device so far:
+ * passes (of three steps each) and single steps. Host only. */
+int fdtd_ctx_step_counts(const fdtd_ctx* ctx, int64_t* passes, int64_t* singles);
+
 /* Average device time of the fused step kernel over the last timed window,
  * measured with HIP events on the context stream (milliseconds). */
 int fdtd_time_steps(fdtd_ctx* ctx, int n_steps, int use_graph, float* ms_total);
@@ -283,6 +287,9 @@ int fdtd_batch_set(fdtd_batch* b, fdtd_ctx* const* ctxs, const int64_t* step_lim
  * n launches, step k of each solve's chunk counted from its counter, then one
  * small launch that moves every counter by n, up to its limit. */
 int fdtd_batch_step_n(fdtd_batch* b, int n_steps, int use_graph);
+/* Launches of fdtd_batch_step_n so far: passes (three steps of every solve that has
+ * as many left) and single steps (with passes two a call, for the steps they leave). */
+int fdtd_batch_step_counts(const fdtd_batch* b, int64_t* passes, int64_t* singles);
 int fdtd_batch_info(fdtd_batch* b, int* n, int* total_waves);
 
 /* ---- per-voxel density / modulus and the adjoint (no reference counterpart) */
@@ -384,6 +391,8 @@ int fdtd_design_adjoint_passes(float* const* lam, const uint8_t* flags, const fl
                                int64_t steps_len, int64_t n_lo, int64_t n_hi, const float* hist_p,
                                const float* hist_div, int64_t hist0, int64_t hist_steps, float* acc, float* face_e,
                                float* pb_box, int planes, float* scratch, void* stream);
+/* Passes and single steps of the calling thread's last forward or adjoint call. */
+int fdtd_design_step_counts(int64_t* passes, int64_t* singles);
 
 /* ---- per-phase entry points (one kernel per reference function) --------- */
 /* All in place, on `stream`, float32, uniform unless noted. */

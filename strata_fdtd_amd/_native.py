@@ -71,6 +71,9 @@ _SIGS = {
                                  _i64, _i64, _i, _vp, _vp, _i64, _i64, _i, _vp]),
     "fdtd_design_adjoint": (_i, [_vp, _vp, _vp, _i, _i, _i, _f, _f, _vp, _vp, _vp, _i, _vp, _vp, _i64, _i64, _i64,
                                  _vp, _vp, _i64, _i64, _vp, _vp, _vp, _i, _vp]),
+    "fdtd_ctx_step_counts": (_i, [_vp, C.POINTER(_i64), C.POINTER(_i64)]),
+    "fdtd_batch_step_counts": (_i, [_vp, C.POINTER(_i64), C.POINTER(_i64)]),
+    "fdtd_design_step_counts": (_i, [C.POINTER(_i64), C.POINTER(_i64)]),
     "fdtd_design_pass_history": (_i, [_vp, _vp, C.POINTER(_i64), C.POINTER(_i64)]),
     "fdtd_design_pass_floats": (_i64, [_vp, _vp, _i]),
     "fdtd_design_forward_passes": (_i, [_vp, _vp, _vp, _i, _i, _i, _f, _f, _vp, _vp, _vp, _vp, _vp, _i, _vp, _vp,

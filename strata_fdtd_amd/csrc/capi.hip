@@ -118,6 +118,8 @@ struct fdtd_ctx {
         size_t bytes = 0;
     } m_cell, m_estart, m_esrc, m_efield, m_eweight, m_pstart, m_pidx, ade_cells, ade_poles, probes;
     int64_t* step_counter = nullptr;  // same as a.step_ptr, writable
+    // passes and single steps: enqueued so far, and of one replay of the graph
+    int64_t n_pass = 0, n_single = 0, graph_pass = 0, graph_single = 0;
     hipGraphExec_t graph = nullptr;
     int graph_steps = 0;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -760,6 +762,7 @@ static int enqueue_steps(fdtd_ctx* c, int n) {
                 if (int rc = check(launch_pass_stations(pa, c->nonuniform, c->patch, mp, c->stream), "station launch"))
                     return rc;
             }
+            ++c->n_pass;
         }
     }
     for (; s < n; ++s) {
@@ -768,6 +771,7 @@ static int enqueue_steps(fdtd_ctx* c, int n) {
                                         nullptr, nullptr, c->bnd.n ? &c->bnd : nullptr),
                            "fused step launch"))
             return rc;
+        ++c->n_single;
     }
     return check(launch_advance(c->step_counter, n, c->stream), "advance launch");
 }
@@ -800,8 +804,13 @@ int fdtd_graph_run(fdtd_ctx* c, int n_steps, int replays) {
         }
         hipStream_t saved = c->stream;
         c->stream = cap;
+        const int64_t n_pass = c->n_pass, n_single = c->n_single;
         int rc = enqueue_steps(c, n_steps);
         c->stream = saved;
+        c->graph_pass = c->n_pass - n_pass;
+        c->graph_single = c->n_single - n_single;
+        c->n_pass = n_pass;
+        c->n_single = n_single;
         hipError_t e = hipStreamEndCapture(cap, &gr);
         if (own) (void)hipStreamDestroy(cap);
         if (rc) { if (gr) (void)hipGraphDestroy(gr); return rc; }
@@ -811,8 +820,19 @@ int fdtd_graph_run(fdtd_ctx* c, int n_steps, int replays) {
         if (int r3 = check(e, "graph instantiate")) return r3;
         c->graph_steps = n_steps;
     }
-    for (int r = 0; r < replays; ++r)
+    for (int r = 0; r < replays; ++r) {
         if (int rc = check(hipGraphLaunch(c->graph, c->stream), "graph launch")) return rc;
+        c->n_pass += c->graph_pass;
+        c->n_single += c->graph_single;
+    }
+    return 0;
+}
+
+int fdtd_ctx_step_counts(const fdtd_ctx* c, int64_t* passes, int64_t* singles) {
+    if (!c) return fail(-1, "null context");
+    if (!passes || !singles) return fail(-2, "null output");
+    *passes = c->n_pass;
+    *singles = c->n_single;
     return 0;
 }
 
@@ -1134,6 +1154,7 @@ struct fdtd_batch {
     int graph_steps = 0;
     int graph_waves = 0;                // wave capacity of the captured grid
     int graph_wgs = 0;                  // workgroup capacity of its passes (0: none)
+    int64_t n_pass = 0, n_single = 0;   // launches so far
     bool graph_nts = true;
 };
 
@@ -1297,13 +1318,15 @@ int fdtd_batch_set(fdtd_batch* b, fdtd_ctx* const* ctxs, const int64_t* step_lim
     return 0;
 }
 
+static bool batch_passes(int cap_wgs, int n_steps) { return cap_wgs > 0 && n_steps >= kPassSteps; }
+
 // A chunk of n_steps steps of every solve: passes of kPassSteps steps where every
 // solve takes them (cap_wgs > 0), then the one or two steps they leave (to the
 // chunk's end or a solve's limit), or n_steps single steps; then one launch that
 // moves the counters. Steps are counted from the solves' counters.
 static int batch_enqueue(fdtd_batch* b, hipStream_t st, int n_steps, int cap_waves, int cap_wgs) {
     int singles = n_steps;
-    const bool passes = cap_wgs > 0 && n_steps >= kPassSteps;
+    const bool passes = batch_passes(cap_wgs, n_steps);
     if (passes) {
         for (int s = 0; s + kPassSteps <= n_steps; s += kPassSteps)
             if (int rc = check(launch_batch_pass(b->table_dev, b->tile_dev, b->meta_dev + b->cap + 2, b->meta_dev, cap_wgs,
@@ -1325,6 +1348,9 @@ int fdtd_batch_step_n(fdtd_batch* b, int n_steps, int use_graph) {
     if (n_steps < 0) return fail(-2, "negative step count");
     if (b->n == 0 || n_steps == 0) return 0;
     DeviceGuard g(b->device);
+    const bool passes = batch_passes(b->total_wgs, n_steps);
+    b->n_pass += passes ? n_steps / kPassSteps : 0;
+    b->n_single += passes ? kPassSteps - 1 : n_steps;
     if (!use_graph) return batch_enqueue(b, b->stream, n_steps, b->total_waves, b->total_wgs);
     if (!b->graph || b->graph_steps != n_steps || b->graph_waves < b->total_waves || b->graph_nts != b->nts ||
         b->graph_wgs < b->total_wgs || (b->graph_wgs > 0) != (b->total_wgs > 0)) {
@@ -1356,6 +1382,14 @@ int fdtd_batch_step_n(fdtd_batch* b, int n_steps, int use_graph) {
         b->graph_nts = b->nts;
     }
     return check(hipGraphLaunch(b->graph, b->stream), "graph launch");
+}
+
+int fdtd_batch_step_counts(const fdtd_batch* b, int64_t* passes, int64_t* singles) {
+    if (!b) return fail(-1, "null batch");
+    if (!passes || !singles) return fail(-2, "null output");
+    *passes = b->n_pass;
+    *singles = b->n_single;
+    return 0;
 }
 
 int fdtd_batch_info(fdtd_batch* b, int* n, int* total_waves) {

@@ -1087,6 +1087,9 @@ static bool pass_ready(DesignArgs& a, float* scratch, PassTile& tile, hipStream_
     return true;
 }
 
+// Passes and single steps of this thread's last forward or adjoint call.
+static thread_local int64_t design_passes = 0, design_singles = 0;
+
 }  // namespace fdtd_amd
 
 using namespace fdtd_amd;
@@ -1184,6 +1187,13 @@ int fdtd_design_pass_history(const int32_t* box_lo, const int32_t* box_hi, int64
     return 0;
 }
 
+int fdtd_design_step_counts(int64_t* passes, int64_t* singles) {
+    if (!passes || !singles) return -2;
+    *passes = design_passes;
+    *singles = design_singles;
+    return 0;
+}
+
 int fdtd_design_forward(float* const* fields, const uint8_t* flags, const float* const* dec, int nx, int ny, int nz,
                         float cv0, float cp0, const int32_t* box_lo, const int32_t* box_hi, const float* rk,
                         const int32_t* src_ijk, const double* wave, int n_probe, const int32_t* probe_ijk,
@@ -1218,12 +1228,13 @@ int fdtd_design_forward_passes(float* const* fields, const uint8_t* flags, const
     hipStream_t st = static_cast<hipStream_t>(stream);
     const bool nts = static_cast<int64_t>(nx) * ny * nz > kCacheResidentCells;
     int m = 0;
+    design_passes = design_singles = 0;
     PassTile tile{};
     if (scratch && n_steps >= kPassSteps && pass_ready(a, scratch, tile, st)) {
-        for (; n_steps - m >= kPassSteps; m += kPassSteps)
+        for (; n_steps - m >= kPassSteps; m += kPassSteps, ++design_passes)
             if (launch_design_forward_pass(a, tile, step0 + m, nts, st) != hipSuccess) return -5;
     }
-    for (; m < n_steps; ++m) {
+    for (; m < n_steps; ++m, ++design_singles) {
         if (nts)
             hipLaunchKernelGGL((k_design_forward<kDesignRows, true>), dim3(blocks), dim3(kBlock), 0, st, a, step0 + m);
         else
@@ -1279,12 +1290,13 @@ int fdtd_design_adjoint_passes(float* const* lam, const uint8_t* flags, const fl
         hipLaunchKernelGGL(k_design_faces, dim3(static_cast<unsigned>((faces + 255) / 256)), dim3(256), 0, st, a);
         if (hipGetLastError() != hipSuccess) return -5;
     }
+    design_passes = design_singles = 0;
     PassTile tile{};
     if (scratch && n_hi - n_lo >= kPassSteps && pass_ready(a, scratch, tile, st)) {
-        for (; n_hi - n_lo >= kPassSteps; n_hi -= kPassSteps)
+        for (; n_hi - n_lo >= kPassSteps; n_hi -= kPassSteps, ++design_passes)
             if (launch_design_adjoint_pass(a, tile, n_hi - 1, nts, st) != hipSuccess) return -5;
     }
-    for (int64_t n = n_hi - 1; n >= n_lo; --n) {
+    for (int64_t n = n_hi - 1; n >= n_lo; --n, ++design_singles) {
         if (nts)
             hipLaunchKernelGGL((k_design_adjoint<kDesignAdjRows, kDesignAdjBoxRows, true>), dim3(blocks), dim3(kBlock),
                                0, st, a, n);

@@ -1,0 +1,125 @@
+"""Which steps go to the device in passes of three and which one by one: both give
+the same bits, so the comparisons with the oracle cannot tell. Counts of passes and
+single steps for the solves, batches and design calls that take passes and for those
+that must not."""
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from helpers import make_solver, seeded_scenario
+
+pytestmark = pytest.mark.gpu
+
+STEPS = 3  # a pass
+POLES = [dict(kind="debye", target="density", tau=2e-5, dchi=0.5),
+         dict(kind="debye", target="modulus", tau=1e-5, dchi=0.3)]
+
+
+def _counts(name, *handle):
+    from strata_fdtd_amd import _native
+    p, s = C.c_int64(), C.c_int64()
+    _native.call(name, *handle, C.byref(p), C.byref(s))
+    return p.value, s.value
+
+
+def ctx_counts(s):
+    return _counts("fdtd_ctx_step_counts", s._ctx)
+
+
+def _every_pass(s):
+    from strata_fdtd_amd import _native
+    _native.call("fdtd_ctx_set_multi_step", s._ctx, 3)
+    return s
+
+
+@pytest.mark.parametrize("scene", ["plain", "nonuniform", "z plane", "poles", "microphone", "70 probes"])
+def test_solves_that_take_passes(scene):
+    sc = seeded_scenario(2, shape=(30, 34, 48), pml=3, nonuniform=scene == "nonuniform")
+    if scene == "z plane":
+        sc.sources.append(("plane", 2, 9, 7000.0))
+    if scene == "poles":
+        sc.material = np.zeros(sc.shape, np.uint8)
+        sc.material[10:14, 10:14, 10:14] = 1
+        sc.materials = {1: POLES}
+    if scene == "70 probes":
+        sc.probes = [(1 + q % 28, 2 + q % 30, q % 48) for q in range(70)]
+    s = _every_pass(make_solver(sc))
+    if scene == "microphone":
+        s.add_microphone(tuple(9.3 * s.dx for _ in range(3)), name="m")
+    assert ctx_counts(s) == (0, 0)
+    s.step_n(31)
+    assert ctx_counts(s) == (10, 1)
+    s.step()
+    s.step_n(2)
+    assert ctx_counts(s) == (10, 4)
+    s.step_n(24, graph_chunk=8)      # three replays of two passes and two steps
+    assert ctx_counts(s) == (16, 10)
+    s.step_n(24, graph_chunk=8)
+    assert ctx_counts(s) == (22, 16)
+
+
+def test_solves_that_step_one_by_one():
+    """A given launch shape; a microphone across the edge of the poles' boxes; a
+    membrane among the sources; boundary planes; a plain grid too small to gain."""
+    import strata_fdtd_amd as sfa
+    sc = seeded_scenario(2, shape=(36, 44, 60), pml=3)
+    tiled = make_solver(sc, tiling=(2, 2))
+    small = make_solver(sc)
+    bounded = _every_pass(make_solver(sc))
+    bounded.add_boundary(sfa.ABCFirstOrder())
+    sc.material = np.zeros(sc.shape, np.uint8)
+    sc.material[14:18, 18:22, 28:32] = 1
+    sc.materials = {1: POLES}
+    edge = _every_pass(make_solver(sc))
+    edge.add_microphone(tuple((v + 0.3) * edge.dx for v in (20, 20, 30)), name="m")
+    for s in (tiled, small, bounded, edge):
+        s.step_n(9)
+        assert ctx_counts(s) == (0, 9)
+    clear = _every_pass(make_solver(sc))
+    clear.add_microphone(tuple((v + 0.3) * clear.dx for v in (25, 20, 30)), name="m")
+    clear.step_n(9)
+    assert ctx_counts(clear) == (3, 0)
+
+
+def test_default_solves_take_passes_from_the_stated_sizes_on():
+    from strata_fdtd_amd import FDTDSolver
+    for shape, passes in (((100, 100, 100), True), ((45, 80, 99), False)):
+        s = FDTDSolver(shape=shape, resolution=1e-3)
+        s.step_n(7)
+        assert ctx_counts(s) == ((2, 1) if passes else (0, 7)), shape
+
+
+@pytest.mark.parametrize("use_graph", [False, True])
+def test_batches_take_passes_and_equal_one_step_kernels(use_graph):
+    """Served solves of 160^3, together beyond the cache, with a launch shape given
+    to the lone solves they are compared with, so that those go step by step."""
+    from strata_fdtd_amd.serving import SweepServer, build_solver, sweep_requests
+    reqs = sweep_requests(n=3, rate=1e6, seed=3, steps=(50, 80), dims=(160,))
+    srv = SweepServer(chunk=16, max_cells=None, policy="fifo", use_graph=use_graph)
+    stats = srv.serve(reqs, realtime=False)
+    chunks = stats.chunks
+    assert _counts("fdtd_batch_step_counts", srv._batch) == (chunks * 5, chunks * (STEPS - 1))
+    srv.close()
+    for res in stats.results:
+        r = next(x for x in reqs if x.rid == res.rid)
+        s = build_solver(r, tiling=(4, 2))
+        s.step_n(r.steps)
+        assert ctx_counts(s) == (0, r.steps)
+        for name, tr in s.get_probe_data().items():
+            assert np.array_equal(res.traces[name], tr)
+
+
+@pytest.mark.parametrize("history,steps", [("all", 31), ("checkpoint", 20)])
+def test_design_calls_take_passes(history, steps):
+    import torch
+    from strata_fdtd_amd import GaussianPulse
+    from strata_fdtd_amd.adjoint import DesignProblem, adjoint_gradients, forward_traces
+    pb = DesignProblem(shape=(24, 26, 30), pml_depth=2, source=GaussianPulse(position=(12, 12, 12), frequency=3e4),
+                       probes=[(13, 12, 12)], steps=steps, box_lo=(6, 6, 6), box_hi=(18, 18, 18), checkpoint=20)
+    rho = torch.full(pb.box_shape, pb.rho * 1.01, device="cuda")
+    tr, saved = forward_traces(pb, rho, None, keep_checkpoints=True, history=history)
+    assert _counts("fdtd_design_step_counts") == (steps // STEPS, steps % STEPS)
+    adjoint_gradients(saved, torch.ones_like(tr))
+    assert _counts("fdtd_design_step_counts") == (steps // STEPS, steps % STEPS)
