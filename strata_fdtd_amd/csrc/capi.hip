@@ -144,6 +144,7 @@ struct fdtd_ctx {
     PatchArgs patch{};
     DevBuf patch_buf;
     std::vector<int32_t> mic_boxes;    // [n_mic][6]: cells of each microphone, and on the device
+    bool probes_fit = false;           // the probes' cells are of this grid
     DevBuf mic_box, station_scratch;
 };
 
@@ -213,6 +214,14 @@ int fdtd_ctx_set_grid(fdtd_ctx* c, int nx, int ny, int nz, int nonuniform, float
     if (nonuniform && (!ifx || !ify || !ifz || !icx || !icy || !icz))
         return fail(-2, "nonuniform grid needs all six spacing tables");
     drop_graph(c);
+    // what passes keep of the microphones, probes and materials set so far is of the
+    // grid that they were set for: on another one the solve steps one by one until
+    // they are set again
+    if (nx != c->a.nx || ny != c->a.ny || nz != c->a.nz) {
+        c->mic_boxes.clear();
+        c->probes_fit = false;
+        c->have_patch = false;
+    }
     c->a.nx = nx; c->a.ny = ny; c->a.nz = nz;
     c->tile_known = false;
     std::fill(std::begin(c->batch_tile_known), std::end(c->batch_tile_known), false);
@@ -385,15 +394,18 @@ int fdtd_ctx_set_probes(fdtd_ctx* c, int n, const int64_t* idx, float* trace, in
     c->a.probe_ijk = static_cast<const int32_t*>(c->probes.p);
     c->a.trace = trace;
     c->a.trace_len = n > 0 ? trace_len : 0;
+    c->probes_fit = true;
     reserve_stations(c, c->a.n_mic);
     return 0;
 }
 
-// The cells of each microphone's gathers.
+// The cells of each microphone's gathers; without them on the device (a failed
+// call, another grid since) the solve steps one by one.
 static int set_mic_boxes(fdtd_ctx* c, int n, const int32_t* idx) {
-    c->mic_boxes.assign(6 * static_cast<size_t>(n), 0);
+    c->mic_boxes.clear();
+    std::vector<int32_t> boxes(6 * static_cast<size_t>(n), 0);
     for (int m = 0; m < n; ++m) {
-        int32_t* b = c->mic_boxes.data() + 6 * static_cast<size_t>(m);
+        int32_t* b = boxes.data() + 6 * static_cast<size_t>(m);
         for (int q = 0; q < 32; ++q) {
             const int f = idx[32 * static_cast<int64_t>(m) + q];
             const int at[3] = {f / c->a.nz / c->a.ny, f / c->a.nz % c->a.ny, f % c->a.nz};
@@ -405,11 +417,13 @@ static int set_mic_boxes(fdtd_ctx* c, int n, const int32_t* idx) {
     }
     reserve_stations(c, n);
     if (n == 0) return 0;
-    if (reserve(c->mic_box, sizeof(int32_t) * c->mic_boxes.size()) != 0) {
+    if (reserve(c->mic_box, sizeof(int32_t) * boxes.size()) != 0) {
         (void)hipGetLastError();
         return 0;
     }
-    return upload(c->mic_box, c->mic_boxes.data(), sizeof(int32_t) * c->mic_boxes.size());
+    if (int rc = upload(c->mic_box, boxes.data(), sizeof(int32_t) * boxes.size())) return rc;
+    c->mic_boxes = std::move(boxes);
+    return 0;
 }
 
 int fdtd_ctx_set_microphones(fdtd_ctx* c, int n, const int32_t* idx, const double* w, const int32_t* f64,
@@ -732,8 +746,9 @@ static bool pass_allowed(fdtd_ctx* c) {
     if (a.n_pole > 0 && !c->have_patch) return false;
     const int64_t n = stations(c, a.n_mic);
     if (n > kMaxStations || c->station_scratch.bytes < sizeof(float) * kMicScratch * static_cast<size_t>(n)) return false;
+    if (a.n_probe > kSweepProbes && !c->probes_fit) return false;
     if (a.n_mic > 0) {
-        if (!c->mic_box.p) return false;
+        if (!c->mic_box.p || c->mic_boxes.size() != 6 * static_cast<size_t>(a.n_mic)) return false;
         for (int m = 0; m < a.n_mic; ++m)
             if (!mic_in_pass(a, c->mic_boxes.data() + 6 * static_cast<size_t>(m))) return false;
     }

@@ -123,3 +123,45 @@ def test_design_calls_take_passes(history, steps):
     assert _counts("fdtd_design_step_counts") == (steps // STEPS, steps % STEPS)
     adjoint_gradients(saved, torch.ones_like(tr))
     assert _counts("fdtd_design_step_counts") == (steps // STEPS, steps % STEPS)
+
+
+@pytest.mark.parametrize("what", ["microphone", "70 probes", "poles"])
+def test_another_grid_ends_passes_until_their_tables_are_set_again(what):
+    """fdtd_ctx_set_grid with other sides: the cells that passes keep of the
+    microphones, probes and materials are of the old grid."""
+    import torch
+    from strata_fdtd_amd import _native
+    sc = seeded_scenario(2, shape=(32, 40, 48), pml=0, geometry=False)
+    if what == "70 probes":
+        sc.probes = [(1 + q % 28, 2 + q % 28, q % 30) for q in range(70)]
+    if what == "poles":
+        sc.material = np.zeros(sc.shape, np.uint8)
+        sc.material[4:10, 4:10, 4:10] = 1
+        sc.materials = {1: POLES}
+    s = _every_pass(make_solver(sc))
+    if what == "microphone":
+        s.add_microphone(tuple(9.3 * s.dx for _ in range(3)), name="m")
+    s._prepare(64)                    # the tables cover every step below
+    ones = torch.ones(48, device="cuda")
+    _native.call("fdtd_ctx_set_pml", s._ctx, *[_native.ptr(ones)] * 3)
+
+    def grid(nx, ny, nz):
+        s.synchronize()
+        _native.call("fdtd_ctx_set_grid", s._ctx, nx, ny, nz, 0, s._coeff_v, s._coeff_p, *[None] * 6)
+
+    def take(n):
+        before = ctx_counts(s)
+        _native.call("fdtd_step_n", s._ctx, n)
+        s.synchronize()
+        return tuple(b - a for a, b in zip(before, ctx_counts(s)))
+
+    assert take(9) == (3, 0)
+    grid(32, 40, 48)                  # the same sides
+    assert take(9) == (3, 0)
+    grid(40, 32, 48)                  # as many cells, other sides
+    assert take(9) == (0, 9)
+    grid(32, 40, 48)
+    assert take(9) == (0, 9)
+    s._dirty_sources = s._dirty_ade = True
+    s._prepare(64)
+    assert take(9) == (3, 0)
