@@ -94,8 +94,8 @@ int fdtd_ctx_set_sources(fdtd_ctx* ctx, int n, const int32_t* kind, const int64_
  * first 64, fewer than 2^30 cells,
  * every source a point or plane, room for a copy of the fields around materials
  * with poles, no microphone at the edge of their box; set it before
- * fdtd_ctx_set_ade) and is not so small that single steps are faster, mode 3 on
- * grids of any size, mode 2 leaves them to a batch the solve is in (a batch takes
+ * fdtd_ctx_set_ade) and single steps are not faster (small grids; pole materials
+ * with much of the grid between them), mode 3 wherever it can, mode 2 leaves them to a batch the solve is in (a batch takes
  * them when all its solves have a mode other than 0). All promise that the field and flag buffers can be read 4 cells
  * past their end. 0 (the default): single steps. No counterpart in the
  * reference, which makes one pass per step. */

@@ -23,6 +23,7 @@ hipError_t launch_pass(const FusedArgs& a, bool nu, const PassTile& m, hipStream
 bool mic_in_pass(const FusedArgs& a, const int32_t box[6]);
 hipError_t launch_pass_stations(const FusedArgs& a, bool nu, const PatchArgs& pt, const StationPass& mp,
                                 hipStream_t st);
+bool patch_pays(const FusedArgs& a);
 int64_t patch_floats(const FusedArgs& a, int64_t off[3]);
 hipError_t launch_patch(const FusedArgs& a, bool nu, const PatchArgs& pt, hipStream_t st);
 hipError_t launch_advance(int64_t* step, int n, hipStream_t st);
@@ -672,7 +673,7 @@ int fdtd_ctx_set_ade(fdtd_ctx* c, int n_pole, const int32_t* mat_id, const int32
     if (int rc = upload(c->ade_poles, poles.data(), sizeof(AdePole) * poles.size())) return rc;
     a.poles = static_cast<const AdePole*>(c->ade_poles.p);
     a.n_pole = n_pole;
-    if (c->multi_step) {
+    if (c->multi_step && (c->every_pass ? static_cast<int64_t>(a.nx) * a.ny * a.nz < kMaxCells32 : patch_pays(a))) {
         int64_t off[3];
         const int64_t floats = patch_floats(a, off);
         // without room for the scratch (up to as much as the fields) the solve steps
@@ -729,7 +730,8 @@ static int ready(fdtd_ctx* c) {
 // 173 7.2 (6.6), 64^3 6.1 (5.6), but 56 x 76 x 113 7.0 (7.8) and 100^3 7.7 (9.5); with
 // one plane each, 74 x 50 x 85 6.0 (6.3), 97 x 40 x 32 5.2 (5.5), and 40^3 5.2 (5.1).
 // Steps of several launches are left for a pass at any size (with a microphone
-// 40^3 takes 8.2 us for 9.0, with poles 11.3 for 12.4).
+// 40^3 takes 8.2 us for 9.0, with poles 11.3 for 12.4); with poles patch_pays has
+// decided when they were set.
 static bool pass_pays(const fdtd_ctx* c) {
     const FusedArgs& a = c->a;
     if (c->every_pass || stations(c, a.n_mic) > 0 || a.n_pole > 0 || a.n_mcell > 0) return true;

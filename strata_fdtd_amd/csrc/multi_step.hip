@@ -880,12 +880,30 @@ static int64_t grown_cells(const FusedArgs& a, int grow) {
     return n;
 }
 
+// Whether a pass and its patch take less than single steps with their fix-up. Cells
+// with poles cost about the same either way (a few percent less in the patch), so
+// what counts is the rest of the grown box, which the patch takes at the price of a
+// plain step's cells (4.8 us per million and step in grids of 2 million cells, 6.2 at
+// 4 million, 7.6 at 7, 7 beyond the cache), against what a pass saves on the whole
+// grid (2.7 us per million, beyond the cache 4; a launch or two where a step is
+// little more than those). Both ways were timed on 469 solves of 40^3 to 320^3 with
+// 1, 3 and 8 poles: pairs of small absorbers at opposite corners of a box of a tenth
+// of the grid up to all of it, full boxes, shells and scattered cells. Where this
+// takes passes none was more than 2% slower than single steps. Pairs at the corners
+// of 128^3: single 23.1 us a step, passes 27.6, and 18.9 in a box of a tenth; 192^3
+// 45.2, 81.2, 34.5; 260^3 176, 182, 75; 320^3 224, 321, 122. Full boxes, three
+// poles: 100^3 40, 31; 192^3 257, 178. Lines between what was measured: at 192^3 a
+// third of the grid is where a pair's two ways meet, at 160^3 and 320^3 a half.
+bool patch_pays(const FusedArgs& a) {
+    const int64_t cells = static_cast<int64_t>(a.nx) * a.ny * a.nz;
+    if (cells >= kMaxCells32) return false;  // no passes at all
+    const double share = cells > 5000000 && cells <= kCacheResidentCells ? 0.33 : 0.45;
+    const int64_t air = grown_cells(a, 2 * kPassSteps - 2) - a.n_ade_cells;
+    return static_cast<double>(air) <= 1e5 + share * static_cast<double>(cells);
+}
+
 // Scratch floats of the patch: the boxes of steps 1 and 2, then the density poles'
-// second J. A patch takes the box's cells faster than the sweep and k_ade_fixup
-// do, so a pass is worth it however much of the grid the box takes: a full box of
-// three-pole cells whose grown box is 59% of 100^3 took 26.6 us a step one by one and
-// takes 22.9, 63% of 192^3 168 and 120, 86% of 160^3 93 and 80, all of 64^3 16.1 and
-// 14.2.
+// second J.
 int64_t patch_floats(const FusedArgs& a, int64_t off[3]) {
     const int64_t first = grown_cells(a, 2 * kPassSteps - 2), second = grown_cells(a, 2 * kPassSteps - 3);
     off[0] = 0;
