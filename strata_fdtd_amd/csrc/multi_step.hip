@@ -881,23 +881,28 @@ static int64_t grown_cells(const FusedArgs& a, int grow) {
 }
 
 // Whether a pass and its patch take less than single steps with their fix-up. Cells
-// with poles cost about the same either way (a few percent less in the patch), so
-// what counts is the rest of the grown box, which the patch takes at the price of a
-// plain step's cells (4.8 us per million and step in grids of 2 million cells, 6.2 at
-// 4 million, 7.6 at 7, 7 beyond the cache), against what a pass saves on the whole
-// grid (2.7 us per million, beyond the cache 4; a launch or two where a step is
-// little more than those). Both ways were timed on 469 solves of 40^3 to 320^3 with
-// 1, 3 and 8 poles: pairs of small absorbers at opposite corners of a box of a tenth
-// of the grid up to all of it, full boxes, shells and scattered cells. Where this
-// takes passes none was more than 2% slower than single steps. Pairs at the corners
-// of 128^3: single 23.1 us a step, passes 27.6, and 18.9 in a box of a tenth; 192^3
-// 45.2, 81.2, 34.5; 260^3 176, 182, 75; 320^3 224, 321, 122. Full boxes, three
-// poles: 100^3 40, 31; 192^3 257, 178. Lines between what was measured: at 192^3 a
-// third of the grid is where a pair's two ways meet, at 160^3 and 320^3 a half.
+// with poles cost about the same either way, so what counts is the rest of the grown
+// box, which the patch takes at the price of a plain step's cells (4.8 us per million
+// and step in grids of 2 million cells, 6.2 at 4 million, 7.6 at 7, 7 to 8 beyond the
+// cache), against what a pass saves on the whole grid: 2.9 us per million in the
+// cache; beyond it 4 where rows are whole 64-byte blocks, 5 of 32 bytes, 6 to 7
+// otherwise (there a single step's accesses cross lines, a pass's halos hit them);
+// and a launch or two where a step is little more than those. The shares below are
+// where the two ways meet, or a little under it. Both were timed on 620 solves of
+// 40^3 to 390^3 with 1, 3 and 8 poles: pairs of small absorbers at opposite corners
+// of a box of a tenth of the grid up to all of it, full boxes, shells and scattered
+// cells. Pairs in a third, half and all of the grid, single steps and passes, us a
+// step: 128^3 23.1 (21.5, 24.7, 27.6); 160^3 33.7 (30.0, 36.3, 45.7); 192^3 45.5 (49.0,
+// 59.0, 81.2); 256^3 126 (97.6, 124, 165); 264^3 173 (115, 142, 193); 390^3 615 (351,
+// 435, 659). Full boxes, three poles: 100^3 40, 31; 192^3 257, 178.
 bool patch_pays(const FusedArgs& a) {
     const int64_t cells = static_cast<int64_t>(a.nx) * a.ny * a.nz;
     if (cells >= kMaxCells32) return false;  // no passes at all
-    const double share = cells > 5000000 && cells <= kCacheResidentCells ? 0.33 : 0.45;
+    double share;
+    if (cells <= 5000000) share = 0.45;
+    else if (cells <= 6000000) share = 0.4;
+    else if (cells <= 7500000) share = 0.33;
+    else share = a.nz % 16 == 0 ? 0.45 : a.nz % 8 == 0 ? 0.58 : cells <= 17000000 ? 0.64 : 0.8;
     const int64_t air = grown_cells(a, 2 * kPassSteps - 2) - a.n_ade_cells;
     return static_cast<double>(air) <= 1e5 + share * static_cast<double>(cells);
 }

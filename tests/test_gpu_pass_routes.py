@@ -183,6 +183,7 @@ def _pole_solver(n, boxes):
     (128, [(30, 50), (78, 98)], True),          # the two a third of the sides apart
     (128, [(0, 128)], True),                    # all of the grid has poles
     (192, [(0, 20), (172, 192)], False),
+    (264, [(40, 60), (204, 224)], True),        # beyond the cache, rows of 32-byte blocks
     (40, [(0, 8), (32, 40)], True)])            # a step's launches outweigh its cells
 def test_passes_with_poles_where_the_patch_pays(n, boxes, passes):
     """Routes that the stated timings give; every one is bit-exact either way
