@@ -488,6 +488,11 @@ static int reserve(fdtd_ctx::DevBuf& b, size_t bytes) {
     return 0;
 }
 
+static void release(fdtd_ctx::DevBuf& b) {
+    if (b.p) (void)hipFree(b.p);
+    b = {};
+}
+
 static int upload(fdtd_ctx::DevBuf& b, const void* host, size_t bytes) {
     if (int rc = reserve(b, bytes)) return rc;
     if (bytes) return check(hipMemcpy(b.p, host, bytes, hipMemcpyHostToDevice), "hipMemcpy");
@@ -606,7 +611,13 @@ int fdtd_ctx_set_ade(fdtd_ctx* c, int n_pole, const int32_t* mat_id, const int32
     // with a pole count over stale tables).
     c->a.n_pole = 0;
     c->have_patch = false;
-    if (n_pole == 0) return 0;
+    if (n_pole == 0) {
+        // scratch up to as large as the fields goes back with the materials (the
+        // free waits for steps in flight)
+        DeviceGuard g(c->device);
+        release(c->patch_buf);
+        return 0;
+    }
     if (!mat_id || !target || !lorentz || !pa || !pb || !pd || !corr || !material || !lo || !hi || !J)
         return fail(-2, "bad ADE arrays");
     if (!c->have_grid) return fail(-3, "set the grid before the ADE materials");
@@ -691,6 +702,7 @@ int fdtd_ctx_set_ade(fdtd_ctx* c, int n_pole, const int32_t* mat_id, const int32
             c->have_patch = true;
         }
     }
+    if (!c->have_patch) release(c->patch_buf);
     c->a = a;
     return 0;
 }

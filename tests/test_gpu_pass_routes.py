@@ -198,3 +198,33 @@ def test_passes_with_poles_where_the_patch_pays(n, boxes, passes):
         one.step()
     for k in ("p", "vx", "vy", "vz"):
         assert np.array_equal(getattr(s, k), getattr(one, k)), k
+
+
+def test_patch_scratch_goes_back_with_the_materials():
+    """The patch's scratch (here two copies of the fields, 67 MB) is given back when
+    the materials are removed, and when they come to lie so that passes do not pay."""
+    import torch
+    n = 128
+    s = _pole_solver(n, [(0, n)])
+
+    def free():
+        s.step_n(3)
+        torch.cuda.synchronize()
+        return torch.cuda.mem_get_info()[0]
+
+    with_patch = free()
+    assert ctx_counts(s) == (1, 0)
+    s._material_id[:] = 0                         # two cells: their box is still all of the grid
+    s._material_id[0, 0, 0] = s._material_id[-1, -1, -1] = 1
+    s._dirty_ade = True
+    apart = free()
+    assert ctx_counts(s) == (1, 3)
+    assert apart - with_patch > 60e6
+    s._material_id[:] = 1
+    s._dirty_ade = True
+    again = free()
+    assert ctx_counts(s) == (2, 3) and apart - again > 60e6
+    s._material_id[:] = 0
+    s._dirty_ade = True
+    assert free() - again > 60e6
+    assert ctx_counts(s)[0] == 3
