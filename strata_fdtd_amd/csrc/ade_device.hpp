@@ -39,13 +39,23 @@ __device__ __forceinline__ float ade_recur(const AdePole& pl, float j0, float* j
 constexpr int kFewPoles = 4;
 struct CellPoles {
     AdePole po[kFewPoles];
+    int row[kFewPoles];             // its J's index in the density J at hand
     float jo[kFewPoles], jp[kFewPoles];
 };
 
-__device__ __forceinline__ void fetch_poles(const FusedArgs& a, int q0, CellPoles& cp) {
+// The density poles' J that a step reads: a.J (rows as registered) or the patch's
+// own (second; density poles alone, rows in the table's order), after the step's
+// update or, fresh, before it.
+struct DensityJ {
+    const float* J;
+    bool second, fresh;
+};
+
+__device__ __forceinline__ void fetch_poles(const FusedArgs& a, const DensityJ& d, int q0, CellPoles& cp) {
 #pragma unroll
     for (int x = 0; x < kFewPoles; ++x) {
         cp.po[x] = pole_at(a.poles, min(q0 + x, a.n_pole - 1));
+        cp.row[x] = d.second ? q0 + x : cp.po[x].slot;
         if (q0 + x >= a.n_pole) cp.po[x].mat = -1;
     }
 }
@@ -64,10 +74,10 @@ __device__ __forceinline__ bool some_lane(const AdePole& po, int m) {
     return __builtin_amdgcn_ballot_w64(po.mat == m) != 0;
 }
 
-// The cell's own J of the poles in cp. fresh: the density poles' J has yet to take
+// The cell's own J of the poles in cp. Where d is fresh, the density poles' J takes
 // this step's update from the cell's pressure p0 (Debye only).
 template <typename IX>
-__device__ __forceinline__ void fetch_own(const FusedArgs& a, const float* Jd, bool fresh, IX b, int m, float p0,
+__device__ __forceinline__ void fetch_own(const FusedArgs& a, const DensityJ& d, IX b, int m, float p0,
                                           CellPoles& cp) {
     const int64_t box_n = box_cells(a);
 #pragma unroll
@@ -75,17 +85,16 @@ __device__ __forceinline__ void fetch_own(const FusedArgs& a, const float* Jd, b
         const AdePole& po = cp.po[x];
         cp.jo[x] = cp.jp[x] = 0.f;
         if (!some_lane(po, m)) continue;
-        cp.jo[x] = ldx(gmem((po.target == 0 ? Jd : a.J) + po.slot * box_n), b);
+        cp.jo[x] = ldx(gmem(po.target == 0 ? d.J + cp.row[x] * box_n : a.J + po.slot * box_n), b);
         if (po.lorentz) cp.jp[x] = ldx(gmem(a.Jprev + po.slot * box_n), b);
-        if (fresh && po.target == 0) cp.jo[x] = ade_recur(po, cp.jo[x], nullptr, p0);
+        if (d.fresh && po.target == 0) cp.jo[x] = ade_recur(po, cp.jo[x], nullptr, p0);
     }
 }
 
 // The complete update of cell (i, j, k) from the input state S; POLES: its
 // material m has some, and the cell is box cell b. out: p before sources, vx, vy,
-// vz, damped. Jd: the density poles' J after this step's update, or, fresh, before
-// it; modulus poles are updated in a.J (own cell only). cp: the table's first poles
-// on entry; the cell's own J of them on return.
+// vz, damped. Modulus poles are updated in a.J (own cell only). cp: the table's first
+// poles on entry; the cell's own J of them on return.
 //
 // Instructions are what an update costs (a sphere's 267,000 cells are 16 waves a
 // CU; 15.2 us where predicated loads took 16.7), so loads are not predicated but read the cell itself where there is no
@@ -94,8 +103,8 @@ __device__ __forceinline__ void fetch_own(const FusedArgs& a, const float* Jd, b
 // table has the Debye poles before the Lorentz ones of each target, so one walk
 // adds each face's corrections in ade.cpp:240-401's order.
 template <bool NU, bool POLES, typename IX>
-__device__ __forceinline__ void ade_cell(const FusedArgs& a, const FieldView& S, const float* Jd, bool fresh, int i,
-                                         int j, int k, int m, IX b, CellPoles& cp, float out[4]) {
+__device__ __forceinline__ void ade_cell(const FusedArgs& a, const FieldView& S, const DensityJ& d, int i, int j,
+                                         int k, int m, IX b, CellPoles& cp, float out[4]) {
     const int nx = a.nx, ny = a.ny, nz = a.nz;
     const IX st[3] = {static_cast<IX>(S.ny) * static_cast<IX>(S.nz), static_cast<IX>(S.nz), 1};
     const IX gs[3] = {static_cast<IX>(ny) * static_cast<IX>(nz), static_cast<IX>(nz), 1};
@@ -139,7 +148,7 @@ __device__ __forceinline__ void ade_cell(const FusedArgs& a, const FieldView& S,
             mh[x] &= above == m;
             ml[x] &= under == m;
         }
-        fetch_own(a, Jd, fresh, b, m, p0, cp);
+        fetch_own(a, d, b, m, p0, cp);
     }
     float hi[3], lo[3];  // v' of the faces above and below, per axis
 #pragma unroll
@@ -152,14 +161,14 @@ __device__ __forceinline__ void ade_cell(const FusedArgs& a, const FieldView& S,
     if constexpr (POLES)
         for (int q0 = 0; q0 < a.n_pole; q0 += kFewPoles) {
             if (q0) {
-                fetch_poles(a, q0, cp);
-                fetch_own(a, Jd, fresh, b, m, p0, cp);
+                fetch_poles(a, d, q0, cp);
+                fetch_own(a, d, b, m, p0, cp);
             }
 #pragma unroll
             for (int q = 0; q < kFewPoles; ++q) {
                 const AdePole& po = cp.po[q];
                 if (po.target != 0 || !some_lane(po, m)) continue;
-                const GMEM float* Jq = gmem(Jd + po.slot * box_n);
+                const GMEM float* Jq = gmem(d.J + cp.row[q] * box_n);
                 float jh[3], jl[3];
 #pragma unroll
                 for (int x = 0; x < 3; ++x) {
@@ -168,7 +177,7 @@ __device__ __forceinline__ void ade_cell(const FusedArgs& a, const FieldView& S,
                 }
 #pragma unroll
                 for (int x = 0; x < 3; ++x) {
-                    if (fresh) {
+                    if (d.fresh) {
                         jh[x] = ade_recur(po, jh[x], nullptr, ph[x]);
                         jl[x] = ade_recur(po, jl[x], nullptr, pl[x]);
                     }
@@ -197,8 +206,8 @@ __device__ __forceinline__ void ade_cell(const FusedArgs& a, const FieldView& S,
         dA += dvz * iz;
         for (int q0 = 0; q0 < a.n_pole; q0 += kFewPoles) {
             if (a.n_pole > kFewPoles) {
-                fetch_poles(a, q0, cp);
-                fetch_own(a, Jd, fresh, b, m, p0, cp);
+                fetch_poles(a, d, q0, cp);
+                fetch_own(a, d, b, m, p0, cp);
             }
 #pragma unroll
             for (int q = 0; q < kFewPoles; ++q) {
@@ -220,22 +229,23 @@ __device__ __forceinline__ void ade_cell(const FusedArgs& a, const FieldView& S,
 }
 
 // The density poles' update of the step after, at box cell b with pressure x: from
-// the J that ade_cell left in cp into `to`.
+// the J that ade_cell left in cp (read from d) into `to`, the other of a.J and the
+// patch's own.
 template <typename IX>
-__device__ __forceinline__ void ade_density_next(const FusedArgs& a, const float* Jd, bool fresh, IX b, int m, float p0,
-                                                 float x, CellPoles& cp, float* to) {
+__device__ __forceinline__ void ade_density_next(const FusedArgs& a, const DensityJ& d, IX b, int m, float p0, float x,
+                                                 CellPoles& cp, float* to) {
     const int64_t box_n = box_cells(a);
     for (int q0 = 0; q0 < a.n_pole; q0 += kFewPoles) {
         if (a.n_pole > kFewPoles) {
-            fetch_poles(a, q0, cp);
-            fetch_own(a, Jd, fresh, b, m, p0, cp);
+            fetch_poles(a, d, q0, cp);
+            fetch_own(a, d, b, m, p0, cp);
         }
 #pragma unroll
         for (int q = 0; q < kFewPoles; ++q) {
             const AdePole& po = cp.po[q];
             if (po.target != 0 || po.mat != m) continue;
             float h = cp.jp[q];
-            stx(gmem(to + po.slot * box_n), b, ade_recur(po, cp.jo[q], po.lorentz ? &h : nullptr, x));
+            stx(gmem(to + (d.second ? po.slot : q0 + q) * box_n), b, ade_recur(po, cp.jo[q], po.lorentz ? &h : nullptr, x));
             if (po.lorentz) stx(gmem(a.Jprev + po.slot * box_n), b, h);
         }
     }

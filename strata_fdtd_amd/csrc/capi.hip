@@ -24,7 +24,7 @@ bool mic_in_pass(const FusedArgs& a, const int32_t box[6]);
 hipError_t launch_pass_stations(const FusedArgs& a, bool nu, const PatchArgs& pt, const StationPass& mp,
                                 hipStream_t st);
 bool patch_pays(const FusedArgs& a);
-int64_t patch_floats(const FusedArgs& a, int64_t off[3]);
+int64_t patch_floats(const FusedArgs& a, int n_density, int64_t off[3]);
 hipError_t launch_patch(const FusedArgs& a, bool nu, const PatchArgs& pt, hipStream_t st);
 hipError_t launch_advance(int64_t* step, int n, hipStream_t st);
 hipError_t launch_stream_ceiling(const FusedArgs& a, hipStream_t st);
@@ -686,7 +686,9 @@ int fdtd_ctx_set_ade(fdtd_ctx* c, int n_pole, const int32_t* mat_id, const int32
     a.n_pole = n_pole;
     if (c->multi_step && (c->every_pass ? static_cast<int64_t>(a.nx) * a.ny * a.nz < kMaxCells32 : patch_pays(a))) {
         int64_t off[3];
-        const int64_t floats = patch_floats(a, off);
+        const int n_density = static_cast<int>(
+            std::count_if(poles.begin(), poles.end(), [](const AdePole& q) { return q.target == 0; }));
+        const int64_t floats = patch_floats(a, n_density, off);
         // without room for the scratch (up to as much as the fields) the solve steps
         // one by one; a quarter of the free memory leaves others theirs
         size_t have = 0, all = 0;

@@ -204,7 +204,7 @@ struct PassTile {
 // Scratch of the cells such a pass leaves to single steps (k_patch_step).
 struct PatchArgs {
     float* box[kPassSteps - 1];     // [4][cells] of the material box grown after steps 1 and 2
-    float* J;                       // [n_pole][box cells]: the density poles' J of step 2
+    float* J;                       // [density poles][box cells]: their J of step 2
     int density;                    // step 1's J is updated by a launch of its own (Lorentz)
 };
 

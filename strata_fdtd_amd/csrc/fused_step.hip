@@ -521,8 +521,9 @@ __global__ __launch_bounds__(256) void k_ade_fixup(const FusedArgs a) {
     float* __restrict__ VYo = a.f[par ^ 1][2];
     float* __restrict__ VZo = a.f[par ^ 1][3];
     const int64_t n_visit = a.ade_cells ? a.n_ade_cells : box_cells(a);
+    const DensityJ density{a.J, false, false};
     CellPoles cp;
-    fetch_poles(a, 0, cp);
+    fetch_poles(a, density, 0, cp);
     for (int64_t e = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; e < n_visit;
          e += static_cast<int64_t>(gridDim.x) * blockDim.x) {
         const int64_t b = a.ade_cells ? static_cast<int64_t>(a.ade_cells[e]) : e;
@@ -533,8 +534,8 @@ __global__ __launch_bounds__(256) void k_ade_fixup(const FusedArgs a) {
         const int m = a.material[c];
         if (!has_pole(a, cp, m)) continue;
         float o[4];
-        ade_cell<NU, true, IX>(a, S, a.J, false, i, j, k, m, static_cast<IX>(b), cp, o);
-        if (a.n_pole > kFewPoles) fetch_poles(a, 0, cp);
+        ade_cell<NU, true, IX>(a, S, density, i, j, k, m, static_cast<IX>(b), cp, o);
+        if (a.n_pole > kFewPoles) fetch_poles(a, density, 0, cp);
         if (s < a.wave_len && (a.flags[c] & FDTD_FLAG_AIR)) o[0] = ade_sources(a, i, j, k, s, o[0]);
         Po[c] = o[0];
         VXo[c] = o[1];

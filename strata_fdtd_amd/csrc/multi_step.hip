@@ -633,23 +633,22 @@ __global__ __launch_bounds__(256) void k_patch_step(const FusedArgs a, const Pat
             const int m = ldx(gmem(a.material), c);
             const bool air = ldx(gmem(a.flags), c) & FDTD_FLAG_AIR;
             const float p0 = ldx(gmem(S.f[0]), lidx<uint32_t>(i - S.oi, j - S.oj, k - S.ok, S.ny, S.nz));
-            const bool fresh = t == 0 && !pt.density;
-            const float* Jd = t == 1 ? pt.J : a.J;
+            const DensityJ d{t == 1 ? pt.J : a.J, t == 1, t == 0 && !pt.density};
             float v[4];
             CellPoles cp;
-            fetch_poles(a, 0, cp);
-            ade_cell<NU, true, uint32_t>(a, S, Jd, fresh, i, j, k, m, b, cp, v);
+            fetch_poles(a, d, 0, cp);
+            ade_cell<NU, true, uint32_t>(a, S, d, i, j, k, m, b, cp, v);
             if (s < a.wave_len && air) v[0] = ade_sources(a, i, j, k, s, v[0]);
-            const uint32_t d = out_at(i, j, k);
+            const uint32_t at_out = out_at(i, j, k);
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                stx(out(g), d, v[g]);
+                stx(out(g), at_out, v[g]);
                 o[g][0] = v[g];
             }
             // density poles' J of the next step, from this step's pressure: from
             // a.J into pt.J and back, since neighbours still read this step's
             if (t < kPassSteps - 1)
-                ade_density_next(a, Jd, fresh, b, m, p0, v[0], cp, t == 1 ? a.J : pt.J);
+                ade_density_next(a, d, b, m, p0, v[0], cp, t == 1 ? a.J : pt.J);
             nk = 1;
             own = 1;
         }
@@ -673,7 +672,7 @@ __global__ __launch_bounds__(256) void k_patch_step(const FusedArgs a, const Pat
                 m &= static_cast<uint32_t>((uint64_t(1) << (8 * stop)) - 1u) & static_cast<uint32_t>(~uint64_t(0) << (8 * skip));
                 if (m) {
                     CellPoles cp;
-                    fetch_poles(a, 0, cp);
+                    fetch_poles(a, DensityJ{}, 0, cp);
 #pragma unroll
                     for (int x = 0; x < 4; ++x) {
                         const int mx = (m >> (8 * x)) & 255u;
@@ -760,7 +759,7 @@ __global__ __launch_bounds__(256) void k_station_pass(const FusedArgs a, const P
                 const int j = b0[1] + r % n[1], i = b0[0] + r / n[1];
                 float o[4];
                 CellPoles cp;
-                ade_cell<NU, false, uint32_t>(a, S, nullptr, false, i, j, k, 0, 0u, cp, o);
+                ade_cell<NU, false, uint32_t>(a, S, DensityJ{}, i, j, k, 0, 0u, cp, o);
                 if (s + t < a.wave_len && (a.flags[lin(i, j, k, a.ny, a.nz)] & FDTD_FLAG_AIR))
                     o[0] = ade_sources(a, i, j, k, s + t, o[0]);
                 for (int g = 0; g < 4; ++g) base[g * cells + tid] = o[g];
@@ -907,14 +906,14 @@ bool patch_pays(const FusedArgs& a) {
     return static_cast<double>(air) <= 1e5 + share * static_cast<double>(cells);
 }
 
-// Scratch floats of the patch: the boxes of steps 1 and 2, then the density poles'
-// second J.
-int64_t patch_floats(const FusedArgs& a, int64_t off[3]) {
+// Scratch floats of the patch: the boxes of steps 1 and 2, then the n_density density
+// poles' second J.
+int64_t patch_floats(const FusedArgs& a, int n_density, int64_t off[3]) {
     const int64_t first = grown_cells(a, 2 * kPassSteps - 2), second = grown_cells(a, 2 * kPassSteps - 3);
     off[0] = 0;
     off[1] = 4 * first;
     off[2] = off[1] + 4 * second;
-    return off[2] + a.n_pole * grown_cells(a, 0) + 4;  // a lane reads up to three cells past its row
+    return off[2] + n_density * grown_cells(a, 0) + 4;  // a lane reads up to three cells past its row
 }
 
 // Whether a pass can record a microphone with the cells [lo, hi): it lies in the

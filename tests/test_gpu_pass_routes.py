@@ -228,3 +228,38 @@ def test_patch_scratch_goes_back_with_the_materials():
     s._dirty_ade = True
     assert free() - again > 60e6
     assert ctx_counts(s)[0] == 3
+
+
+@pytest.mark.parametrize("density", [0, 1])
+def test_patch_scratch_has_a_second_J_of_density_poles_alone(density):
+    """Eight modulus poles all over 128^3: two copies of the fields (67 MB), and 8.4
+    MB for each density pole, registered last."""
+    import torch
+    import strata_fdtd_amd as sfa
+    n = 128
+    poles = [sfa.Pole(sfa.PoleType.DEBYE, 0.02 * (q + 1), "modulus", tau=1e-5 * (q + 1)) for q in range(8)]
+    poles += [sfa.Pole(sfa.PoleType.DEBYE, 0.3, "density", tau=2e-5)] * density
+    solvers = []
+    for _ in range(2):
+        s = sfa.FDTDSolver(shape=(n, n, n), resolution=1e-3)
+        s.register_material(sfa.SimpleMaterial(name="m", _rho=1.2, _c=343.0, _poles=poles), material_id=1)
+        s.set_material_box(1, *[(0, n)] * 3)
+        s.p = np.random.default_rng(3).standard_normal((n, n, n)).astype(np.float32)
+        solvers.append(s)
+    s, one = solvers
+    one.set_tiling(2, 2)
+    s.step_n(9)
+    for _ in range(9):
+        one.step()
+    assert ctx_counts(s) == (3, 0)
+    for k in ("p", "vx", "vy", "vz"):
+        assert np.array_equal(getattr(s, k), getattr(one, k)), k
+    torch.cuda.synchronize()
+    with_patch = torch.cuda.mem_get_info()[0]
+    s._material_id[:] = 0
+    s._dirty_ade = True
+    s.step_n(3)
+    torch.cuda.synchronize()
+    scratch = torch.cuda.mem_get_info()[0] - with_patch
+    cells = 4 * n**3
+    assert (8 + density) * cells <= scratch < (9.5 + density) * cells
