@@ -15,11 +15,6 @@ struct FieldView {
     __device__ __forceinline__ int64_t at(int i, int j, int k) const { return lin(i - oi, j - oj, k - ok, ny, nz); }
 };
 
-__device__ __forceinline__ int64_t box_index(const FusedArgs& a, int i, int j, int k) {
-    const int by = a.box_hi[1] - a.box_lo[1], bz = a.box_hi[2] - a.box_lo[2];
-    return ((static_cast<int64_t>(i - a.box_lo[0]) * by) + (j - a.box_lo[1])) * bz + (k - a.box_lo[2]);
-}
-
 __device__ __forceinline__ int64_t box_cells(const FusedArgs& a) {
     return static_cast<int64_t>(a.box_hi[0] - a.box_lo[0]) * (a.box_hi[1] - a.box_lo[1]) *
            (a.box_hi[2] - a.box_lo[2]);
