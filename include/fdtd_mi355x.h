@@ -348,7 +348,8 @@ int fdtd_adjoint_run(int dtype, void* const* lam, void* const* states, int64_t n
  * touch a row at or past steps_len return -4).
  * History (device float32): p on the box grown by one cell
  * ((hx+2)(hy+2)(hz+2) per step) and div on the box (hx hy hz per step) for
- * steps [hist0, hist0 + hist_steps); fdtd_design_history_bytes gives the size.
+ * steps [hist0, hist0 + hist_steps); fdtd_design_history_bytes gives the size
+ * (of these calls: the box's own rows).
  * The forward records it when hist_p is not NULL; the adjoint (steps
  * n_hi - 1 down to n_lo) reads it and Kahan-accumulates into acc, device
  * float32 [hx][hy][hz][4]: (sum, compensation) of dL/d(rho/rho0), then of

@@ -190,8 +190,9 @@ class _Fast:
     PLANES = 2
     ADJ_PLANES = 4
 
-    def __init__(self, dv: _Device, adjoint: bool = False):
-        """adjoint: the solve records the history its adjoint will read."""
+    def __init__(self, dv: _Device, adjoint: bool = False, passes: bool = True):
+        """adjoint: the solve records the history its adjoint will read. passes:
+        False for single steps and a history of the box's own rows."""
         import torch
         self.dv = dv
         pb = dv.pb
@@ -205,18 +206,15 @@ class _Fast:
         # its steps' velocities and pb on the box), kept with the solve. Without
         # room for it every step is taken singly, and the history's rows are the
         # box's own rather than whole 4-cell lanes.
-        n = _lib().fdtd_design_pass_floats(dv.lo.ctypes.data, dv.hi.ctypes.data, int(adjoint))
+        n = pass_scratch_bytes(pb, adjoint) // 4 if passes else 0
         try:
             self._scratch = torch.empty(n, dtype=torch.float32, device=dv.dev) if n > 0 else None
         except torch.cuda.OutOfMemoryError:
             self._scratch = None
-        if self._scratch is not None:
-            e, d = C.c_int64(), C.c_int64()
-            _native.call("fdtd_design_pass_history", dv.lo.ctypes.data, dv.hi.ctypes.data, C.byref(e), C.byref(d))
-            self.ecells, self.bcells = e.value, d.value
-        else:
-            lo, hi = np.array(pb.box_lo), np.array(pb.box_hi)
-            self.ecells, self.bcells = int(np.prod(hi - lo + 2)), int(np.prod(hi - lo))
+        self._rows()
+
+    def _rows(self):
+        self.ecells, self.bcells = _history_cells(self.dv.pb, self._scratch is not None)
 
     @staticmethod
     def _sets(sets):
@@ -238,6 +236,20 @@ class _Fast:
                 _ptr(rk))
 
     def history(self, steps):
+        """Room for `steps` steps' history. Where that of whole lanes does not fit
+        (a design box a voxel or two thick along z takes up to three times its own
+        rows), that of the box's rows, and single steps from here on."""
+        import torch
+        try:
+            return self._history(steps)
+        except torch.cuda.OutOfMemoryError:
+            if self._scratch is None:
+                raise
+        self._scratch = None
+        self._rows()
+        return self._history(steps)
+
+    def _history(self, steps):
         import torch
         return (torch.empty(steps * self.ecells, dtype=torch.float32, device=self.dv.dev),
                 torch.empty(steps * self.bcells, dtype=torch.float32, device=self.dv.dev))
@@ -265,24 +277,48 @@ class _Fast:
                      _ptr(self._scratch), self.dv.stream)
 
 
-def history_bytes(pb: DesignProblem, steps: int | None = None) -> int:
-    """HBM bytes of the float32 forward history (p on the box grown by one
-    cell, div on the box) for `steps` steps."""
-    lo, hi = np.array(pb.box_lo), np.array(pb.box_hi)
-    return 4 * int(np.prod(hi - lo + 2) + np.prod(hi - lo)) * (pb.steps if steps is None else steps)
+def _history_cells(pb: DesignProblem, lanes: bool) -> tuple[int, int]:
+    """Floats per step of the history's p and div: rows of whole 4-cell lanes (the
+    passes'), or the box's own."""
+    lo, hi = np.array(pb.box_lo, dtype=np.int32), np.array(pb.box_hi, dtype=np.int32)
+    if not lanes:
+        return int(np.prod(hi - lo + 2)), int(np.prod(hi - lo))
+    e, d = C.c_int64(), C.c_int64()
+    _native.call("fdtd_design_pass_history", lo.ctypes.data, hi.ctypes.data, C.byref(e), C.byref(d))
+    return e.value, d.value
 
 
-def _pick_history(pb: DesignProblem, history: str, device) -> str:
+def history_bytes(pb: DesignProblem, steps: int | None = None, lanes: bool = True) -> int:
+    """HBM bytes of the float32 forward history (p on the box grown by one cell,
+    div on the box) for `steps` steps, with the rows of whole 4-cell lanes that
+    multi-step passes store (lanes) or the box's own."""
+    return 4 * sum(_history_cells(pb, lanes)) * (pb.steps if steps is None else steps)
+
+
+def pass_scratch_bytes(pb: DesignProblem, adjoint: bool = True) -> int:
+    """HBM bytes of the passes' scratch (0: no passes for this box)."""
+    lo, hi = np.array(pb.box_lo, dtype=np.int32), np.array(pb.box_hi, dtype=np.int32)
+    return 4 * max(0, _lib().fdtd_design_pass_floats(lo.ctypes.data, hi.ctypes.data, int(adjoint)))
+
+
+def _pick_history(pb: DesignProblem, history: str, device) -> tuple[str, bool]:
+    """(history mode, passes): "auto" keeps every step where that takes at most half
+    of the free memory, for passes with their scratch, else with the box's own rows
+    and single steps."""
     if history != "auto":
-        return history
+        return history, True
     import torch
     free, _total = torch.cuda.mem_get_info(device)
-    return "all" if history_bytes(pb) <= 0.5 * free else "checkpoint"
+    if history_bytes(pb) + pass_scratch_bytes(pb) <= 0.5 * free:
+        return "all", True
+    if history_bytes(pb, lanes=False) <= 0.5 * free:
+        return "all", False
+    return "checkpoint", True
 
 
-def _forward_fast(pb, r, kappa, dv, history: str):
+def _forward_fast(pb, r, kappa, dv, history: str, passes: bool = True):
     import torch
-    fast = _Fast(dv, adjoint=history in ("all", "checkpoint"))
+    fast = _Fast(dv, adjoint=history in ("all", "checkpoint"), passes=passes)
     rk = fast.pack(r, kappa)
     rec = None
     if history == "checkpoint":
@@ -366,8 +402,8 @@ def forward_traces(pb: DesignProblem, rho=None, K=None, dtype=None, device="cuda
     if impl == "fast":
         if dtype != torch.float32:
             raise ValueError("the fast design kernels are float32")
-        mode = _pick_history(pb, history, dev) if keep_checkpoints else "none"
-        return _forward_fast(pb, r, kappa, dv, mode)
+        mode, passes = _pick_history(pb, history, dev) if keep_checkpoints else ("none", True)
+        return _forward_fast(pb, r, kappa, dv, mode, passes)
     a, b = dv.zeros_state(), dv.zeros_state()
     traces = torch.zeros((pb.steps, max(dv.n_probe, 1)), dtype=dtype, device=device)
     ckpts = []
