@@ -291,7 +291,7 @@ class FDTDSolver:
         _native.call("fdtd_ctx_set_counters", ctx, _native.ptr(self._step_dev), _native.ptr(self._health))
         tiling = self._tiling or pick_tiling(self.shape, not self._grid.is_uniform, False)
         _native.call("fdtd_ctx_set_tiling", ctx, *tiling)
-        _native.call("fdtd_ctx_set_multi_step", ctx, 1 if self._tiling is None else 2)
+        self._allow_passes(self._tiling is None)
 
     def set_tiling(self, rows: int, planes: int, stack: int = 1) -> None:
         """Launch shape of the fused kernel: rows per wave, planes per wave and
@@ -299,8 +299,13 @@ class FDTDSolver:
         shape is given takes every step with that kernel; by default step_n
         takes three steps per pass where the solve allows it."""
         self._tiling = normalize_tiling((rows, planes, stack))
-        _native.call("fdtd_ctx_set_multi_step", self._ctx, 2)
+        self._allow_passes(False)
         _native.call("fdtd_ctx_set_tiling", self._ctx, *self._tiling)
+
+    def _allow_passes(self, on: bool) -> None:
+        """Whether step_n may take several steps per pass."""
+        self._passes = on
+        _native.call("fdtd_ctx_set_multi_step", self._ctx, 1 if on else 2)
 
     @property
     def tiling(self) -> tuple[int, int, int]:

@@ -263,3 +263,24 @@ def test_patch_scratch_has_a_second_J_of_density_poles_alone(density):
     scratch = torch.cuda.mem_get_info()[0] - with_patch
     cells = 4 * n**3
     assert (8 + density) * cells <= scratch < (9.5 + density) * cells
+
+
+def test_autotune_keeps_passes_where_they_are_faster():
+    """The launch shape that it sets is of single steps; a solver that took passes
+    still does where the fastest shape is slower (128^3: 16 us a step against 11),
+    with materials or without; one made with a launch shape does not begin to."""
+    from strata_fdtd_amd import FDTDSolver
+    from strata_fdtd_amd.autotune import autotune
+    shapes = [(2, 2, 1), (4, 4, 1)]
+    plain, poles = FDTDSolver(shape=(128, 128, 128), resolution=1e-3), _pole_solver(128, [(54, 74)])
+    given = FDTDSolver(shape=(128, 128, 128), resolution=1e-3, tiling=(2, 2))
+    for s, passes in ((plain, True), (poles, True), (given, False)):
+        best, table = autotune(s, candidates=shapes, store=False)
+        assert s.tiling == best and best in shapes and len(table) == 2
+        before = ctx_counts(s)
+        s.step_n(9)
+        assert tuple(b - a for a, b in zip(before, ctx_counts(s))) == ((3, 0) if passes else (0, 9))
+    plain.set_tiling(2, 2)
+    before = ctx_counts(plain)
+    plain.step_n(9)
+    assert ctx_counts(plain) == (before[0], before[1] + 9)
