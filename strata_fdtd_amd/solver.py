@@ -931,20 +931,22 @@ class FDTDSolver:
                     # the steps up to and with the next one that is recorded go
                     # to the device as one run, so that passes of several steps
                     # can end on it (with a progress bar, runs of at most 256
-                    # steps, each waited for before the bar moves)
+                    # steps, waited for before the bar moves unless they are a
+                    # recorded step alone, which waits for nothing)
                     limit = min(n_steps, step + 256) if bar is not None else n_steps
                     first, j, fires = self._step_count - step, step, False
                     while j < limit and not fires:
                         fires = self._hooks_fire(first + j) or (h5_snaps is not None and j % snapshot_interval == 0)
                         j += 1
                     self.step_n(j - step)
+                    if bar is not None and j - step > fires:
+                        self._stream.synchronize()
                     if fires:
                         t_before = self._step_times[-1]
                         self._after_step_hooks(self._step_count - 1, t_before)
                         if h5_snaps is not None and (j - 1) % snapshot_interval == 0:
                             h5_snaps.append((t_before, self._snapshot_p()))
                     if bar is not None:
-                        self._stream.synchronize()
                         bar.update(j - step)
                     step = j
                     continue

@@ -44,3 +44,28 @@ def test_pass_sources_of_a_solver_on_a_side_stream(oracle_lib):
     s.step_n(n)
     torch.cuda.synchronize()
     _compare(sc, s, st_o, tr_o)
+
+
+@pytest.mark.parametrize("every,waits", [(1, 0), (4, 10), (None, 1)])
+def test_progress_bar_waits_for_runs_of_steps_only(every, waits, monkeypatch):
+    """run(progress=True): a recorded step by itself is enqueued and not waited for
+    (snapshots of every step would otherwise each stop the device); between recorded
+    steps one wait per run of steps."""
+    import torch
+    from strata_fdtd_amd import FDTDSolver
+    s = FDTDSolver(shape=(24, 24, 24), resolution=1e-3)
+    if every:
+        s.enable_snapshots(every)
+    s.step_n(40 if every is None else 4 * every)       # set up
+    s.reset()
+    n = []
+    real = torch.cuda.Stream.synchronize
+    monkeypatch.setattr(torch.cuda.Stream, "synchronize", lambda self: (n.append(1), real(self))[1])
+    during = []
+    from tqdm import tqdm
+    close = tqdm.close
+    monkeypatch.setattr(tqdm, "close", lambda self: (during.append(len(n)), close(self))[1])
+    s.run(39.5 * s.dt, progress=True)
+    assert during[0] == waits
+    if every:
+        assert len(s.get_snapshots()) == 40 // every
