@@ -799,6 +799,7 @@ static bool pass_windows(int nx, int ny, int nz, int nt, int nseg, PassTile& m) 
     if (nseg == 1) {
         m.ko = m.kt = lanes;
     } else {
+        if (lanes < nseg) return false;
         m.ko = ((lanes - 1 + nseg - 1) / nseg + 3) & ~3;  // segments start on 64-byte blocks of the row
         m.kt = m.ko + 2;
         // every segment has lanes to store, and the last one's fit its window
@@ -834,9 +835,9 @@ bool pick_pass_tile(int nx, int ny, int nz, int only_nt, double share, PassTile&
             PassTile m{};
             if (!pass_windows(nx, ny, nz, nt, nseg, m)) continue;
             const int nwin = m.nseg * m.njt;
-            for (int c = 1; c <= nx; ++c) {
-                const int units = (nx + c - 1) / c;
-                if (c > 1 && units == (nx + c - 2) / (c - 1)) continue;  // the same split as c - 1
+            // chunks c: the fewest of each chunk length (2 sqrt(nx) of them at most)
+            for (int c = 1, units = 0; c <= nx; c = units > 1 ? (nx + units - 2) / (units - 1) : nx + 1) {
+                units = (nx + c - 1) / c;
                 const int64_t n = static_cast<int64_t>(nwin) * ((nx + units - 1) / units);
                 const double planes = units + 2 * kPassSteps - 1;
                 auto plane_us = [&](int64_t wgs) {

@@ -58,3 +58,13 @@ def test_windows_cover_the_grid_once(shape):
 def test_no_passes_beyond_32_bit_offsets():
     assert _tiling((1024, 1024, 1024))["steps"] == 0
     assert _tiling((1024, 1024, 1023))["steps"] == STEPS
+
+
+def test_long_grids_are_split_quickly():
+    """The split of 10^8 planes takes milliseconds (one look at each chunk length,
+    not at each number of chunks: 82 seconds)."""
+    import time
+    start = time.perf_counter()
+    t = _tiling((100_000_000, 2, 2))
+    assert time.perf_counter() - start < 5.0
+    assert (t["units"], t["nwg"], t["nseg"]) == (97657, 1024, 1)
