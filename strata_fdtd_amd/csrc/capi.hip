@@ -1180,6 +1180,8 @@ struct fdtd_batch {
     int n = 0;
     int total_waves = 0;
     int total_wgs = 0;                  // workgroups of a pass; 0: single steps only
+    int64_t cells = 0;                  // of all solves
+    bool every_pass = false;            // a solve asks for passes wherever they can be taken
     bool nts = true;                    // non-temporal stores (the solves exceed the cache)
     hipGraphExec_t graph = nullptr;
     int graph_steps = 0;
@@ -1345,11 +1347,25 @@ int fdtd_batch_set(fdtd_batch* b, fdtd_ctx* const* ctxs, const int64_t* step_lim
     b->n = n;
     b->total_waves = total;
     b->total_wgs = total_wgs;
+    b->cells = cells;
+    b->every_pass = std::any_of(ctxs, ctxs + n, [](const fdtd_ctx* c) { return c->every_pass; });
     b->nts = cells > kCacheResidentCells;
     return 0;
 }
 
-static bool batch_passes(int cap_wgs, int n_steps) { return cap_wgs > 0 && n_steps >= kPassSteps; }
+// Workgroups of the passes of a chunk of n_steps steps, 0 for single steps: too few
+// steps, a solve without passes, or solves too small together. A pass takes what
+// its planes' latency takes, and a chunk ends with two launches for the steps that
+// its passes leave, which in a graph are 0.9 us each also where they leave none. Us a
+// step, single steps and passes: chunks of 3 steps, one 64^3 solve 7.9 and 9.1, four
+// of 56^3 11.1 and 10.6, one of 96^3 12.0 and 11.1; of 100, one 40^3 5.1 and 5.3, four
+// of 32^3 5.5 and 5.3, eight 6.1 and 5.5. A graph that has passes keeps them when
+// solves leave: another capture costs more than the steps would gain.
+static int batch_wgs(const fdtd_batch* b, int n_steps, bool use_graph) {
+    if (n_steps < kPassSteps) return 0;
+    if (use_graph && b->graph && b->graph_steps == n_steps && b->graph_wgs > 0) return b->total_wgs;
+    return b->every_pass || b->cells >= 300000 || (b->cells >= 120000 && n_steps >= 64) ? b->total_wgs : 0;
+}
 
 // A chunk of n_steps steps of every solve: passes of kPassSteps steps where every
 // solve takes them (cap_wgs > 0), then the one or two steps they leave (to the
@@ -1357,7 +1373,7 @@ static bool batch_passes(int cap_wgs, int n_steps) { return cap_wgs > 0 && n_ste
 // moves the counters. Steps are counted from the solves' counters.
 static int batch_enqueue(fdtd_batch* b, hipStream_t st, int n_steps, int cap_waves, int cap_wgs) {
     int singles = n_steps;
-    const bool passes = batch_passes(cap_wgs, n_steps);
+    const bool passes = cap_wgs > 0;
     if (passes) {
         for (int s = 0; s + kPassSteps <= n_steps; s += kPassSteps)
             if (int rc = check(launch_batch_pass(b->table_dev, b->tile_dev, b->meta_dev + b->cap + 2, b->meta_dev, cap_wgs,
@@ -1379,18 +1395,18 @@ int fdtd_batch_step_n(fdtd_batch* b, int n_steps, int use_graph) {
     if (n_steps < 0) return fail(-2, "negative step count");
     if (b->n == 0 || n_steps == 0) return 0;
     DeviceGuard g(b->device);
-    const bool passes = batch_passes(b->total_wgs, n_steps);
-    b->n_pass += passes ? n_steps / kPassSteps : 0;
-    b->n_single += passes ? kPassSteps - 1 : n_steps;
-    if (!use_graph) return batch_enqueue(b, b->stream, n_steps, b->total_waves, b->total_wgs);
+    const int wgs = batch_wgs(b, n_steps, use_graph != 0);
+    b->n_pass += wgs > 0 ? n_steps / kPassSteps : 0;
+    b->n_single += wgs > 0 ? kPassSteps - 1 : n_steps;
+    if (!use_graph) return batch_enqueue(b, b->stream, n_steps, b->total_waves, wgs);
     if (!b->graph || b->graph_steps != n_steps || b->graph_waves < b->total_waves || b->graph_nts != b->nts ||
-        b->graph_wgs < b->total_wgs || (b->graph_wgs > 0) != (b->total_wgs > 0)) {
+        b->graph_wgs < wgs || (b->graph_wgs > 0) != (wgs > 0)) {
         // capture with head room so that later tables of up to this many waves
         // replay it; a recapture for another reason keeps the capacity
         int cap_waves = b->graph_waves;
         if (cap_waves < b->total_waves) cap_waves = std::max(b->total_waves + b->total_waves / 2, b->graph_waves * 2);
-        int cap_wgs = b->total_wgs > 0 ? b->graph_wgs : 0;
-        if (cap_wgs < b->total_wgs) cap_wgs = std::max(b->total_wgs + b->total_wgs / 2, cap_wgs * 2);
+        int cap_wgs = wgs > 0 ? b->graph_wgs : 0;
+        if (cap_wgs < wgs) cap_wgs = std::max(wgs + wgs / 2, cap_wgs * 2);
         batch_drop_graph(b);
         hipStream_t cap = nullptr;
         if (int rc = check(hipStreamCreateWithFlags(&cap, hipStreamNonBlocking), "hipStreamCreate")) return rc;

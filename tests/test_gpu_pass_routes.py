@@ -284,3 +284,52 @@ def test_autotune_keeps_passes_where_they_are_faster():
     before = ctx_counts(plain)
     plain.step_n(9)
     assert ctx_counts(plain) == (before[0], before[1] + 9)
+
+
+@pytest.mark.parametrize("n,count,chunk,passes", [(40, 1, 100, False), (32, 4, 100, True), (64, 1, 16, False),
+                                                  (64, 1, 99, True), (96, 1, 3, True), (96, 1, 2, False)])
+@pytest.mark.parametrize("use_graph", [0, 1])
+def test_batches_take_passes_where_they_pay(n, count, chunk, passes, use_graph):
+    """Small solves in short chunks step one by one; two chunks of either way equal
+    the lone solves' one-step kernels; a captured chunk of passes stays when a solve
+    leaves."""
+    import torch
+    from strata_fdtd_amd import FDTDSolver, GaussianPulse, _native
+
+    def solve():
+        s = FDTDSolver(shape=(n, n, n), resolution=1e-3, tiling=(2, 2))
+        s.add_source(GaussianPulse(position=(n // 2,) * 3, frequency=5e3))
+        s.add_probe("p", (n // 3,) * 3)
+        s.p = np.random.default_rng(1).standard_normal((n, n, n)).astype(np.float32)
+        s._prepare(3 * chunk)
+        return s
+
+    batch, one = [solve() for _ in range(count)], solve()
+    h = _native._vp()
+    _native.call("fdtd_batch_create", 0, torch.cuda.current_stream().cuda_stream, 2, C.byref(h))
+    try:
+        def serve(solves, chunks):
+            ctxs = (_native._vp * count)(*[s._ctx for s in solves])
+            limits = np.full(count, 3 * chunk, dtype=np.int64)
+            _native.call("fdtd_batch_set", h.value, ctxs, limits.ctypes.data, len(solves))
+            before = _counts("fdtd_batch_step_counts", h.value)
+            for _ in range(chunks):
+                _native.call("fdtd_batch_step_n", h.value, chunk, use_graph)
+            torch.cuda.synchronize()
+            return tuple(b - a for a, b in zip(before, _counts("fdtd_batch_step_counts", h.value)))
+
+        in_passes, singly = (chunk // STEPS, STEPS - 1), (0, chunk)
+        want = in_passes if passes else singly
+        assert serve(batch, 2) == (2 * want[0], 2 * want[1])
+        if count > 1:
+            assert serve(batch[:1], 1) == (in_passes if use_graph else singly)
+        else:
+            serve(batch, 1)
+    finally:
+        _native.load().fdtd_batch_destroy(h.value)
+    one.step_n(3 * chunk)
+    first = batch[0]
+    first._advance_host(3 * chunk)
+    for k in ("p", "vx", "vy", "vz"):
+        assert np.array_equal(getattr(first, k), getattr(one, k)), k
+    assert np.array_equal(first.get_probe_data()["p"], one.get_probe_data()["p"])
