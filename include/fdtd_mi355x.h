@@ -114,6 +114,12 @@ int fdtd_ctx_set_pass_sources(fdtd_ctx* ctx, int n, const int32_t* kind, const i
  * Host only. */
 int fdtd_pass_tiling(int nx, int ny, int nz, int32_t* out);
 
+/* A given split of the context's grid in its place, until the grid is set again:
+ * 256, 512 or 1024 threads per workgroup, windows along k, planes per workgroup, and
+ * whether the fields are stored past the caches. threads 0: the split of
+ * fdtd_pass_tiling again. Fails where the grid has no such windows. */
+int fdtd_ctx_set_pass_tiling(fdtd_ctx* ctx, int threads, int segments, int planes, int non_temporal);
+
 /* Probes: host flat indices; trace: device float32 [trace_len][n]; step s
  * writes row s. Replaces _record_probes (core/solver.py:2435-2439). */
 int fdtd_ctx_set_probes(fdtd_ctx* ctx, int n, const int64_t* flat_idx, float* trace,

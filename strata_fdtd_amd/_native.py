@@ -39,6 +39,7 @@ _SIGS = {
     "fdtd_ctx_set_multi_step": (_i, [_vp, _i]),
     "fdtd_ctx_set_pass_sources": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _i64]),
     "fdtd_pass_tiling": (_i, [_i, _i, _i, _vp]),
+    "fdtd_ctx_set_pass_tiling": (_i, [_vp, _i, _i, _i, _i]),
     "fdtd_ctx_set_probes": (_i, [_vp, _i, _vp, _vp, _i64]),
     "fdtd_ctx_set_membranes": (_i, [_vp, _i, _vp, _vp, _i, _vp, _vp, _vp, _vp, _i, _vp, _i, _vp, _i64]),
     "fdtd_ctx_set_microphones": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _i64]),

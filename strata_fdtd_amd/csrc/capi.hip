@@ -19,7 +19,8 @@ int fused_grid(FusedArgs& a, int rows, int planes, int stack);
 hipError_t launch_fused(const FusedArgs& a, int rows, int stack, bool nu, bool ade, int blocks,
                         hipStream_t st, hipEvent_t ev_before, hipEvent_t ev_after, const BoundarySet* bnd);
 bool pick_pass_tile(int nx, int ny, int nz, int only_nt, double share, PassTile& best);
-hipError_t launch_pass(const FusedArgs& a, bool nu, const PassTile& m, hipStream_t st);
+bool pass_tile_of(int nx, int ny, int nz, int nt, int nseg, int units, PassTile& m);
+hipError_t launch_pass(const FusedArgs& a, bool nu, const PassTile& m, bool nts, hipStream_t st);
 bool mic_in_pass(const FusedArgs& a, const int32_t box[6]);
 hipError_t launch_pass_stations(const FusedArgs& a, bool nu, const PatchArgs& pt, const StationPass& mp,
                                 hipStream_t st);
@@ -136,7 +137,7 @@ struct fdtd_ctx {
         int64_t wave_len = 0;
     } pass_src;
     bool multi_step = false, every_pass = false, padded = false, have_pass_src = false;
-    bool tile_known = false, tile_ok = false;
+    bool tile_known = false, tile_ok = false, tile_nts = false;
     PassTile tile{};
     // in a batch: the windows for a share of the chip of 1, 1/2, 1/4 .. 1/64
     bool batch_tile_known[7] = {}, batch_tile_ok[7] = {};
@@ -351,6 +352,20 @@ int fdtd_pass_tiling(int nx, int ny, int nz, int32_t* out) {
     const bool ok = pick_pass_tile(nx, ny, nz, 0, 1.0, m);
     const int32_t v[9] = {ok ? kPassSteps : 0, m.nt, m.kt, m.ko, m.rows, m.nseg, m.njt, m.units, m.nwg};
     std::copy(v, v + 9, out);
+    return 0;
+}
+
+int fdtd_ctx_set_pass_tiling(fdtd_ctx* c, int threads, int segments, int planes, int non_temporal) {
+    if (!c) return fail(-1, "null context");
+    if (!c->have_grid) return fail(-3, "set the grid before the windows of its passes");
+    PassTile m{};
+    if (threads != 0 && !pass_tile_of(c->a.nx, c->a.ny, c->a.nz, threads, segments, planes, m))
+        return fail(-2, "no windows of %d threads and %d segments marching %d planes for this grid", threads, segments,
+                    planes);
+    drop_graph(c);
+    c->tile_known = c->tile_ok = threads != 0;
+    c->tile = m;
+    c->tile_nts = non_temporal != 0;
     return 0;
 }
 
@@ -771,6 +786,7 @@ static bool pass_allowed(fdtd_ctx* c) {
     if (!c->tile_known) {
         c->tile_known = true;
         c->tile_ok = pick_pass_tile(a.nx, a.ny, a.nz, 0, 1.0, c->tile);
+        c->tile_nts = static_cast<int64_t>(a.nx) * a.ny * a.nz > kCacheResidentCells;
     }
     return c->tile_ok && pass_pays(c);
 }
@@ -784,7 +800,7 @@ static int enqueue_steps(fdtd_ctx* c, int n) {
         if (a.n_mcell > 0) use_sources(pa, c->pass_src);
         for (; n - s >= kPassSteps; s += kPassSteps) {
             pa.koff = s;
-            if (int rc = check(launch_pass(pa, c->nonuniform, c->tile, c->stream), "multi-step pass launch")) return rc;
+            if (int rc = check(launch_pass(pa, c->nonuniform, c->tile, c->tile_nts, c->stream), "multi-step pass launch")) return rc;
             if (pa.n_pole > 0)
                 if (int rc = check(launch_patch(pa, c->nonuniform, c->patch, c->stream), "patch launch")) return rc;
             if (stations(c, pa.n_mic) > 0) {

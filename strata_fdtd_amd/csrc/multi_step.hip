@@ -863,13 +863,22 @@ bool pick_pass_tile(int nx, int ny, int nz, int only_nt, double share, PassTile&
     return found;
 }
 
+// The given split instead; false where the grid has no such windows.
+bool pass_tile_of(int nx, int ny, int nz, int nt, int nseg, int units, PassTile& m) {
+    m = PassTile{};
+    const bool sizes = (nt == 256 || nt == 512 || nt == 1024) && nseg >= 1 && units >= 1 && units <= nx;
+    if (static_cast<int64_t>(nx) * ny * nz >= kMaxCells32 || !sizes || !pass_windows(nx, ny, nz, nt, nseg, m)) return false;
+    const int64_t n = static_cast<int64_t>(m.nseg) * m.njt * ((nx + units - 1) / units);
+    m.units = units;
+    m.nwg = static_cast<int>(n);
+    return n < (1 << 30);
+}
+
 template <bool NU, int NT>
-static hipError_t launch_pass_t(const FusedArgs& a, const PassTile& m, hipStream_t st) {
+static hipError_t launch_pass_t(const FusedArgs& a, const PassTile& m, bool nts, hipStream_t st) {
     const int blocks = (m.nwg + 7) & ~7;
-    if (static_cast<int64_t>(a.nx) * a.ny * a.nz <= kCacheResidentCells)
-        hipLaunchKernelGGL((k_multi_step<NU, NT, false>), dim3(blocks), dim3(NT), 0, st, a, m);
-    else
-        hipLaunchKernelGGL((k_multi_step<NU, NT, true>), dim3(blocks), dim3(NT), 0, st, a, m);
+    if (nts) hipLaunchKernelGGL((k_multi_step<NU, NT, true>), dim3(blocks), dim3(NT), 0, st, a, m);
+    else hipLaunchKernelGGL((k_multi_step<NU, NT, false>), dim3(blocks), dim3(NT), 0, st, a, m);
     return hipGetLastError();
 }
 
@@ -957,12 +966,12 @@ hipError_t launch_patch(const FusedArgs& a, bool nu, const PatchArgs& pt, hipStr
     return e;
 }
 
-// Steps koff .. koff + kPassSteps - 1 of a chunk in one pass.
-hipError_t launch_pass(const FusedArgs& a, bool nu, const PassTile& m, hipStream_t st) {
+// Steps koff .. koff + kPassSteps - 1 of a chunk in one pass. nts: non-temporal stores.
+hipError_t launch_pass(const FusedArgs& a, bool nu, const PassTile& m, bool nts, hipStream_t st) {
     switch (m.nt) {
-        case 1024: return nu ? launch_pass_t<true, 1024>(a, m, st) : launch_pass_t<false, 1024>(a, m, st);
-        case 512: return nu ? launch_pass_t<true, 512>(a, m, st) : launch_pass_t<false, 512>(a, m, st);
-        case 256: return nu ? launch_pass_t<true, 256>(a, m, st) : launch_pass_t<false, 256>(a, m, st);
+        case 1024: return nu ? launch_pass_t<true, 1024>(a, m, nts, st) : launch_pass_t<false, 1024>(a, m, nts, st);
+        case 512: return nu ? launch_pass_t<true, 512>(a, m, nts, st) : launch_pass_t<false, 512>(a, m, nts, st);
+        case 256: return nu ? launch_pass_t<true, 256>(a, m, nts, st) : launch_pass_t<false, 256>(a, m, nts, st);
         default: return hipErrorInvalidValue;
     }
 }
