@@ -90,8 +90,9 @@ def tune_shapes(requests, rows: int = 2, planes=(1, 2, 4, 8), steps: int = 20, d
     is timed with each candidate (rows, planes) strip (``autotune.autotune``,
     device time over `steps` steps) and the fastest is stored in the tiling
     cache, where ``pick_tiling`` (used by the server and by single solves)
-    finds it. `rows` is the batched sweep's row count, so only the strip
-    length along i is chosen per shape. Returns {shape: (tiling, ms per step)}.
+    finds it. They are shapes of single steps, which batches in passes take for the
+    steps that passes leave. `rows` is the batched sweep's row count, so only the
+    strip length along i is chosen per shape. Returns {shape: (tiling, ms per step)}.
 
     Measured on the 64-request sweep (62 shapes, tuned in 0.2 s), one step per
     launch: the tuned
@@ -211,8 +212,9 @@ class SweepServer:
 
     CACHE_RESIDENT_CELLS = 6 << 20
     # batched rate (cell-updates per second) that converts a request's work
-    # into seconds for the "aged" order (about the measured rate of a
-    # cache-resident batch)
+    # into seconds for the "aged" order: about that of a cache-resident batch
+    # stepped one by one (in passes the 64-request sweep runs at 265e9; the
+    # smaller rate gives small requests the more credit)
     NOMINAL_RATE = 120e9
 
     def __init__(self, device: int = 0, rows: int = 2, chunk: int = 100, max_active: int = 64,
